@@ -2,20 +2,13 @@
 // operator and the generic scalar convection, the node-ordered assembly gather,
 // and their drop-in C-ABI entry points.
 //
-// Layout and mapping (gfx950):
-//  * one element per workgroup of NT = roundup((p+1)^3, 64) lanes; lane a owns
-//    element-local node / quadrature point a (the reference's gmsh order);
-//  * the element's nodal fields are staged field-major in LDS; each lane builds
-//    once, in registers, the LDS offsets of the p other nodes on its three GLL
-//    lines and the matching rows of the derivative table (and of its transpose
-//    for the weak divergence of the viscous fluxes);
-//  * blocks walk the elements in a grid-stride loop whose block -> element map
-//    gives each XCD (blockIdx % 8) one contiguous eighth of the elements, so
-//    nodes shared by neighbouring elements are re-read from the same L2;
-//  * element residuals go to a scratch array of 5-field records per element-node
-//    (whole elements: coalesced writes); a second kernel gathers them per node through
-//    the node-ordered incidence table in the reference's serial (element, node)
-//    order -- deterministic, no atomics.
+// The operators run on the element pipeline of pipe.hpp (lane-per-node, line
+// order, geometry through LDS); the fused stage at p=3 and the entropy and
+// velocity operators have kernels of their own below.  Element residuals go to a
+// scratch array of 5-field records per element-node (whole elements: coalesced
+// writes); a second kernel gathers them per node through the node-ordered
+// incidence table in the reference's serial (element, node) order --
+// deterministic, no atomics.
 //
 // Arithmetic restatement: the split forms are evaluated through identities that
 // hold for arbitrary nodal inputs (linearity of the discrete derivative and
@@ -25,13 +18,15 @@
 //  * advective derivatives a.grad(f) use contravariant components
 //    sum_j He(j,k) a_j at the quadrature point;
 //  * flux divergences sum_j d_j(s u_j) are evaluated from the line values of s
-//    times the contravariant velocity sum_j He_g(j,k) u_j(m) at the line node m.
+//    times the contravariant velocity sum_j He_g(j,k) u_j(m) at the line node m,
+//    with the advective derivative of s folded into the same line sum (k_rhs).
 #include <cstdio>
 #include <type_traits>
 
 #include "common.hpp"
 #include "device.hpp"
 #include "element.hpp"
+#include "pipe.hpp"
 
 #ifndef SODHIP_SPLIT_WAVES
 #define SODHIP_SPLIT_WAVES 2
@@ -59,32 +54,6 @@
 
 namespace sodhip {
 
-// Copies the geometry block of one element (HEB bytes of He, then GVB bytes of
-// gpvol) HBM -> LDS with the direct-to-LDS loads of gfx950: one wave
-// instruction moves a row of 64 lanes x W bytes; the NW waves of the
-// workgroup take alternate rows.  Lanes past the end re-read the last W bytes.
-template <int W, int HEB, int GVB, int NW>
-__device__ __forceinline__ void geo_copy(const unsigned char *he, const unsigned char *gv,
-                                         unsigned char *geo, int wl, int wv)
-{
-    constexpr int R = 64 * W, ROWS = (HEB + GVB + R - 1) / R;
-#pragma unroll
-    for (int r0 = 0; r0 < ROWS; r0 += NW) {
-        const int r = r0 + wv;
-        if (r < ROWS) {
-            const int byte = r * R + wl * W;
-            const unsigned char *src = byte < HEB ? he + byte : gv + min(byte - HEB, GVB - W);
-            // offset applied in the LDS address space (a generic round trip of a
-            // constant LDS address miscompiles)
-            auto *dst = (__attribute__((address_space(3))) unsigned char *)geo + r * R;
-            if constexpr (W == 16)
-                __builtin_amdgcn_global_load_lds((const void *)src, dst, 16, 0, 0);
-            else
-                __builtin_amdgcn_global_load_lds((const void *)src, dst, 4, 0, 0);
-        }
-    }
-}
-
 template <typename T> struct RhsArgs {
     int nelem, npoin;
     size_t EN;
@@ -104,6 +73,7 @@ template <typename T> struct RhsArgs {
     const int *perm; // element-local scratch position of each node
     T *out;          // records of 5 (mass, mom1, mom2, mom3, energy) per element-node;
                      // (e,a) at record e*NN + perm[a]
+    int run, wide;   // unit_range of k_rhs
     int geo16;       // He and gpvol blocks of every element are 16-byte aligned
     // brick-local assembly of the fused p=3 stage (see ClusterTables): the
     // element order, local-node tables, the partial records of surface nodes,
@@ -132,454 +102,461 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
     return mu_factor * T(0.000001458) * (Tk * sqrt(Tk)) / (Tk + T(110.4));
 }
 
-// CONV: split-form convection (full_convec_ijk); DIFF: viscous operator
+// The operators of one right-hand side on the element pipeline (pipe.hpp).
+// CONV: split-form convection (full_convec_ijk); VISC: viscous operator
 // (full_diffusion_ijk); CONS: inputs are the conserved FP64 state (the fused
 // stage forms the primitives of updateF's EOS block and Sutherland's viscosity
 // in-kernel) instead of the primitive arrays.
 //
-// Per element (one lane per node / quadrature point), in phases that keep the
-// live register set small (values cross phases through LDS):
-//   stage   nodal fields -> LDS;
-//   conv    velocity lines: d/dxi u_i, the contravariant line weights
-//           W_k(m) = D_k(m) sum_j He_g(j,k) u_j(m), div(u_i u), div u; then the
-//           density, pressure, H, rho*H and momentum lines against W;
-//   diff 1  density, temperature and velocity lines -> grad rho, grad T, grad u
-//           -> viscous fluxes mapped to contravariant components
-//           G_k(F) = gpvol sum_d He(d,k) F_d, staged in LDS;
-//   diff 2  weak divergence sum_k sum_{b on k-line} dl(b,k,I_k(a)) G_k(F)(b)
-//           with the transposed coefficients kept per lane in LDS;
-//   out     residuals written to the element's scratch block.
-template <int P, typename T, bool CONV, bool DIFF, bool CONS>
-__global__ __launch_bounds__(EG<P>::NT, 2) void k_rhs(RhsArgs<T> A)
+// Convection in two line coefficients.  With D_k(m) the derivative row of the
+// lane's k-line, U_k = sum_j He(j,k) u_j(own), Q_k the same of q, and
+// U_k(m) = sum_j He(j,k) u_j(m) at the line node m, the split form's terms
+//   rho div(s u) + q.grad s   (s = u_i and H)     carry  E_k(m) = D_k(m) (Q_k + rho U_k(m)),
+//   div(s u) + u.grad s       (s = q_i and rho H) carry  C_k(m) = D_k(m) (U_k + U_k(m)),
+// so each of the eight fields costs one multiply-add per line node, and no
+// line weight is kept: 22 multiply-adds per line node, where separate
+// derivatives and W-weighted sums took 36 and held the weights in registers.
+//
+// Per unit, in phases (a workgroup of one wave has no barriers):
+//   in      the unit's geometry (LDS), state (registers) and node ids (LDS) have
+//           arrived; He and gpvol go to registers, the previous unit's residual
+//           records leave LDS, and the copies and gathers of the next units start;
+//   stage   nodal records -> LDS: u1 u2 | u3 rho | p H | rhoH q1 | q2 q3 (80 bytes
+//           in FP64: 16 consecutive records start in 16 different banks);
+//   lines   convection and the line derivatives of u, rho and T;
+//   fluxes  G_k(F) = gpvol sum_d He(d,k) F_d -> LDS over the nodal records, the own
+//           node's share of the weak divergence kept in registers;
+//   weak    sum_k sum_b dl(b,k,I_k(a)) G_k(F)(b);
+//   out     residual records -> LDS, dense, written by the next "in".
+//
+// What bounds it: the convection moves 8 GB between L1 and L2 at 553k elements, p=3
+// (5 GB of them from HBM) and waits for them most of the time; it runs at about
+// 5 TB/s of HBM traffic against 5.7 TB/s of a large copy.  The viscous operator adds
+// the element-fastest mu arrays (64 lines per element and array), the kernel of both
+// operators LDS reads (51 of 16 bytes per lane at p=4) and FP64 arithmetic.  Against
+// one element per workgroup in gmsh lane order with W-weighted sums, and geometry
+// in 4-byte rows at odd p=4 elements (kernel times, one box):
+//   p=3 FP64, 553k elements: convection 1.64 -> 1.25 ms, viscous 1.94 -> 1.54 ms
+//   p=4 FP64,  63k elements: convection 0.77 -> 0.34 ms, viscous 0.80 -> 0.34 ms
+//   p=4 FP32,  46k elements: convection 0.30 -> 0.15 ms, viscous 0.36 -> 0.18 ms
+//   both, fused stage: p=4 FP64, 48k elements 1.57 -> 0.42 ms (it spilled 124
+//   registers); p=2 FP64, 152k elements 0.47 -> 0.16 ms
+template <int P, typename T, bool CONV, bool VISC> struct ElemLDS {
+    using Q = EP<P, T>;
+    // nodal records (values), flux records and residual records share one area
+    // of one stride, so that a line neighbour has one LDS offset
+    static constexpr int REC = VISC ? 18 : 10, AREA = REC * Q::NT;
+    // at p=4 the transposed coefficients of both operators' kernel do not fit in
+    // the registers beside the rest: they stay in LDS, one column per lane
+    static constexpr bool TLDS = CONV && VISC && P == 4;
+};
+
+// waves per SIMD asked of the compiler: the FP64 kernels hold He, the three
+// derivative rows and the unit's state in registers
+template <int P, typename T, bool CONV, bool VISC> constexpr int elem_waves()
 {
-    constexpr int N1 = EG<P>::N1, NN = EG<P>::NN, NT = EG<P>::NT;
-    constexpr int F_RHO = 0, F_U = 1, F_T = 4;
-    constexpr int F_C = DIFF ? 5 : 4; // first convection-only field
-    constexpr int F_P = F_C, F_H = F_C + 1, F_RH = F_C + 2, F_Q = F_C + 3;
-    constexpr int NF1 = CONV ? F_C + 6 : F_C;
-    constexpr int NF2 = DIFF ? 18 : 0;
-    // nodal fields (s1) and contravariant viscous fluxes (s2): the fluxes are
-    // staged while the convective lines still read the nodal fields
-    __shared__ T s1[NF1 * NT];
-    __shared__ T s2[(NF2 > 0 ? NF2 : 1) * NT];
+    return sizeof(T) == 4 ? 3 : 2;
+}
 
-    const int lane = threadIdx.x;
-    const bool act = lane < NN;
-    const int a = act ? lane : 0;
-    LineTab<P, T> lt;
-    build_linetab<P, T>(a, A.dl, A.inv, A.gI, A.gJ, A.gK, lt);
-    const int pa = min(max(A.perm[a], 0), NN - 1); // scratch position within the element
-    // line derivative d/dxi_k of LDS field f at the lane's point
-    auto dxi = [&](int f, int k, T own) {
-        T v = lt.ds[k] * own;
-#pragma unroll
-        for (int o = 0; o < P; ++o) v += lt.d[k][o] * s1[f * NT + lt.off[k][o]];
-        return v;
+template <int P, typename T, bool CONV, bool VISC, bool CONS>
+__global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) void k_rhs(RhsArgs<T> A)
+{
+    using Q = EP<P, T>;
+    using L = ElemLDS<P, T, CONV, VISC>;
+    using V2 = T __attribute__((ext_vector_type(2)));
+    constexpr int NN = Q::NN, NL = Q::NL, NT = Q::NT, NE = Q::NE, NW = Q::NW, G = Q::G;
+    constexpr int REC = L::REC;
+    __shared__ __attribute__((aligned(16))) T area_s[G * L::AREA];
+    __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * Q::GEO];
+    __shared__ int conn_s[G * 2 * NT];
+    // this thread's unit of the group, and its LDS
+    const int sb = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    T *const area = area_s + sb * L::AREA;
+    unsigned char *const geo = geo_s + sb * Q::GEO;
+    int *const conn = conn_s + sb * 2 * NT;
+    const unsigned geo_at = lds_addr(geo_s) + sb * Q::GEO;
+    const unsigned conn_at = lds_addr(conn_s) + sb * 2 * NT * 4;
+    const int lane = threadIdx.x % NT, wl = lane & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(lane >> 6);
+
+    const int nunits = (A.nelem + NE - 1) / NE;
+    // over groups of G consecutive units; past the last unit it is evaluated
+    // again, and not stored
+    const UnitRange er = unit_range((nunits + G - 1) / G, A.run, A.wide);
+    auto unit = [&](int g) { return min(g * G + sb, nunits - 1); };
+    if (er.begin >= er.end) return;
+    const int ulast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
+    const LexLane<P, T, VISC> ln(lane, A.dl, A.inv, A.perm);
+    const size_t EN = (size_t)A.nelem * NN, np = (size_t)A.npoin;
+    auto conn_issue = [&](int u, int slot) {
+        const size_t i = (size_t)u * NL + lane;
+        dma_lds<4>(A.connecT + (i < EN ? i : EN - 1), conn_at + (slot * NT + wv * 64) * 4);
     };
+    __shared__ T tcol[L::TLDS ? 3 * P * Q::NT : 1];
+    if constexpr (L::TLDS)
+        if (sb == 0)
+#pragma unroll
+            for (int i = 0; i < 3 * P; ++i) tcol[i * NT + lane] = ln.t[i / P][i % P];
+    int nb[3][P]; // LDS offsets of the line neighbours' records
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int o = 0; o < P; ++o) nb[k][o] = ln.nb[k][o] * REC;
+    auto ld2 = [&](int i) { return *(const V2 *)(area + i); };
+    auto st2 = [&](int i, T x, T y) { *(V2 *)(area + i) = V2{x, y}; };
 
-    // Inputs of one element at the lane's node; the next element's are loaded
-    // while the current one is computed (software pipelining of the global
-    // loads, whose latency would otherwise be exposed at low occupancy).
+    // inputs of one unit at the lane's node (loaded one unit ahead)
     struct In {
-        double cr, cq[3], cE;                // conserved state (CONS)
+        double cr, cq[3], cE;                     // conserved state (CONS)
         T rho, u[3], q[3], pr, E, Tem, rhon, muf; // primitive inputs (drop-in)
         T mue, musgs;
     };
-    auto load = [&](In &x, int e, int n) {
-        const size_t ea = (size_t)e * NN + a;
+    auto load = [&](In &x, int u, int slot) {
+        const int n = conn[slot * NT + ln.sub * NN + ln.a];
         if constexpr (CONS) {
             x.cr = A.cr[n];
             x.cq[0] = A.cq[n];
-            x.cq[1] = A.cq[n + A.npoin];
-            x.cq[2] = A.cq[n + 2 * (size_t)A.npoin];
+            x.cq[1] = A.cq[n + np];
+            x.cq[2] = A.cq[n + 2 * np];
             x.cE = A.cE[n];
         } else {
             x.rho = A.rho[n];
 #pragma unroll
-            for (int d = 0; d < 3; ++d) x.u[d] = A.u[n + (size_t)A.npoin * d];
+            for (int d = 0; d < 3; ++d) x.u[d] = A.u[n + np * d];
             if constexpr (CONV) {
 #pragma unroll
-                for (int d = 0; d < 3; ++d) x.q[d] = A.q[n + (size_t)A.npoin * d];
+                for (int d = 0; d < 3; ++d) x.q[d] = A.q[n + np * d];
                 x.pr = A.pr[n];
                 x.E = A.E[n];
             }
-            if constexpr (DIFF) {
+            if constexpr (VISC) {
                 x.Tem = A.Tem[n];
                 x.rhon = A.rho_n[n];
                 x.muf = A.mu_fluid[n];
-                x.musgs = A.mu_sgs ? A.mu_sgs[e + (size_t)A.nelem * a] : T(0);
             }
         }
-        if constexpr (DIFF) x.mue = A.mu_e[e + (size_t)A.nelem * a];
+        if constexpr (VISC) {
+            const size_t eg = (size_t)min(u * NE + ln.sub, A.nelem - 1) + (size_t)A.nelem * ln.a;
+            x.mue = A.mu_e[eg];
+            if constexpr (!CONS) x.musgs = A.mu_sgs ? A.mu_sgs[eg] : T(0);
+        }
+    };
+    // the dense residual records of unit u (in `area`) to its block of A.out:
+    // read into registers, then stored SB contiguous bytes per lane
+    constexpr int SB = gcd16(5 * NL * (int)sizeof(T)), CH = 5 * NL * (int)sizeof(T) / SB,
+                  NC = (CH + NT - 1) / NT;
+    using U4 = unsigned __attribute__((ext_vector_type(4)));
+    using U2 = unsigned __attribute__((ext_vector_type(2)));
+    using SV = std::conditional_t<SB == 16, U4, std::conditional_t<SB == 8, U2, unsigned>>;
+    auto rec_read = [&](SV v[NC]) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[i] = ((const SV *)area)[min(lane + i * NT, CH - 1)];
+    };
+    auto rec_store = [&](const SV v[NC], int u) {
+        SV *o = (SV *)(A.out + (size_t)u * 5 * NL);
+        if (NE == 1 || (u + 1) * NE <= A.nelem) {
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                if (lane + i * NT < CH) o[lane + i * NT] = v[i];
+        } else { // the odd last element of a unit of two
+            const T *s = area;
+            for (int i = lane; i < 5 * NN; i += NT) ((T *)o)[i] = s[i];
+        }
     };
 
-    // Geometry of one element (He, then gpvol) is copied HBM -> LDS by the
-    // direct-to-LDS loads of gfx950 (no registers involved), one element ahead:
-    // the copy of element e+stride runs during the arithmetic of element e.  A
-    // wave instruction copies one row of 64 lanes x W bytes (W = 16 when the
-    // per-element blocks are 16-byte aligned, else 4); the waves of the
-    // workgroup take alternate rows.
-    constexpr int HE_BYTES = 9 * NN * (int)sizeof(T), GV_BYTES = NN * (int)sizeof(T);
-    constexpr int NW = NT / 64;
-    constexpr int ROWS16 = (HE_BYTES + GV_BYTES + 1023) / 1024;
-    constexpr int ROWS4 = (HE_BYTES + GV_BYTES + 255) / 256;
-    __shared__ __attribute__((aligned(16))) unsigned char
-        geo[(ROWS16 * 1024 > ROWS4 * 256 ? ROWS16 * 1024 : ROWS4 * 256)];
-    const int wl = lane & 63, wv = lane >> 6;
-    auto geo_issue = [&](int e) {
-        const unsigned char *he = (const unsigned char *)(A.He + (size_t)e * 9 * NN);
-        const unsigned char *gv = (const unsigned char *)(A.gpvol + (size_t)e * NN);
-        if (A.geo16)
-            geo_copy<16, HE_BYTES, GV_BYTES, NW>(he, gv, geo, wl, wv);
-        else
-            geo_copy<4, HE_BYTES, GV_BYTES, NW>(he, gv, geo, wl, wv);
-    };
-    auto esync = [&]() { lds_barrier(); };
-    constexpr int WAIT_VM0 = kWaitVm0, WAIT_LGKM0 = kWaitLgkm0;
-
-    const ElemRange er = elem_range(A.nelem);
-    if (er.begin >= er.end) return;
-    // element indices past the block's range are clamped to its last element:
-    // the extra loads are harmless and keep the load stream unconditional
-    const int elast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
     In cur, nxt;
-    geo_issue(er.begin);
-    load(cur, er.begin, A.connecT[(size_t)er.begin * NN + a]);
-    int n_nx = A.connecT[(size_t)min(er.begin + er.stride, elast) * NN + a];
-    for (int e = er.begin; e < er.end; e += er.stride) {
-        const int e2 = min(e + er.stride, elast), e3 = min(e + 2 * er.stride, elast);
-        // geometry of element e: wait for its copy (and the state loads issued
-        // with it), move it to registers, then start the copies of element e2
-        __builtin_amdgcn_s_waitcnt(WAIT_VM0);
-        esync();
+    GeoAt at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, unit(er.begin), geo_at, wl, wv);
+    conn_issue(unit(er.begin), 0);
+    conn_issue(unit(min(er.begin + er.stride, ulast)), 1);
+    wait_vm<0>();
+    lds_barrier();
+    load(cur, unit(er.begin), 0);
+    int slot = 1, prev = -1;
+    for (int g = er.begin; g < er.end; g += er.stride, slot ^= 1) {
+        const int u = unit(g), u2 = unit(min(g + er.stride, ulast)),
+                  u3 = unit(min(g + 2 * er.stride, ulast));
+        // ---------------- in
+        wait_vm<0>();
+        lds_barrier();
         T He[3][3];
         {
-            const T *hp = (const T *)geo + 9 * a;
+            const T *hp = (const T *)(geo + at.he) + 9 * (ln.sub * NN + ln.a);
 #pragma unroll
             for (int j = 0; j < 3; ++j)
 #pragma unroll
                 for (int i = 0; i < 3; ++i) He[i][j] = hp[i + 3 * j];
         }
-        const T vol = ((const T *)geo)[9 * NN + a];
-        __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-        esync();
-        geo_issue(e2);
-        load(nxt, e2, n_nx);
-        const int n_nx2 = A.connecT[(size_t)e3 * NN + a];
-        T mue = T(0), musgs = T(0), muf = T(0), rhon = T(0);
-        if constexpr (DIFF) mue = cur.mue;
-        // ---------------- stage own node values
-        {
-            T rho, u[3], Tk = T(0), p = T(0), H = T(0), rhoH = T(0), q[3] = {T(0), T(0), T(0)};
-            if constexpr (CONS) {
-                const double r = cur.cr;
-                const double ri = 1.0 / r;
-                double ud[3], umag = 0.0;
+        const T vol = ((const T *)(geo + Q::HEA + at.gv))[ln.sub * NN + ln.a];
+        SV out[NC];
+        rec_read(out);
+        lds_done();
+        if (prev >= 0) rec_store(out, prev);
+        load(nxt, u2, slot);
+        unit_sync<NW>();
+        at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
+        conn_issue(u3, slot ^ 1);
+        prev = g * G + sb < nunits ? u : -1;
+        // ---------------- stage
+        T rho, v[3], q[3] = {0, 0, 0}, H = 0, rhoH = 0, p = 0, Tk = 0, muf = 0, rhon = 0, musgs = 0;
+        const T mue = VISC ? cur.mue : T(0);
+        if constexpr (CONS) {
+            const double r = cur.cr, ri = 1.0 / r;
+            double ud[3], umag = 0.0;
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    ud[d] = cur.cq[d] * ri;
-                    umag += ud[d] * ud[d];
-                }
-                const double eint = cur.cE * ri - 0.5 * umag;
-                const double pd = r * (A.gamma - 1.0) * eint;
-                const double hd = (A.gamma / (A.gamma - 1.0)) * pd * ri;
-                const double Td = pd * ri / A.Rgas;
-                rho = T(r);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    u[d] = T(ud[d]);
-                    q[d] = T(cur.cq[d]);
-                }
-                // only grad p enters: a uniform reference pressure is removed
-                // before the (possibly FP32) operator arithmetic
-                p = T(pd - A.p_ref);
-                H = T(hd + 0.5 * umag);
-                rhoH = T(r * (hd + 0.5 * umag));
-                Tk = T(Td);
-                rhon = rho;
-                muf = T(sutherland<double>(A.mu_factor_e ? A.mu_factor_e[e] : A.mu_factor, Td));
-            } else {
-                rho = cur.rho;
-#pragma unroll
-                for (int d = 0; d < 3; ++d) u[d] = cur.u[d];
-                if constexpr (CONV) {
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) q[d] = cur.q[d];
-                    p = cur.pr;
-                    const T kin = u[0] * u[0] * T(0.5) + u[1] * u[1] * T(0.5) + u[2] * u[2] * T(0.5);
-                    H = cur.E + kin;
-                    rhoH = rho * H;
-                }
-                if constexpr (DIFF) {
-                    Tk = cur.Tem;
-                    rhon = cur.rhon;
-                    muf = cur.muf;
-                    musgs = cur.musgs;
-                }
+            for (int d = 0; d < 3; ++d) {
+                ud[d] = cur.cq[d] * ri;
+                umag += ud[d] * ud[d];
             }
-            if (act) {
-                s1[F_RHO * NT + a] = rho;
+            const double eint = cur.cE * ri - 0.5 * umag;
+            const double pd = r * (A.gamma - 1.0) * eint;
+            const double hd = (A.gamma / (A.gamma - 1.0)) * pd * ri;
+            const double Td = pd * ri / A.Rgas;
+            rho = T(r);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) s1[(F_U + d) * NT + a] = u[d];
-                if constexpr (DIFF) s1[F_T * NT + a] = Tk;
-                if constexpr (CONV) {
-                    s1[F_P * NT + a] = p;
-                    s1[F_H * NT + a] = H;
-                    s1[F_RH * NT + a] = rhoH;
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) s1[(F_Q + d) * NT + a] = q[d];
-                }
+            for (int d = 0; d < 3; ++d) {
+                v[d] = T(ud[d]);
+                q[d] = T(cur.cq[d]);
             }
-        }
-        esync();
-
-        T Rm = 0, Rq[3] = {0, 0, 0}, Re = 0;
-        T gR[3] = {0, 0, 0};                           // DIFF: grad rho
-        T gU[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}; // DIFF: gU[i][j] = d u_i / d x_j
-        const T rho = s1[F_RHO * NT + a];
-        T u[3];
+            // only grad p enters: a uniform reference pressure is removed
+            // before the (possibly FP32) operator arithmetic
+            p = T(pd - A.p_ref);
+            H = T(hd + 0.5 * umag);
+            rhoH = T(r * (hd + 0.5 * umag));
+            Tk = T(Td);
+            rhon = rho;
+            muf = T(sutherland<double>(
+                A.mu_factor_e ? A.mu_factor_e[min(u * NE + ln.sub, A.nelem - 1)] : A.mu_factor, Td));
+        } else {
+            rho = cur.rho;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) u[i] = s1[(F_U + i) * NT + a];
-        // ---------------- velocity lines: d/dxi u_i (-> grad u) and, for the
-        // convection, the contravariant line weights W and div(u_i u), div u
-        T Wo[3], Wx[3][P];
-        T divUw = 0;
-        {
-            T q[3] = {0, 0, 0}, Qt[3] = {0, 0, 0}, Ut[3] = {0, 0, 0}, divFuu[3] = {0, 0, 0};
+            for (int d = 0; d < 3; ++d) v[d] = cur.u[d];
             if constexpr (CONV) {
 #pragma unroll
-                for (int i = 0; i < 3; ++i) q[i] = s1[(F_Q + i) * NT + a];
+                for (int d = 0; d < 3; ++d) q[d] = cur.q[d];
+                p = cur.pr;
+                H = cur.E + (v[0] * v[0] * T(0.5) + v[1] * v[1] * T(0.5) + v[2] * v[2] * T(0.5));
+                rhoH = rho * H;
+            }
+            if constexpr (VISC) {
+                Tk = cur.Tem;
+                rhon = cur.rhon;
+                muf = cur.muf;
+                musgs = cur.musgs;
+            }
+        }
+        // (lanes without a node write records of their own past the unit's: a
+        // condition here would let the compiler sink the arithmetic behind it)
+        const int own = lane * REC;
+        st2(own, v[0], v[1]);
+        st2(own + 2, v[2], rho);
+        if constexpr (CONV) {
+            st2(own + 4, p, H);
+            st2(own + 6, rhoH, q[0]);
+            st2(own + 8, q[1], q[2]);
+        }
+        if constexpr (VISC) area[own + 10] = Tk;
+        unit_sync<NW>();
+
+        // ---------------- lines
+        T Rm = 0, Rq[3] = {0, 0, 0}, Re = 0;
+        T du[3][3], dT[3]; // d u_i / d xi_k, d T / d xi_k
+        T gR[3];           // grad rho
+        {
+            T Ut[3] = {0, 0, 0}, Qt[3] = {0, 0, 0};
+            T divU = 0, divQ = 0, dr[3], dp[3];
+            // Sums start with the own node's share.  FP32 sums the differences to the
+            // own node's values (whose share is then the row sum rs of D, zero but for
+            // rounding), so that a field's mean costs no digits of its derivative.
+            // FP64 has digits to spare and sums the values.
+            constexpr bool DELTA = sizeof(T) == 4;
+            T rs[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                double r = ln.ds[k]; // in 64 bits: the coefficients all but cancel
+                if constexpr (DELTA)
+#pragma unroll
+                    for (int o = 0; o < P; ++o) r += ln.d[k][o];
+                rs[k] = T(r);
+            }
+            T a0 = 0, b0 = 0;
+            if constexpr (CONV) {
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    Ut[k] = He[0][k] * u[0] + He[1][k] * u[1] + He[2][k] * u[2];
+                    Ut[k] = He[0][k] * v[0] + He[1][k] * v[1] + He[2][k] * v[2];
                     Qt[k] = He[0][k] * q[0] + He[1][k] * q[1] + He[2][k] * q[2];
+                    a0 += rs[k] * Ut[k];
+                    b0 += rs[k] * Qt[k];
                 }
+                divU = a0;
+                divQ = b0;
             }
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const T c0 = lt.ds[k];
-                T du[3];
+                // sums of one line first: shorter chains of roundings
+                T rq[3] = {0, 0, 0}, re = 0, dvu = 0, dvq = 0;
+                // E = c (eb + rho u'), C = c (cb + u') with u' = U_k(m), or its
+                // difference to U_k
+                const T eb = DELTA ? Qt[k] + rho * Ut[k] : Qt[k], cb = DELTA ? T(2) * Ut[k] : Ut[k];
+                dr[k] = rs[k] * rho;
+                if constexpr (CONV) dp[k] = rs[k] * p;
+                if constexpr (VISC) {
+                    dT[k] = rs[k] * Tk;
 #pragma unroll
-                for (int i = 0; i < 3; ++i) du[i] = c0 * u[i];
-                if constexpr (CONV) {
-                    Wo[k] = c0 * Ut[k];
-                    divUw += Wo[k];
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) divFuu[i] += Wo[k] * u[i];
+                    for (int i = 0; i < 3; ++i) du[i][k] = rs[k] * v[i];
                 }
 #pragma unroll
                 for (int o = 0; o < P; ++o) {
-                    const int b = lt.off[k][o];
-                    const T c = lt.d[k][o];
-                    T ub[3];
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) {
-                        ub[i] = s1[(F_U + i) * NT + b];
-                        du[i] += c * ub[i];
+                    const int b = nb[k][o];
+                    const T c = ln.d[k][o];
+                    V2 x01 = ld2(b), x2r = ld2(b + 2);
+                    if constexpr (DELTA) {
+                        x01 -= V2{v[0], v[1]};
+                        x2r -= V2{v[2], rho};
                     }
+                    dr[k] += c * x2r.y;
                     if constexpr (CONV) {
-                        const T w = c * (He[0][k] * ub[0] + He[1][k] * ub[1] + He[2][k] * ub[2]);
-                        Wx[k][o] = w;
-                        divUw += w;
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) divFuu[i] += w * ub[i];
+                        V2 xpH = ld2(b + 4), xHq = ld2(b + 6), xqq = ld2(b + 8);
+                        if constexpr (DELTA) {
+                            xpH -= V2{p, H};
+                            xHq -= V2{rhoH, q[0]};
+                            xqq -= V2{q[1], q[2]};
+                        }
+                        const T ut = He[0][k] * x01.x + He[1][k] * x01.y + He[2][k] * x2r.x;
+                        const T qt = He[0][k] * xHq.y + He[1][k] * xqq.x + He[2][k] * xqq.y;
+                        dvu += c * ut;
+                        dvq += c * qt;
+                        const T C = c * (cb + ut), E = c * (eb + rho * ut);
+                        rq[0] += E * x01.x;
+                        rq[1] += E * x01.y;
+                        rq[2] += E * x2r.x;
+                        re += E * xpH.y;
+                        re += C * xHq.x;
+                        rq[0] += C * xHq.y;
+                        rq[1] += C * xqq.x;
+                        rq[2] += C * xqq.y;
+                        dp[k] += c * xpH.x;
                     }
+                    if constexpr (VISC) {
+                        du[0][k] += c * x01.x;
+                        du[1][k] += c * x01.y;
+                        du[2][k] += c * x2r.x;
+                        dT[k] += c * (DELTA ? area[b + 10] - Tk : area[b + 10]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 if constexpr (CONV) {
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) Rq[i] += Qt[k] * du[i];
-                }
-                if constexpr (DIFF) {
-#pragma unroll
-                    for (int i = 0; i < 3; ++i)
-#pragma unroll
-                        for (int j = 0; j < 3; ++j) gU[i][j] += He[j][k] * du[i];
+                    for (int i = 0; i < 3; ++i) Rq[i] += rq[i];
+                    Re += re;
+                    divU += dvu;
+                    divQ += dvq;
                 }
             }
+            if constexpr (VISC)
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    gR[i] = He[i][0] * dr[0] + He[i][1] * dr[1] + He[i][2] * dr[2];
             if constexpr (CONV) {
+                const T urho = Ut[0] * dr[0] + Ut[1] * dr[1] + Ut[2] * dr[2];
+                const T s = divQ + urho;
+                // the own values' coefficients: div q + u.grad rho for u_i and H,
+                // div u for q_i and rho H, and the own share of sum E and sum C (all of
+                // it where differences are summed)
+                const T ce = s + (b0 + rho * (DELTA ? divU : a0));
+                const T cc = DELTA ? T(2) * divU + a0 : divU + T(2) * a0;
+                Rm = vol * (T(0.5) * (s + rho * divU));
+                Re = vol * (T(0.25) * (Re + (H * ce + rhoH * cc)));
 #pragma unroll
-                for (int i = 0; i < 3; ++i) Rq[i] = T(0.25) * (Rq[i] + rho * divFuu[i]);
-            }
-        }
-        // ---------------- density line: grad rho (viscous) and u.grad rho terms
-        // (convection)
-        {
-            const T *sf = s1 + F_RHO * NT;
-            T d[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                T v = lt.ds[k] * rho;
-#pragma unroll
-                for (int o = 0; o < P; ++o) v += lt.d[k][o] * sf[lt.off[k][o]];
-                d[k] = v;
-            }
-            if constexpr (DIFF) {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) gR[i] = He[i][0] * d[0] + He[i][1] * d[1] + He[i][2] * d[2];
-            }
-            if constexpr (CONV) {
-                T Ut[3];
-#pragma unroll
-                for (int k = 0; k < 3; ++k) Ut[k] = He[0][k] * u[0] + He[1][k] * u[1] + He[2][k] * u[2];
-                const T urho = Ut[0] * d[0] + Ut[1] * d[1] + Ut[2] * d[2];
-                Rm += T(0.5) * urho;
-#pragma unroll
-                for (int i = 0; i < 3; ++i) Rq[i] += T(0.25) * u[i] * urho;
-                Re += T(0.25) * s1[F_H * NT + a] * urho;
+                for (int i = 0; i < 3; ++i)
+                    Rq[i] = vol * (T(0.25) * (Rq[i] + (v[i] * ce + q[i] * cc)) +
+                                   (He[i][0] * dp[0] + He[i][1] * dp[1] + He[i][2] * dp[2]));
             }
         }
 
-        // ---------------- viscous fluxes, staged as contravariant components
-        // G_k(F) = gpvol sum_d He(d,k) F_d for the weak divergence of pass 2
-        if constexpr (DIFF) {
-            const T mufg = muf + rhon * musgs;
-            const T mut = mufg + mue;
-            const T divU = gU[0][0] + gU[1][1] + gU[2][2];
-            const T tt = mufg * T(2.0 / 3.0) * divU;
-            T tau[3][3];
+        if constexpr (VISC) {
+            // ---------------- fluxes.  Record per k: grad rho, grad T | tau u, tau_1 |
+            // tau_2, tau_3 (contravariant, times gpvol)
+            T W[6] = {0, 0, 0, 0, 0, 0};
+            {
+                T tau[3][3], gt[3];
+                const T mufg = muf + rhon * musgs, mut = mufg + mue;
+                T gU[3][3];
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
+                for (int i = 0; i < 3; ++i)
 #pragma unroll
-                for (int j = 0; j < 3; ++j) tau[i][j] = mut * (gU[i][j] + gU[j][i]);
+                    for (int j = 0; j < 3; ++j)
+                        gU[i][j] = He[j][0] * du[i][0] + He[j][1] * du[i][1] + He[j][2] * du[i][2];
+                const T tt = mufg * T(2.0 / 3.0) * (gU[0][0] + gU[1][1] + gU[2][2]);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) tau[i][i] -= tt;
-            T dT[3];
-            const T Tk = s1[F_T * NT + a];
+                for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int k = 0; k < 3; ++k) dT[k] = dxi(F_T, k, Tk);
-            T gt[3];
+                    for (int j = 0; j < 3; ++j) tau[i][j] = mut * (gU[i][j] + gU[j][i]);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) gt[i] = He[i][0] * dT[0] + He[i][1] * dT[1] + He[i][2] * dT[2];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const T h0 = vol * He[0][k], h1 = vol * He[1][k], h2 = vol * He[2][k];
-                T tuk = 0;
-#pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    const T g = h0 * tau[r][0] + h1 * tau[r][1] + h2 * tau[r][2];
-                    if (act) s2[(9 + 3 * r + k) * NT + a] = g;
-                    tuk += g * u[r]; // tau is symmetric: contravariant (tau u)_k
+                for (int i = 0; i < 3; ++i) {
+                    tau[i][i] -= tt;
+                    gt[i] = He[i][0] * dT[0] + He[i][1] * dT[1] + He[i][2] * dT[2];
                 }
-                if (act) {
-                    s2[(6 + k) * NT + a] = tuk;
-                    s2[(0 + k) * NT + a] = h0 * gR[0] + h1 * gR[1] + h2 * gR[2];
-                    s2[(3 + k) * NT + a] = h0 * gt[0] + h1 * gt[1] + h2 * gt[2];
-                }
-            }
-        }
-
-        // ---------------- convective scalar and momentum lines, one field per
-        // (rolled) iteration: line derivative d and the W-weighted line sum
-        // `div` = div(s u) folded at once into the residuals
-        T divQ = 0;
-        if constexpr (CONV) {
-#pragma unroll 1
-            for (int fi = 1; fi < 7; ++fi) { // p, H, rhoH, q1, q2, q3
-                const int f = fi == 1 ? F_P : (fi == 2 ? F_H : (fi == 3 ? F_RH : F_Q + fi - 4));
-                const T *sf = s1 + f * NT;
-                const T own = sf[a];
-                T d[3], div = 0;
+                if constexpr (NW > 1) lds_barrier(); // every wave has read the nodal records
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    T v = lt.ds[k] * own, w = Wo[k] * own;
+                    const T h0 = vol * He[0][k], h1 = vol * He[1][k], h2 = vol * He[2][k];
+                    T F[6];
+                    F[2] = 0;
 #pragma unroll
-                    for (int o = 0; o < P; ++o) {
-                        const T x = sf[lt.off[k][o]];
-                        v += lt.d[k][o] * x;
-                        w += Wx[k][o] * x;
+                    for (int r = 0; r < 3; ++r) {
+                        F[3 + r] = h0 * tau[r][0] + h1 * tau[r][1] + h2 * tau[r][2];
+                        F[2] += F[3 + r] * v[r]; // tau is symmetric: contravariant (tau u)_k
                     }
-                    d[k] = v;
-                    div += w;
-                }
-                if (fi == 1) {
+                    F[0] = h0 * gR[0] + h1 * gR[1] + h2 * gR[2];
+                    F[1] = h0 * gt[0] + h1 * gt[1] + h2 * gt[2];
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) Rq[i] += He[i][0] * d[0] + He[i][1] * d[1] + He[i][2] * d[2];
-                } else if (fi == 2) { // H: q.grad H + rho div(H u)
-                    T qt = 0;
-#pragma unroll
-                    for (int k = 0; k < 3; ++k)
-                        qt += (He[0][k] * s1[F_Q * NT + a] + He[1][k] * s1[(F_Q + 1) * NT + a] +
-                               He[2][k] * s1[(F_Q + 2) * NT + a]) * d[k];
-                    Re += T(0.25) * (qt + rho * div);
-                } else { // rho H, q_i: u.grad s + div(s u)
-                    T ut = 0;
-#pragma unroll
-                    for (int k = 0; k < 3; ++k)
-                        ut += (He[0][k] * u[0] + He[1][k] * u[1] + He[2][k] * u[2]) * d[k];
-                    const T c = T(0.25) * (ut + div);
-                    if (fi == 3) {
-                        Re += c;
-                    } else {
-                        const int i = fi - 4;
-                        const T dq = He[i][0] * d[0] + He[i][1] * d[1] + He[i][2] * d[2];
-                        divQ += dq;
-                        if (i == 0) Rq[0] += c;
-                        else if (i == 1) Rq[1] += c;
-                        else Rq[2] += c;
-                    }
+                    for (int f = 0; f < 6; ++f) W[f] += ln.ds[k] * F[f];
+                    st2(own + 6 * k, F[0], F[1]);
+                    st2(own + 6 * k + 2, F[2], F[3]);
+                    st2(own + 6 * k + 4, F[4], F[5]);
                 }
             }
-        }
-        if constexpr (CONV) {
-            const T H = s1[F_H * NT + a], rhoH = s1[F_RH * NT + a];
-            Rm += T(0.5) * (divQ + rho * divUw);
+            unit_sync<NW>();
+            // ---------------- weak divergence
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
-                Rq[i] += T(0.25) * (u[i] * divQ + s1[(F_Q + i) * NT + a] * divUw);
-            Re += T(0.25) * (H * divQ + rhoH * divUw);
-            Rm *= vol;
-            Re *= vol;
+            for (int k = 0; k < 3; ++k) {
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) Rq[i] *= vol;
-        }
-
-        // ---------------- viscous operator, pass 2
-        if constexpr (DIFF) {
-            esync(); // every lane's fluxes are in s2
-            // pass 2: weak divergence with the transposed coefficients
-            // dl(b,k,I_k(a)) of the lane's lines
-            T W6[6];
-#pragma unroll 1
-            for (int fl = 0; fl < 6; ++fl) {
-                T acc = 0;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const T *sf = s2 + (3 * fl + k) * NT;
-                    T v = lt.ds[k] * sf[a];
-#pragma unroll
-                    for (int o = 0; o < P; ++o) v += lt.t[k][o] * sf[lt.off[k][o]];
-                    acc += v;
+                for (int o = 0; o < P; ++o) {
+                    const int b = nb[k][o] + 6 * k;
+                    const T c = L::TLDS ? tcol[(k * P + o) * NT + lane] : ln.t[k][o];
+                    const V2 x01 = ld2(b), x23 = ld2(b + 2), x45 = ld2(b + 4);
+                    W[0] += c * x01.x;
+                    W[1] += c * x01.y;
+                    W[2] += c * x23.x;
+                    W[3] += c * x23.y;
+                    W[4] += c * x45.x;
+                    W[5] += c * x45.y;
                 }
-                if (fl == 0) W6[0] = acc;
-                else if (fl == 1) W6[1] = acc;
-                else if (fl == 2) W6[2] = acc;
-                else if (fl == 3) W6[3] = acc;
-                else if (fl == 4) W6[4] = acc;
-                else W6[5] = acc;
             }
-            const T nu_e = A.c_rho * mue / rhon;
+            Rm += A.c_rho * mue / rhon * W[0];
             const T kappa = muf * A.Cp / A.Pr + A.c_ener * mue * A.Cp / A.Pr +
                             A.Cp * rhon * musgs / T(0.9);
-            Rm += nu_e * W6[0];
-            Re += W6[2] + kappa * W6[1];
+            Re += W[2] + kappa * W[1];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) Rq[i] += W6[3 + i];
+            for (int i = 0; i < 3; ++i) Rq[i] += W[3 + i];
         }
-
-        if (act) {
-            T *o = A.out + 5 * ((size_t)e * NN + pa);
-            o[0] = Rm;
-            o[1] = Rq[0];
-            o[2] = Rq[1];
-            o[3] = Rq[2];
-            o[4] = Re;
-        }
+        // ---------------- out
+        unit_sync<NW>(); // every wave is done with the records in `area`
+        T *o = area + 5 * ln.rec;
+        o[0] = Rm;
+        o[1] = Rq[0];
+        o[2] = Rq[1];
+        o[3] = Rq[2];
+        o[4] = Re;
         cur = nxt;
-        n_nx = n_nx2;
-        esync();
     }
-    // no copy may still be writing LDS when the workgroup ends
-    __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+    lds_barrier();
+    SV out[NC];
+    rec_read(out);
+    if (prev >= 0) rec_store(out, prev);
+    // no copy may still be writing this block's LDS when it retires
+    wait_vm<0>();
 }
 
 // generic_scalar_convec_ijk (elem_convec.f90:472-594):
@@ -943,24 +920,6 @@ template <int P, typename T> struct SplitState {
     double cr, cq[3], cE;
     T mue;
 };
-
-// direct-to-LDS copy of W (4 or 16) bytes per lane from g to lds + W*lane
-// (lds wave-uniform), issued outside the compiler's wait tracking
-template <int W> __device__ __forceinline__ void dma_lds(const void *g, unsigned lds)
-{
-    const unsigned m = __builtin_amdgcn_readfirstlane(lds);
-    if constexpr (W == 16)
-        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m) : "memory");
-    else
-        asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "{m0}"(m) : "memory");
-}
-
-// wait until at most N of this wave's vector-memory operations are outstanding
-template <int N> __device__ __forceinline__ void wait_vm()
-{
-    static_assert(N >= 0 && N <= 63, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | kWaitVm0 | ((N >> 4) << 14));
-}
 
 // Copies of element e into the ring slot at LDS address slot and, by wave 0,
 // the connectivity row of element ec to LDS address crow.  n0 and n1 are the
@@ -1807,25 +1766,27 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
 
 template <typename T>
 static int launch_rhs(sodhip_ctx ctx, int porder, bool conv, bool diff, bool cons,
-                      const RhsArgs<T> &A0, int grid)
+                      const RhsArgs<T> &A0)
 {
-    // 16-byte geometry copies need every element's He and gpvol block on a
-    // 16-byte boundary
     RhsArgs<T> A = A0;
-    const size_t nn = (size_t)nnode_of(porder);
-    A.geo16 = ((uintptr_t)A.He % 16 == 0) && ((uintptr_t)A.gpvol % 16 == 0) &&
-              (9 * nn * sizeof(T)) % 16 == 0 && (nn * sizeof(T)) % 16 == 0;
+    // 16-byte geometry copies start from 16-byte boundaries of the arrays
+    A.geo16 = ((uintptr_t)A.He % 16 == 0) && ((uintptr_t)A.gpvol % 16 == 0);
 #define SODHIP_RHS_CASE(PP)                                                                \
-    case PP:                                                                               \
+    case PP: {                                                                             \
+        const UnitShape us = unit_shape<PP, T>(ctx, A.nelem);                              \
+        const int nt = EP<PP, T>::NTB;                                                     \
+        A.run = us.run;                                                                    \
+        A.wide = us.wide;                                                                  \
         if (conv && diff && cons)                                                          \
-            k_rhs<PP, T, true, true, true><<<grid, EG<PP>::NT, 0, ctx->stream>>>(A);       \
+            k_rhs<PP, T, true, true, true><<<us.grid, nt, 0, ctx->stream>>>(A);            \
         else if (conv && !diff && !cons)                                                   \
-            k_rhs<PP, T, true, false, false><<<grid, EG<PP>::NT, 0, ctx->stream>>>(A);     \
+            k_rhs<PP, T, true, false, false><<<us.grid, nt, 0, ctx->stream>>>(A);          \
         else if (!conv && diff && !cons)                                                   \
-            k_rhs<PP, T, false, true, false><<<grid, EG<PP>::NT, 0, ctx->stream>>>(A);     \
+            k_rhs<PP, T, false, true, false><<<us.grid, nt, 0, ctx->stream>>>(A);          \
         else                                                                               \
             return set_error(SODHIP_ERR_UNSUPPORTED, "unsupported operator combination");  \
-        break;
+        break;                                                                             \
+    }
     switch (porder) {
         SODHIP_RHS_CASE(2)
         SODHIP_RHS_CASE(3)
@@ -1897,7 +1858,7 @@ int conv_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *He, c
     A.E = E;
     A.out = out;
     int tok = prof_begin(ctx, 0);
-    const int rc = launch_rhs<T>(ctx, porder, true, false, false, A, elem_grid(ctx, m->nelem, 128));
+    const int rc = launch_rhs<T>(ctx, porder, true, false, false, A);
     prof_end(ctx, tok);
     return rc;
 }
@@ -1943,7 +1904,7 @@ static int full_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const i
     A.E = E;
     A.out = (T *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 0);
-    rc = launch_rhs<T>(ctx, porder, true, false, false, A, elem_grid(ctx, nelem, 128));
+    rc = launch_rhs<T>(ctx, porder, true, false, false, A);
     prof_end(ctx, tok);
     if (rc) return rc;
     tok = prof_begin(ctx, 1);
@@ -1997,7 +1958,7 @@ static int full_diffusion(sodhip_ctx ctx, int porder, int nelem, int npoin, cons
     A.c_ener = c_ener;
     A.out = (T *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 0);
-    rc = launch_rhs<T>(ctx, porder, false, true, false, A, elem_grid(ctx, nelem, 128));
+    rc = launch_rhs<T>(ctx, porder, false, true, false, A);
     prof_end(ctx, tok);
     if (rc) return rc;
     tok = prof_begin(ctx, 1);
@@ -2080,7 +2041,7 @@ int rhs_fused_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *
     }
     if (!done)
 #endif
-        rc = launch_rhs<T>(ctx, porder, true, true, true, A, elem_grid(ctx, m->nelem, 128));
+        rc = launch_rhs<T>(ctx, porder, true, true, true, A);
     prof_end(ctx, tok);
     return rc;
 }
