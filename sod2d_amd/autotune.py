@@ -1,7 +1,7 @@
 """Launch-shape autotuner of the fused Runge-Kutta stage.
 
-The stage's element kernel walks the elements grid-stride, so its grid (blocks
-per CU) sets how many elements each workgroup takes; its geometry moves
+The blocks per CU of the stage's element kernel set how many elements each
+workgroup takes; its geometry moves
 through LDS in 16-byte or 4-byte lane rows (two LDS layouts of the same
 records); the gather/update runs in blocks of 64, 128 or 256 nodes.  None of
 these changes a result.  tune_stage() times every candidate shape on the

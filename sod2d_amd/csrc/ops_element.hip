@@ -116,6 +116,10 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
 // so each of the eight fields costs one multiply-add per line node, and no
 // line weight is kept: 22 multiply-adds per line node, where separate
 // derivatives and W-weighted sums took 36 and held the weights in registers.
+// The fused FP64 stage has q = rho u and rho H itself: with z = D_k(m) (U_k + U_k(m))
+// the two coefficients meet in K = z (rho + rho(m)) on the four fields u_i and H,
+// and div q + u.grad rho = sum z rho(m): 14 multiply-adds and seven values read per
+// line node instead of 22 and eleven.
 //
 // Per unit, in phases (a workgroup of one wave has no barriers):
 //   in      the unit's geometry (LDS), state (registers) and node ids (LDS) have
@@ -139,8 +143,12 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
 //   p=3 FP64, 553k elements: convection 1.64 -> 1.25 ms, viscous 1.94 -> 1.54 ms
 //   p=4 FP64,  63k elements: convection 0.77 -> 0.34 ms, viscous 0.80 -> 0.34 ms
 //   p=4 FP32,  46k elements: convection 0.30 -> 0.15 ms, viscous 0.36 -> 0.18 ms
-//   both, fused stage: p=4 FP64, 48k elements 1.57 -> 0.42 ms (it spilled 124
-//   registers); p=2 FP64, 152k elements 0.47 -> 0.16 ms
+//   both, fused stage: p=4 FP64, 48k elements 1.57 -> 0.30 ms (it spilled 124
+//   registers; 0.42 ms with q and rho H as fields of their own); p=2 FP64, 152k elements
+//   0.47 -> 0.15 ms; p=3 FP64, 262k elements 0.83 -> 0.76 ms and p=3 with FP32
+//   operators, 87k elements 0.21 -> 0.17 ms against two waves per element, one per
+//   operator, that hand over through LDS.  At p=3 FP64 the vector ALU is busy 42 %
+//   and LDS 38 % of the time with two waves per SIMD.
 template <int P, typename T, bool CONV, bool VISC> struct ElemLDS {
     using Q = EP<P, T>;
     // nodal records (values), flux records and residual records share one area
@@ -150,6 +158,15 @@ template <int P, typename T, bool CONV, bool VISC> struct ElemLDS {
     // the registers beside the rest: they stay in LDS, one column per lane
     static constexpr bool TLDS = CONV && VISC && P == 4;
 };
+
+// Values per residual record of the fused stage's element kernel.  With FP32
+// operators at p=3 the five residuals are padded to six, so that a record starts on
+// an 8-byte boundary and the stage's gather reads it with three 8-byte loads (the
+// gather then takes 0.25 instead of 0.43 ms at 64^3 elements); in FP64 the 20 %
+// larger records cost the element kernel more than the gather gains, and the
+// drop-in operators' FP32 gather gains nothing (p=4, 46k elements: 51 us against
+// 47 us with five).
+template <int P, typename T> constexpr int stage_rw() { return sizeof(T) == 4 && P == 3 ? 6 : 5; }
 
 // waves per SIMD asked of the compiler: the FP64 kernels hold He, the three
 // derivative rows and the unit's state in registers
@@ -165,7 +182,12 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     using L = ElemLDS<P, T, CONV, VISC>;
     using V2 = T __attribute__((ext_vector_type(2)));
     constexpr int NN = Q::NN, NL = Q::NL, NT = Q::NT, NE = Q::NE, NW = Q::NW, G = Q::G;
-    constexpr int REC = L::REC;
+    constexpr int REC = L::REC, RW = CONS ? stage_rw<P, T>() : 5;
+    // q = rho u and rho H formed from the other values, in FP64 only: in FP32 the
+    // separately rounded q and u average their rounding errors (q of a 0.2-Mach flow
+    // is 20 to 45 % less exact without)
+    constexpr bool RHOU = CONS && sizeof(T) == 8;
+    constexpr int TEM = 10; // temperature's place in the nodal record
     __shared__ __attribute__((aligned(16))) T area_s[G * L::AREA];
     __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * Q::GEO];
     __shared__ int conn_s[G * 2 * NT];
@@ -243,7 +265,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     };
     // the dense residual records of unit u (in `area`) to its block of A.out:
     // read into registers, then stored SB contiguous bytes per lane
-    constexpr int SB = gcd16(5 * NL * (int)sizeof(T)), CH = 5 * NL * (int)sizeof(T) / SB,
+    constexpr int SB = gcd16(RW * NL * (int)sizeof(T)), CH = RW * NL * (int)sizeof(T) / SB,
                   NC = (CH + NT - 1) / NT;
     using U4 = unsigned __attribute__((ext_vector_type(4)));
     using U2 = unsigned __attribute__((ext_vector_type(2)));
@@ -253,14 +275,14 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         for (int i = 0; i < NC; ++i) v[i] = ((const SV *)area)[min(lane + i * NT, CH - 1)];
     };
     auto rec_store = [&](const SV v[NC], int u) {
-        SV *o = (SV *)(A.out + (size_t)u * 5 * NL);
+        SV *o = (SV *)(A.out + (size_t)u * RW * NL);
         if (NE == 1 || (u + 1) * NE <= A.nelem) {
 #pragma unroll
             for (int i = 0; i < NC; ++i)
                 if (lane + i * NT < CH) o[lane + i * NT] = v[i];
         } else { // the odd last element of a unit of two
             const T *s = area;
-            for (int i = lane; i < 5 * NN; i += NT) ((T *)o)[i] = s[i];
+            for (int i = lane; i < RW * NN; i += NT) ((T *)o)[i] = s[i];
         }
     };
 
@@ -349,12 +371,12 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         const int own = lane * REC;
         st2(own, v[0], v[1]);
         st2(own + 2, v[2], rho);
-        if constexpr (CONV) {
-            st2(own + 4, p, H);
+        if constexpr (CONV) st2(own + 4, p, H);
+        if constexpr (CONV && !RHOU) {
             st2(own + 6, rhoH, q[0]);
             st2(own + 8, q[1], q[2]);
         }
-        if constexpr (VISC) area[own + 10] = Tk;
+        if constexpr (VISC) area[own + TEM] = Tk;
         unit_sync<NW>();
 
         // ---------------- lines
@@ -363,6 +385,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         T gR[3];           // grad rho
         {
             T Ut[3] = {0, 0, 0}, Qt[3] = {0, 0, 0};
+            // RHOU: divQ holds sum z rho(m) = div q + u.grad rho
             T divU = 0, divQ = 0, dr[3], dp[3];
             // Sums start with the own node's share.  FP32 sums the differences to the
             // own node's values (whose share is then the row sum rs of D, zero but for
@@ -383,12 +406,12 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
                     Ut[k] = He[0][k] * v[0] + He[1][k] * v[1] + He[2][k] * v[2];
-                    Qt[k] = He[0][k] * q[0] + He[1][k] * q[1] + He[2][k] * q[2];
+                    if constexpr (!RHOU) Qt[k] = He[0][k] * q[0] + He[1][k] * q[1] + He[2][k] * q[2];
                     a0 += rs[k] * Ut[k];
                     b0 += rs[k] * Qt[k];
                 }
                 divU = a0;
-                divQ = b0;
+                divQ = RHOU ? T(2) * rho * a0 : b0;
             }
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -414,7 +437,18 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                         x2r -= V2{v[2], rho};
                     }
                     dr[k] += c * x2r.y;
-                    if constexpr (CONV) {
+                    if constexpr (CONV && RHOU) {
+                        const V2 xpH = ld2(b + 4);
+                        const T ut = He[0][k] * x01.x + He[1][k] * x01.y + He[2][k] * x2r.x;
+                        const T z = c * (Ut[k] + ut), K = z * (rho + x2r.y);
+                        dvu += c * ut;
+                        dvq += z * x2r.y;
+                        rq[0] += K * x01.x;
+                        rq[1] += K * x01.y;
+                        rq[2] += K * x2r.x;
+                        re += K * xpH.y;
+                        dp[k] += c * xpH.x;
+                    } else if constexpr (CONV) {
                         V2 xpH = ld2(b + 4), xHq = ld2(b + 6), xqq = ld2(b + 8);
                         if constexpr (DELTA) {
                             xpH -= V2{p, H};
@@ -440,7 +474,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                         du[0][k] += c * x01.x;
                         du[1][k] += c * x01.y;
                         du[2][k] += c * x2r.x;
-                        dT[k] += c * (DELTA ? area[b + 10] - Tk : area[b + 10]);
+                        dT[k] += c * (DELTA ? area[b + TEM] - Tk : area[b + TEM]);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -456,7 +490,16 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
                     gR[i] = He[i][0] * dr[0] + He[i][1] * dr[1] + He[i][2] * dr[2];
-            if constexpr (CONV) {
+            if constexpr (CONV && RHOU) {
+                // the own values' coefficient: s + rho div u and the own share of sum K
+                const T s = divQ, B = s + rho * (divU + T(4) * a0);
+                Rm = vol * (T(0.5) * (s + rho * divU));
+                Re = vol * (T(0.25) * (Re + H * B));
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    Rq[i] = vol * (T(0.25) * (Rq[i] + v[i] * B) +
+                                   (He[i][0] * dp[0] + He[i][1] * dp[1] + He[i][2] * dp[2]));
+            } else if constexpr (CONV) {
                 const T urho = Ut[0] * dr[0] + Ut[1] * dr[1] + Ut[2] * dr[2];
                 const T s = divQ + urho;
                 // the own values' coefficients: div q + u.grad rho for u_i and H,
@@ -543,7 +586,8 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         }
         // ---------------- out
         unit_sync<NW>(); // every wave is done with the records in `area`
-        T *o = area + 5 * ln.rec;
+        T *o = area + RW * ln.rec;
+        if constexpr (RW == 6) o[5] = T(0);
         o[0] = Rm;
         o[1] = Rq[0];
         o[2] = Rq[1];
@@ -1764,29 +1808,35 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
 #undef GL2
 }
 
+// Launches the operators' element kernel.  bpc: the stage's blocks-per-CU setting
+// (16: the kernel's own launch shape; others scale the units a block takes).
+template <int P, typename T, bool CONV, bool VISC, bool CONS>
+static void launch_rhs_p(sodhip_ctx ctx, RhsArgs<T> A, int bpc)
+{
+    const UnitShape us = unit_shape<P, T>(ctx, A.nelem, bpc);
+    A.run = us.run;
+    A.wide = us.wide;
+    k_rhs<P, T, CONV, VISC, CONS><<<us.grid, EP<P, T>::NTB, 0, ctx->stream>>>(A);
+}
+
 template <typename T>
 static int launch_rhs(sodhip_ctx ctx, int porder, bool conv, bool diff, bool cons,
-                      const RhsArgs<T> &A0)
+                      const RhsArgs<T> &A0, int bpc = 16, int geo16 = 1)
 {
     RhsArgs<T> A = A0;
     // 16-byte geometry copies start from 16-byte boundaries of the arrays
-    A.geo16 = ((uintptr_t)A.He % 16 == 0) && ((uintptr_t)A.gpvol % 16 == 0);
+    A.geo16 = geo16 && ((uintptr_t)A.He % 16 == 0) && ((uintptr_t)A.gpvol % 16 == 0);
 #define SODHIP_RHS_CASE(PP)                                                                \
-    case PP: {                                                                             \
-        const UnitShape us = unit_shape<PP, T>(ctx, A.nelem);                              \
-        const int nt = EP<PP, T>::NTB;                                                     \
-        A.run = us.run;                                                                    \
-        A.wide = us.wide;                                                                  \
+    case PP:                                                                               \
         if (conv && diff && cons)                                                          \
-            k_rhs<PP, T, true, true, true><<<us.grid, nt, 0, ctx->stream>>>(A);            \
+            launch_rhs_p<PP, T, true, true, true>(ctx, A, bpc);                            \
         else if (conv && !diff && !cons)                                                   \
-            k_rhs<PP, T, true, false, false><<<us.grid, nt, 0, ctx->stream>>>(A);          \
+            launch_rhs_p<PP, T, true, false, false>(ctx, A, bpc);                          \
         else if (!conv && diff && !cons)                                                   \
-            k_rhs<PP, T, false, true, false><<<us.grid, nt, 0, ctx->stream>>>(A);          \
+            launch_rhs_p<PP, T, false, true, false>(ctx, A, bpc);                          \
         else                                                                               \
             return set_error(SODHIP_ERR_UNSUPPORTED, "unsupported operator combination");  \
-        break;                                                                             \
-    }
+        break;
     switch (porder) {
         SODHIP_RHS_CASE(2)
         SODHIP_RHS_CASE(3)
@@ -1800,10 +1850,9 @@ static int launch_rhs(sodhip_ctx ctx, int porder, bool conv, bool diff, bool con
 }
 
 template <typename TS, typename TR>
-static int launch_gather(sodhip_ctx ctx, const MeshCache *m, const TS *scr, size_t EN, int nf,
+static int launch_gather(sodhip_ctx ctx, const MeshCache *m, const TS *scr, int nf,
                          TR *R0, TR *R1, TR *R2, TR *R3, TR *R4, int init, TR fact)
 {
-    (void)EN;
     const int bs = 256;
     const int grid = ((m->npoin + bs - 1) / bs + 7) / 8 * 8;
 #define SODHIP_GATHER(NFV)                                                                     \
@@ -1908,7 +1957,7 @@ static int full_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const i
     prof_end(ctx, tok);
     if (rc) return rc;
     tok = prof_begin(ctx, 1);
-    rc = launch_gather<T, T>(ctx, m, A.out, EN, 5, Rmass, Rmom, Rmom + npoin,
+    rc = launch_gather<T, T>(ctx, m, A.out, 5, Rmass, Rmom, Rmom + npoin,
                              Rmom + 2 * (size_t)npoin, Rener, initialize, fact);
     prof_end(ctx, tok);
     return rc;
@@ -1962,7 +2011,7 @@ static int full_diffusion(sodhip_ctx ctx, int porder, int nelem, int npoin, cons
     prof_end(ctx, tok);
     if (rc) return rc;
     tok = prof_begin(ctx, 1);
-    rc = launch_gather<T, T>(ctx, m, A.out, EN, 5, Rmass, Rmom, Rmom + npoin,
+    rc = launch_gather<T, T>(ctx, m, A.out, 5, Rmass, Rmom, Rmom + npoin,
                              Rmom + 2 * (size_t)npoin, Rener, initialize, fact);
     prof_end(ctx, tok);
     return rc;
@@ -1973,12 +2022,7 @@ static int full_diffusion(sodhip_ctx ctx, int porder, int nelem, int npoin, cons
 // values per record of rhs_fused_elements' output (operator precision 8 or 4)
 int fused_record_width(int porder, int op_bytes)
 {
-#if SODHIP_SPLIT_RHS
-    if (porder == 3) return op_bytes == 4 ? split_rw<float>() : split_rw<double>();
-#endif
-    (void)porder;
-    (void)op_bytes;
-    return 5;
+    return op_bytes == 4 && porder == 3 ? stage_rw<3, float>() : 5;
 }
 
 template <typename T>
@@ -2017,31 +2061,8 @@ int rhs_fused_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *
     A.c_ener = T(c_ener);
     A.out = out;
     int tok = prof_begin(ctx, 0);
-    int rc = SODHIP_OK;
-#if SODHIP_SPLIT_RHS
-    // p=3: one wave per operator (in FP64 a single wave holding both spills;
-    // in FP32 the split is also faster); at p=2 a single wave holds both
-    // operators with fewer spills, p=4 needs two waves per operator
-    bool done = false;
-    {
-        if (porder == 3) {
-            const size_t nn = (size_t)nnode_of(porder);
-            A.geo16 = ctx->stage_geo16 && ((uintptr_t)A.He % 16 == 0) &&
-                      ((uintptr_t)A.gpvol % 16 == 0) && (9 * nn * sizeof(T)) % 16 == 0 &&
-                      (nn * sizeof(T)) % 16 == 0;
-            const int grid = elem_grid(ctx, m->nelem, ctx->stage_bpc);
-            if (A.geo16)
-                k_rhs_split<3, T, true><<<grid, 128, 0, ctx->stream>>>(A);
-            else
-                k_rhs_split<3, T, false><<<grid, 128, 0, ctx->stream>>>(A);
-            if (hipGetLastError() != hipSuccess)
-                rc = set_error(SODHIP_ERR_HIP, "k_rhs_split launch failed");
-            done = true;
-        }
-    }
-    if (!done)
-#endif
-        rc = launch_rhs<T>(ctx, porder, true, true, true, A);
+    const int rc = launch_rhs<T>(ctx, porder, true, true, true, A, ctx->stage_bpc,
+                                 ctx->stage_geo16);
     prof_end(ctx, tok);
     return rc;
 }
@@ -2266,7 +2287,7 @@ static int scalar_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const
         }
         return set_error(SODHIP_ERR_UNSUPPORTED, "entropy residual in FP64 only");
     }
-    return launch_gather<T, T>(ctx, m, A.out, EN, 1, Rconvec, nullptr, nullptr, nullptr, nullptr,
+    return launch_gather<T, T>(ctx, m, A.out, 1, Rconvec, nullptr, nullptr, nullptr, nullptr,
                                initialize, fact);
 }
 
@@ -2323,12 +2344,12 @@ static int div_curl(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
     SODHIP_TRY_HIP(hipGetLastError());
     T *c0 = curlU, *c1 = curlU ? curlU + npoin : nullptr, *c2 = curlU ? curlU + 2 * (size_t)npoin : nullptr;
     if (divU && curlU)
-        rc = launch_gather<T, T>(ctx, m, A.out, EN, 4, divU, c0, c1, c2, nullptr, 1, T(1));
+        rc = launch_gather<T, T>(ctx, m, A.out, 4, divU, c0, c1, c2, nullptr, 1, T(1));
     else if (divU)
-        rc = launch_gather<T, T>(ctx, m, A.out, EN, 1, divU, nullptr, nullptr, nullptr, nullptr, 1,
+        rc = launch_gather<T, T>(ctx, m, A.out, 1, divU, nullptr, nullptr, nullptr, nullptr, 1,
                                  T(1));
     else
-        rc = launch_gather<T, T>(ctx, m, A.out, EN, 3, c0, c1, c2, nullptr, nullptr, 1, T(1));
+        rc = launch_gather<T, T>(ctx, m, A.out, 3, c0, c1, c2, nullptr, nullptr, 1, T(1));
     if (rc == SODHIP_OK && curlU && lelpn) {
         k_per_elem_count<T><<<(npoin_w + 255) / 256, 256, 0, ctx->stream>>>(npoin, npoin_w, lpoin_w,
                                                                            lelpn, curlU);

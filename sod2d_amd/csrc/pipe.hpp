@@ -19,6 +19,8 @@
 // would run past the end of the arrays.
 #pragma once
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "device.hpp"
 #include "element.hpp"
@@ -108,15 +110,16 @@ __device__ __forceinline__ UnitRange unit_range(int nunits, int run, int wide)
 // The launch over nelem elements.  A tile is as wide as the XCD has CUs (four
 // times that for blocks of one wave), and a block takes up to 16 groups of
 // units, fewer where that would leave the chip with less than two rounds of
-// blocks.  At 553k elements, p=3, FP64 the convection takes 1.25 ms with 16 groups
-// in tiles of 32 blocks, 1.29 ms with tiles of 128 and 1.26 ms with 8 groups;
-// at 63k elements, p=4, 336, 349 and 347 us.  (One grid-stride walk over 128
-// blocks per CU, which amortises a block's tables over fewer units and drifts
-// apart, took 1.46 ms and 429 us.)
+// blocks; bpc, the stage's blocks-per-CU setting, scales it (16: as is).  At 553k
+// elements, p=3, FP64 the convection takes 1.25 ms with 16 groups in tiles of 32
+// blocks, 1.29 ms with tiles of 128 and 1.26 ms with 8 groups; at 63k elements,
+// p=4, 336, 349 and 347 us.  (One grid-stride walk over 128 blocks per CU, which
+// amortises a block's tables over fewer units and drifts apart, took 1.46 ms and
+// 429 us.)
 struct UnitShape {
     int run, wide, grid;
 };
-template <int P, typename T> inline UnitShape unit_shape(sodhip_ctx ctx, int nelem)
+template <int P, typename T> inline UnitShape unit_shape(sodhip_ctx ctx, int nelem, int bpc = 16)
 {
     using Q = EP<P, T>;
     const int nunits = (nelem + Q::NE - 1) / Q::NE, ngroups = (nunits + Q::G - 1) / Q::G;
@@ -125,6 +128,7 @@ template <int P, typename T> inline UnitShape unit_shape(sodhip_ctx ctx, int nel
     UnitShape s;
     s.run = chunk / (2 * round);
     s.run = s.run < 1 ? 1 : (s.run > 16 ? 16 : s.run);
+    if (bpc != 16) s.run = std::min(std::max(s.run * 16 / bpc, 1), 64);
     s.wide = cus * (4 / waves);
     const int tile = s.run * s.wide;
     s.grid = 8 * ((chunk + tile - 1) / tile * s.wide);
