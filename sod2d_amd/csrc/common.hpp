@@ -205,16 +205,23 @@ int gather_update_on(sodhip_ctx ctx, int npoin, int nw, const int *list, const i
                      double dt, double lam1, double lams, double gam, const double *rho1,
                      const double *q1, const double *E1, double *rho, double *q, double *E,
                      double *Rmass, double *Rmom, double *Rener, const NextStage *next);
-// convection and the LPS-stabilised viscous operator (full_diff_stab_ijk) of
-// the fused LPS stage at p=3, FP64, from the conserved state, with the node
-// projection records prj (kProjRec per node) and comp_tau's tau; records of
-// five per element-node into out (ops_element.hip)
-int rhs_lps_elements(sodhip_ctx ctx, const MeshCache *m, const double *He, const double *gpvol,
-                     const double *dl, const int *inv, const int *gI, const int *gJ, const int *gK,
-                     const double *rho, const double *q, const double *E, const double *mu_e,
-                     const double *prj, const double *tau, double gamma, double Rgas, double Cp,
-                     double Pr, double mu_factor, double c_rho, double c_ener, double c_lps,
-                     double *out);
+// inputs of the LPS operators' element kernels (device pointers, reference
+// layouts); out receives the records: 5 values per element-node (12 for the
+// projections) at e*nnode + perm[a]
+struct LpsArgs {
+    const double *He, *gpvol, *dl;
+    const int *inv;
+    const double *rho_n, *rho, *u, *Tem, *mu_fluid, *mu_e, *mu_sgs; // primitive inputs
+    const double *cr, *cq, *cE;                    // conserved inputs (the fused stage)
+    const double *pMass, *pEner, *pMX, *pMY, *pMZ; // projections (npoin,3) (drop-in)
+    const double *prj;                             // or kProjRec values per node (stage)
+    const double *tau;                             // tau_stab(nelem)
+    double gamma, Rgas, mu_factor, Cp, Pr, c_rho, c_ener, c_lps;
+    double *out;
+};
+enum class LpsKernel { stage, stab, proj };
+// launches one of them over mesh m (ops_element.hip)
+int lps_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const LpsArgs &L, LpsKernel what);
 // the fused p=3 FP64 stage's element kernel in cluster mode: interior nodes
 // updated in place, surface partial records into rec (ops_element.hip)
 int rhs_cluster_stage(sodhip_ctx ctx, const MeshCache *m, const ClusterTables *cl,
@@ -234,9 +241,4 @@ int gather_update(sodhip_ctx ctx, const MeshCache *m, int npoin, int npoin_w,
                   double fact, double dt, double lam1, double lams, double gam,
                   const double *rho1, const double *q1, const double *E1, double *rho, double *q,
                   double *E, double *Rmass, double *Rmom, double *Rener, const NextStage *next);
-// full_convec_ijk element records (ops_element.hip)
-template <typename T>
-int conv_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *He, const T *gpvol,
-                  const T *dl, const int *inv, const int *gI, const int *gJ, const int *gK,
-                  const T *u, const T *q, const T *rho, const T *pr, const T *E, T *out);
 } // namespace sodhip

@@ -28,30 +28,6 @@
 #include "element.hpp"
 #include "pipe.hpp"
 
-#ifndef SODHIP_SPLIT_WAVES
-#define SODHIP_SPLIT_WAVES 2
-#endif
-#ifndef SODHIP_SPLIT_RHS
-#define SODHIP_SPLIT_RHS 1
-#endif
-#ifndef SODHIP_SPLIT_WAVES_F32
-#define SODHIP_SPLIT_WAVES_F32 2
-#endif
-// ring depth (elements in flight per block) in FP64 and FP32 operators: in
-// FP64 two keep four blocks per CU within 160 KB of LDS
-// consecutive elements a block evaluates in a row (runs of one block, XCD-
-// aware over runs): they share the 128-byte lines and pages of the element-
-// fastest mu_e(nelem,ngaus)
-#ifndef SODHIP_SPLIT_RUN
-#define SODHIP_SPLIT_RUN 4
-#endif
-#ifndef SODHIP_SPLIT_AHEAD64
-#define SODHIP_SPLIT_AHEAD64 2
-#endif
-#ifndef SODHIP_SPLIT_AHEAD32
-#define SODHIP_SPLIT_AHEAD32 3
-#endif
-
 namespace sodhip {
 
 template <typename T> struct RhsArgs {
@@ -94,6 +70,7 @@ template <typename T> struct RhsArgs {
     // projection records (kProjRec values), comp_tau's tau_stab, c_lps
     const double *prj, *tau;
     double c_lps;
+    const double *pMass, *pEner, *pMX, *pMY, *pMZ; // or arrays (npoin,3) (drop-in)
 };
 
 // Sutherland's law (mod_fluid_viscosity.f90:21-41)
@@ -103,8 +80,11 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
 }
 
 // The operators of one right-hand side on the element pipeline (pipe.hpp).
-// CONV: split-form convection (full_convec_ijk); VISC: viscous operator
-// (full_diffusion_ijk); CONS: inputs are the conserved FP64 state (the fused
+// CONV: split-form convection (full_convec_ijk).  VISC: 1 the viscous operator
+// (full_diffusion_ijk); 2 its LPS-stabilised form (full_diff_stab_ijk,
+// elem_stab.f90:207-438); 3 full_proj_ijk's element part (elem_stab.f90:489-563),
+// records of 12 values: gpvol times the upper triangle t11 t12 t13 t22 t23 t33 of
+// 2 S - 2/3 div u I, grad rho and grad T.  CONS: inputs are the conserved FP64 state (the fused
 // stage forms the primitives of updateF's EOS block and Sutherland's viscosity
 // in-kernel) instead of the primitive arrays.
 //
@@ -149,14 +129,26 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
 //   operators, 87k elements 0.21 -> 0.17 ms against two waves per element, one per
 //   operator, that hand over through LDS.  At p=3 FP64 the vector ALU is busy 42 %
 //   and LDS 38 % of the time with two waves per SIMD.
-template <int P, typename T, bool CONV, bool VISC> struct ElemLDS {
+//   LPS: p=4, 41k elements, convection and stabilised operator 0.77 (two kernels, the
+//   second adding to the first one's records) -> 0.40 ms, projections 0.36 -> 0.20 ms;
+//   p=3, 111k elements, 0.55 (two waves per element) -> 0.34 ms and 0.41 -> 0.27 ms;
+//   drop-in stabilised operator p=4, 28k elements 0.38 -> 0.24 ms (these read He with
+//   72-byte strides per lane).
+template <int P, typename T, bool CONV, int VISC, bool CONS> struct ElemLDS {
     using Q = EP<P, T>;
     // nodal records (values), flux records and residual records share one area
     // of one stride, so that a line neighbour has one LDS offset
-    static constexpr int REC = VISC ? 18 : 10, AREA = REC * Q::NT;
+    static constexpr int REC = VISC == 3 ? 12 : VISC ? 18 : 10, AREA = REC * Q::NT;
     // at p=4 the transposed coefficients of both operators' kernel do not fit in
     // the registers beside the rest: they stay in LDS, one column per lane
     static constexpr bool TLDS = CONV && VISC && P == 4;
+    // the fused LPS stage reads each node's projections as one 96-byte record
+    // (kProjRec); they come through LDS in 16-byte pieces, consecutive lanes on
+    // consecutive pieces, into the geometry's buffer once He is in registers (the
+    // next geometry then follows them)
+    static constexpr bool PJ = VISC == 2 && CONS;
+    static constexpr int PROWS = (6 * Q::NL + 63) / 64, PI = (PROWS + Q::NW - 1) / Q::NW;
+    static constexpr int GEO = PJ && PI * Q::NW * 1024 > Q::GEO ? PI * Q::NW * 1024 : Q::GEO;
 };
 
 // Values per residual record of the fused stage's element kernel.  With FP32
@@ -170,33 +162,36 @@ template <int P, typename T> constexpr int stage_rw() { return sizeof(T) == 4 &&
 
 // waves per SIMD asked of the compiler: the FP64 kernels hold He, the three
 // derivative rows and the unit's state in registers
-template <int P, typename T, bool CONV, bool VISC> constexpr int elem_waves()
+template <int P, typename T, bool CONV, int VISC> constexpr int elem_waves()
 {
-    return sizeof(T) == 4 ? 3 : 2;
+    return sizeof(T) == 4 || (VISC == 3 && !CONV) ? 3 : 2;
 }
 
-template <int P, typename T, bool CONV, bool VISC, bool CONS>
+template <int P, typename T, bool CONV, int VISC, bool CONS>
 __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) void k_rhs(RhsArgs<T> A)
 {
     using Q = EP<P, T>;
-    using L = ElemLDS<P, T, CONV, VISC>;
+    using L = ElemLDS<P, T, CONV, VISC, CONS>;
+    constexpr bool FLUX = VISC == 1 || VISC == 2, LPS = VISC == 2, PROJ = VISC == 3;
+    static_assert(!(LPS || PROJ) || sizeof(T) == 8, "LPS: FP64");
+    constexpr int GEO = L::GEO;
     using V2 = T __attribute__((ext_vector_type(2)));
     constexpr int NN = Q::NN, NL = Q::NL, NT = Q::NT, NE = Q::NE, NW = Q::NW, G = Q::G;
-    constexpr int REC = L::REC, RW = CONS ? stage_rw<P, T>() : 5;
+    constexpr int REC = L::REC, RW = PROJ ? 12 : CONS ? stage_rw<P, T>() : 5;
     // q = rho u and rho H formed from the other values, in FP64 only: in FP32 the
     // separately rounded q and u average their rounding errors (q of a 0.2-Mach flow
     // is 20 to 45 % less exact without)
     constexpr bool RHOU = CONS && sizeof(T) == 8;
     constexpr int TEM = 10; // temperature's place in the nodal record
     __shared__ __attribute__((aligned(16))) T area_s[G * L::AREA];
-    __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * Q::GEO];
+    __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * GEO];
     __shared__ int conn_s[G * 2 * NT];
     // this thread's unit of the group, and its LDS
     const int sb = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
     T *const area = area_s + sb * L::AREA;
-    unsigned char *const geo = geo_s + sb * Q::GEO;
+    unsigned char *const geo = geo_s + sb * GEO;
     int *const conn = conn_s + sb * 2 * NT;
-    const unsigned geo_at = lds_addr(geo_s) + sb * Q::GEO;
+    const unsigned geo_at = lds_addr(geo_s) + sb * GEO;
     const unsigned conn_at = lds_addr(conn_s) + sb * 2 * NT * 4;
     const int lane = threadIdx.x % NT, wl = lane & 63;
     const int wv = __builtin_amdgcn_readfirstlane(lane >> 6);
@@ -208,7 +203,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     auto unit = [&](int g) { return min(g * G + sb, nunits - 1); };
     if (er.begin >= er.end) return;
     const int ulast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
-    const LexLane<P, T, VISC> ln(lane, A.dl, A.inv, A.perm);
+    const LexLane<P, T, FLUX> ln(lane, A.dl, A.inv, A.perm);
     const size_t EN = (size_t)A.nelem * NN, np = (size_t)A.npoin;
     auto conn_issue = [&](int u, int slot) {
         const size_t i = (size_t)u * NL + lane;
@@ -224,6 +219,15 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     for (int k = 0; k < 3; ++k)
 #pragma unroll
         for (int o = 0; o < P; ++o) nb[k][o] = ln.nb[k][o] * REC;
+    // the fused LPS stage: this lane's pieces of the unit's projection records, by the
+    // place of their node in the unit's row of node ids
+    __shared__ int pj_node[L::PJ ? L::PI * NT : 1];
+    if constexpr (L::PJ)
+        if (sb == 0)
+            for (int i = 0; i < L::PI; ++i) {
+                const int l = min(((wv + NW * i) * 64 + wl) / 6, NL - 1);
+                pj_node[i * NT + lane] = l / NN * NN + min(max(A.inv[l % NN] - 1, 0), NN - 1);
+            }
     auto ld2 = [&](int i) { return *(const V2 *)(area + i); };
     auto st2 = [&](int i, T x, T y) { *(V2 *)(area + i) = V2{x, y}; };
 
@@ -232,6 +236,8 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         double cr, cq[3], cE;                     // conserved state (CONS)
         T rho, u[3], q[3], pr, E, Tem, rhon, muf; // primitive inputs (drop-in)
         T mue, musgs;
+        double tau; // LPS
+        int n;
     };
     auto load = [&](In &x, int u, int slot) {
         const int n = conn[slot * NT + ln.sub * NN + ln.a];
@@ -251,13 +257,15 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 x.pr = A.pr[n];
                 x.E = A.E[n];
             }
-            if constexpr (VISC) {
-                x.Tem = A.Tem[n];
+            if constexpr (VISC != 0) x.Tem = A.Tem[n];
+            if constexpr (FLUX) {
                 x.rhon = A.rho_n[n];
                 x.muf = A.mu_fluid[n];
             }
+            if constexpr (LPS) x.n = n;
         }
-        if constexpr (VISC) {
+        if constexpr (LPS) x.tau = A.tau[min(u * NE + ln.sub, A.nelem - 1)];
+        if constexpr (FLUX) {
             const size_t eg = (size_t)min(u * NE + ln.sub, A.nelem - 1) + (size_t)A.nelem * ln.a;
             x.mue = A.mu_e[eg];
             if constexpr (!CONS) x.musgs = A.mu_sgs ? A.mu_sgs[eg] : T(0);
@@ -314,13 +322,35 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         lds_done();
         if (prev >= 0) rec_store(out, prev);
         load(nxt, u2, slot);
+        int pn[L::PJ ? L::PI : 1];
+        if constexpr (L::PJ) {
+#pragma unroll
+            for (int i = 0; i < L::PI; ++i) pn[i] = conn[(slot ^ 1) * NT + pj_node[i * NT + lane]];
+        }
         unit_sync<NW>();
-        at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
-        conn_issue(u3, slot ^ 1);
+        if constexpr (L::PJ) {
+#pragma unroll
+            for (int i = 0; i < L::PI; ++i) {
+                const int r = wv + NW * i;
+                dma_lds<16>(A.prj + kProjRec * (size_t)pn[i] + 2 * ((r * 64 + wl) % 6), geo_at + r * 1024);
+            }
+        } else {
+            at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
+            conn_issue(u3, slot ^ 1);
+        }
+        // the drop-in LPS operator's projections, for the fluxes
+        double pj[LPS ? 15 : 1]; // rows of the projected tensor, grad rho, grad T
+        if constexpr (LPS && !CONS) {
+            const double *pf[5] = {A.pMX, A.pMY, A.pMZ, A.pMass, A.pEner};
+#pragma unroll
+            for (int f = 0; f < 5; ++f)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) pj[3 * f + d] = pf[f][cur.n + np * d];
+        }
         prev = g * G + sb < nunits ? u : -1;
         // ---------------- stage
         T rho, v[3], q[3] = {0, 0, 0}, H = 0, rhoH = 0, p = 0, Tk = 0, muf = 0, rhon = 0, musgs = 0;
-        const T mue = VISC ? cur.mue : T(0);
+        const T mue = FLUX ? cur.mue : T(0);
         if constexpr (CONS) {
             const double r = cur.cr, ri = 1.0 / r;
             double ud[3], umag = 0.0;
@@ -359,8 +389,8 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 H = cur.E + (v[0] * v[0] * T(0.5) + v[1] * v[1] * T(0.5) + v[2] * v[2] * T(0.5));
                 rhoH = rho * H;
             }
-            if constexpr (VISC) {
-                Tk = cur.Tem;
+            if constexpr (VISC != 0) Tk = cur.Tem;
+            if constexpr (FLUX) {
                 rhon = cur.rhon;
                 muf = cur.muf;
                 musgs = cur.musgs;
@@ -376,7 +406,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             st2(own + 6, rhoH, q[0]);
             st2(own + 8, q[1], q[2]);
         }
-        if constexpr (VISC) area[own + TEM] = Tk;
+        if constexpr (VISC != 0) area[own + TEM] = Tk;
         unit_sync<NW>();
 
         // ---------------- lines
@@ -422,7 +452,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 const T eb = DELTA ? Qt[k] + rho * Ut[k] : Qt[k], cb = DELTA ? T(2) * Ut[k] : Ut[k];
                 dr[k] = rs[k] * rho;
                 if constexpr (CONV) dp[k] = rs[k] * p;
-                if constexpr (VISC) {
+                if constexpr (VISC != 0) {
                     dT[k] = rs[k] * Tk;
 #pragma unroll
                     for (int i = 0; i < 3; ++i) du[i][k] = rs[k] * v[i];
@@ -470,7 +500,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                         rq[2] += C * xqq.y;
                         dp[k] += c * xpH.x;
                     }
-                    if constexpr (VISC) {
+                    if constexpr (VISC != 0) {
                         du[0][k] += c * x01.x;
                         du[1][k] += c * x01.y;
                         du[2][k] += c * x2r.x;
@@ -486,7 +516,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                     divQ += dvq;
                 }
             }
-            if constexpr (VISC)
+            if constexpr (VISC != 0)
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
                     gR[i] = He[i][0] * dr[0] + He[i][1] * dr[1] + He[i][2] * dr[2];
@@ -516,30 +546,109 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             }
         }
 
-        if constexpr (VISC) {
-            // ---------------- fluxes.  Record per k: grad rho, grad T | tau u, tau_1 |
-            // tau_2, tau_3 (contravariant, times gpvol)
-            T W[6] = {0, 0, 0, 0, 0, 0};
-            {
-                T tau[3][3], gt[3];
-                const T mufg = muf + rhon * musgs, mut = mufg + mue;
-                T gU[3][3];
+        if constexpr (CONV && LPS) {
+            // formed here, not where they are used: sunk past the copies' branches
+            // below they would keep the convection's inputs alive
+            pin(Rm);
+            pin(Re);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) pin(Rq[i]);
+        }
+        double po[PROJ ? 12 : 1];
+        if constexpr (VISC != 0) {
+            // physical gradients: gU[i][j] = d u_i / d x_j, and grad T
+            T gU[3][3], gt[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    gU[i][j] = He[j][0] * du[i][0] + He[j][1] * du[i][1] + He[j][2] * du[i][2];
+                gt[i] = He[i][0] * dT[0] + He[i][1] * dT[1] + He[i][2] * dT[2];
+            }
+            const T dv = gU[0][0] + gU[1][1] + gU[2][2];
+            if constexpr (PROJ) {
+                int f = 0;
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
-                    for (int j = 0; j < 3; ++j)
-                        gU[i][j] = He[j][0] * du[i][0] + He[j][1] * du[i][1] + He[j][2] * du[i][2];
-                const T tt = mufg * T(2.0 / 3.0) * (gU[0][0] + gU[1][1] + gU[2][2]);
+                    for (int d = i; d < 3; ++d)
+                        po[f++] = vol * (gU[i][d] + gU[d][i] - (i == d ? (2.0 / 3.0) * dv : 0.0));
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    po[6 + d] = vol * gR[d];
+                    po[9 + d] = vol * gt[d];
+                }
+            }
+            if constexpr (FLUX) {
+            // ---------------- fluxes.  Record per k: grad rho, grad T | tau u, tau_1 |
+            // tau_2, tau_3 (contravariant, times gpvol)
+            T W[6] = {0, 0, 0, 0, 0, 0};
+            const T mufg = muf + rhon * musgs, mut = mufg + mue;
+            const T kappa = muf * A.Cp / A.Pr + A.c_ener * mue * A.Cp / A.Pr +
+                            A.Cp * rhon * musgs / T(0.9);
+            if constexpr (L::PJ) wait_vm<0>(); // the projections
+            if constexpr (NW > 1) lds_barrier(); // every wave has read the nodal records
+            if constexpr (LPS) {
+                // per point (nu_e and kappa_e inside): the stabilising terms -c_lps tau
+                // (Proj - grad), times rho for momentum and rho Cp/Pr for energy.
+                // Record per k: mass, energy | momentum 1, 2 | 3
+                const T cl = -A.c_lps * cur.tau, clr = cl * rhon, tt = T(2.0 / 3.0) * dv;
+                const T nu_e = A.c_rho * mue / rhon, cle = clr * A.Cp / A.Pr;
+                // projection j of the node (rows of the tensor from its upper triangle)
+                auto prj = [&](int j) -> T {
+                    if constexpr (L::PJ) {
+                        const int tri[15] = {0, 1, 2, 1, 3, 4, 2, 4, 5, 6, 7, 8, 9, 10, 11};
+                        return ((const T *)(geo + 96 * lane))[tri[j]];
+                    } else {
+                        return pj[j];
+                    }
+                };
+                T h[3][3], tu[3] = {0, 0, 0};
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) h[k][d] = vol * He[d][k];
+                // flux f (its three components F) to the records and its own share of W;
+                // one flux at a time, to keep few values alive
+                auto flux = [&](int f, int at, const T F[3]) {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const T X = h[k][0] * F[0] + h[k][1] * F[1] + h[k][2] * F[2];
+                        W[f] += ln.ds[k] * X;
+                        area[own + 6 * k + at] = X;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    T F[3];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const T S = gU[i][d] + gU[d][i], St = i == d ? S - tt : S;
+                        const T ts = i == d ? mut * S - mufg * tt : mut * S;
+                        F[d] = clr * (prj(3 * i + d) - St) + ts;
+                        tu[d] += ts * v[i];
+                    }
+                    flux(1 + i, 2 + i, F);
+                }
+                {
+                    T F[3];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) F[d] = cl * (prj(9 + d) - gR[d]) + nu_e * gR[d];
+                    flux(0, 0, F);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) F[d] = cle * (prj(12 + d) - gt[d]) + kappa * gt[d] + tu[d];
+                    flux(4, 1, F);
+                }
+            } else {
+                const T tt = mufg * T(2.0 / 3.0) * dv;
+                T tau[3][3];
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
                     for (int j = 0; j < 3; ++j) tau[i][j] = mut * (gU[i][j] + gU[j][i]);
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    tau[i][i] -= tt;
-                    gt[i] = He[i][0] * dT[0] + He[i][1] * dT[1] + He[i][2] * dT[2];
-                }
-                if constexpr (NW > 1) lds_barrier(); // every wave has read the nodal records
+                for (int i = 0; i < 3; ++i) tau[i][i] -= tt;
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
                     const T h0 = vol * He[0][k], h1 = vol * He[1][k], h2 = vol * He[2][k];
@@ -560,6 +669,13 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 }
             }
             unit_sync<NW>();
+            if constexpr (L::PJ) {
+#pragma unroll
+                for (int f = 0; f < 5; ++f) pin(W[f]);
+                lds_done(); // this wave has read its projections; with a barrier, all have
+                at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
+                conn_issue(u3, slot ^ 1);
+            }
             // ---------------- weak divergence
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -568,31 +684,51 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 for (int o = 0; o < P; ++o) {
                     const int b = nb[k][o] + 6 * k;
                     const T c = L::TLDS ? tcol[(k * P + o) * NT + lane] : ln.t[k][o];
-                    const V2 x01 = ld2(b), x23 = ld2(b + 2), x45 = ld2(b + 4);
-                    W[0] += c * x01.x;
-                    W[1] += c * x01.y;
-                    W[2] += c * x23.x;
-                    W[3] += c * x23.y;
-                    W[4] += c * x45.x;
-                    W[5] += c * x45.y;
+                    const V2 x01 = ld2(b), x23 = ld2(b + 2);
+                    if constexpr (LPS) { // W: mass, momentum 1, 2, 3, energy
+                        W[0] += c * x01.x;
+                        W[4] += c * x01.y;
+                        W[1] += c * x23.x;
+                        W[2] += c * x23.y;
+                        W[3] += c * area[b + 4];
+                    } else {
+                        const V2 x45 = ld2(b + 4);
+                        W[0] += c * x01.x;
+                        W[1] += c * x01.y;
+                        W[2] += c * x23.x;
+                        W[3] += c * x23.y;
+                        W[4] += c * x45.x;
+                        W[5] += c * x45.y;
+                    }
                 }
             }
-            Rm += A.c_rho * mue / rhon * W[0];
-            const T kappa = muf * A.Cp / A.Pr + A.c_ener * mue * A.Cp / A.Pr +
-                            A.Cp * rhon * musgs / T(0.9);
-            Re += W[2] + kappa * W[1];
+            if constexpr (LPS) {
+                Rm += W[0];
+                Re += W[4];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) Rq[i] += W[3 + i];
+                for (int i = 0; i < 3; ++i) Rq[i] += W[1 + i];
+            } else {
+                Rm += A.c_rho * mue / rhon * W[0];
+                Re += W[2] + kappa * W[1];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) Rq[i] += W[3 + i];
+            }
+            } // FLUX
         }
         // ---------------- out
         unit_sync<NW>(); // every wave is done with the records in `area`
-        T *o = area + RW * ln.rec;
-        if constexpr (RW == 6) o[5] = T(0);
-        o[0] = Rm;
-        o[1] = Rq[0];
-        o[2] = Rq[1];
-        o[3] = Rq[2];
-        o[4] = Re;
+        if constexpr (PROJ) {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) st2(12 * ln.rec + 2 * i, po[2 * i], po[2 * i + 1]);
+        } else {
+            T *o = area + RW * ln.rec;
+            if constexpr (RW == 6) o[5] = T(0);
+            o[0] = Rm;
+            o[1] = Rq[0];
+            o[2] = Rq[1];
+            o[3] = Rq[2];
+            o[4] = Re;
+        }
         cur = nxt;
     }
     lds_barrier();
@@ -881,7 +1017,8 @@ __global__ __launch_bounds__(256) void k_gather_entropy(int npoin, const int *__
 
 // ---------------------------------------------------------------- launch helpers
 // ---------------------------------------------------------------------------
-// Fused-stage element kernel with the work of each element split over two
+// Element kernel of the brick-local assembly (the opt-in mode of the fused FP64
+// stage at p=3), with the work of each element split over two
 // waves that share its LDS: wave 0 evaluates the split-form convection, wave 1
 // the viscous operator and hands its residuals to wave 0 through LDS; wave 0
 // puts their sum back into the same LDS slots and wave 1 stores it during the
@@ -912,50 +1049,33 @@ __global__ __launch_bounds__(256) void k_gather_entropy(int npoin, const int *__
 //   B3  line derivatives of u and rho handed over: wave 0 forms them for the
 //       convection terms, and wave 1 takes them for grad u and grad rho
 //       instead of forming the same sums again
-// values per residual record written by the two-wave kernel.  With FP32
-// operators the five residuals are padded to six, so that a record starts on
-// an 8-byte boundary and the gather reads it with three 8-byte loads (the
-// gather then takes 0.25 instead of 0.43 ms at 64^3 elements); in FP64 the
-// 20 % larger records cost the element kernel more than the gather gains.
-template <typename T> constexpr int split_rw() { return sizeof(T) == 4 ? 6 : 5; }
-
-template <int P, typename T, bool G16, int RUNV = SODHIP_SPLIT_RUN, bool LPSV = false>
-struct SplitLDS {
+template <int P, typename T, bool G16> struct SplitLDS {
     static constexpr int NN = (P + 1) * (P + 1) * (P + 1);
-    static constexpr int AH = sizeof(T) == 8 ? SODHIP_SPLIT_AHEAD64 : SODHIP_SPLIT_AHEAD32;
+    static constexpr int AH = 2; // ring depth (elements in flight per block)
     // geometry, He then gpvol, copied in 64-lane rows of GW bytes per lane
     static constexpr int HE_BYTES = 9 * NN * (int)sizeof(T), GV_BYTES = NN * (int)sizeof(T);
     static constexpr int GW = G16 ? 16 : 4, GROW = 64 * GW;
     static constexpr int GROWS = (HE_BYTES + GV_BYTES + GROW - 1) / GROW, GEO = GROWS * GROW;
     // conserved fields rho, q1, q2, q3, E (FP64, node-major), then mu_e
     // mu_e(nelem,ngaus) is element-fastest: the 64 values of one element lie
-    // nelem apart.  In FP64 it is copied per run of RUN consecutive elements,
-    // RUN values per node, into one of three blocks, two runs ahead (each
-    // 64-lane row then reads 8 runs of 32 contiguous bytes instead of 32
-    // scattered doubles); with FP32 operators per element into its slot.
-    static constexpr int RUN = RUNV;
-    static constexpr bool MUBLK = sizeof(T) == 8;
-    static constexpr int ST = 5 * NN * 8, MU = MUBLK ? 0 : NN * (int)sizeof(T);
-    // LPS: the projection records of the element's nodes (kProjRec doubles
-    // per node, lexicographic order: 6 rows of 64 16-byte pieces) and its
-    // tau_stab (the first 8 bytes of one 4-byte-per-lane row)
-    static constexpr int PJ_AT = GEO + ST + MU, PJ = LPSV ? NN * kProjRec * 8 : 0;
-    static constexpr int PJ_ROWS = PJ / 1024, TAU_AT = PJ_AT + PJ, TAU = LPSV ? 256 : 0;
-    static_assert(!LPSV || (NN == 64 && PJ == PJ_ROWS * 1024), "LPS records: whole rows");
-    static constexpr int SLOT = GEO + ST + MU + PJ + TAU;
+    // nelem apart.  It is copied per run of RUN = 2 consecutive elements of the
+    // cluster order (they pair up as e, e+1 on a box mesh), RUN values per node,
+    // into one of three blocks, two runs ahead
+    static constexpr int RUN = 2;
+    static constexpr int ST = 5 * NN * 8;
+    static constexpr int SLOT = GEO + ST;
     // connectivity rows: AH + 1 in use at a time
     static constexpr int CROWS = AH + 1, CROW = NN * 4;
-    static constexpr int MUB = RUN * NN * (int)sizeof(T), MUBS = MUBLK ? 3 : 0;
+    static constexpr int MUB = RUN * NN * (int)sizeof(T), MUBS = 3;
     static constexpr int MUB_AT = AH * SLOT + CROWS * CROW;
     static constexpr int BYTES = MUB_AT + MUBS * MUB;
     static constexpr int MU_OPS = (int)sizeof(T) / 4;
-    static_assert(!MUBLK || ((RUN == 4 || RUN == 2) && MUB == 256 * MU_OPS * RUN),
+    static_assert(MUB == 256 * MU_OPS * RUN,
                   "one run's mu_e block in MU_OPS rows per element");
     // copies per element: wave 0 takes the connectivity row, the even
     // geometry rows and rho, q1, q2; wave 1 the odd rows, q3, E and mu_e
-    // (with LPS the viscous wave also copies the projection rows and tau)
     static constexpr int NOPS0 = 1 + (GROWS + 1) / 2 + 6,
-                         NOPS1 = GROWS / 2 + 4 + MU_OPS + (LPSV ? PJ_ROWS + 1 : 0);
+                         NOPS1 = GROWS / 2 + 4 + MU_OPS;
     static_assert(SLOT % 16 == 0, "ring slots must stay 16-byte aligned");
     static_assert(AH >= 2 && AH * NOPS0 <= 63 && AH * NOPS1 <= 63, "vmcnt range");
 };
@@ -977,7 +1097,7 @@ __device__ __forceinline__ void split_issue(const RhsArgs<T> &A, unsigned slot, 
 {
     using L = SplitLDS<P, T, G16>;
     constexpr int NN = L::NN;
-    const int hw = 4 * (lane & 1), nd = lane >> 1;
+    const int hw = 4 * (lane & 1);
     if constexpr (ROLE == 0) dma_lds<4>(A.connecT + (size_t)ec * NN + lane, crow);
     const unsigned char *he = (const unsigned char *)(A.He + (size_t)e * 9 * NN);
     const unsigned char *gv = (const unsigned char *)(A.gpvol + (size_t)e * NN);
@@ -997,36 +1117,9 @@ __device__ __forceinline__ void split_issue(const RhsArgs<T> &A, unsigned slot, 
         dma_lds<4>((const char *)(fld[f] + n0) + hw, st + f * NN * 8);
         dma_lds<4>((const char *)(fld[f] + n1) + hw, st + f * NN * 8 + 256);
     }
-    if constexpr (ROLE == 1 && !L::MUBLK) {
-        const unsigned mu = st + L::ST;
-        if constexpr (sizeof(T) == 8) {
-            dma_lds<4>((const char *)(A.mu_e + e + (size_t)A.nelem * nd) + hw, mu);
-            dma_lds<4>((const char *)(A.mu_e + e + (size_t)A.nelem * (32 + nd)) + hw, mu + 256);
-        } else {
-            dma_lds<4>(A.mu_e + e + (size_t)A.nelem * lane, mu);
-        }
-    }
 }
 
-// FP64 mu_e copies of one iteration: rows 2j and 2j+1 of the block of the run
-// starting at element rfirst (j = iteration within its run).  The block is
-// node-major and element-fastest: lane L moves half L&1 of
-// mu_e(e0 + (L/2)&3, 8i + L/8) of row i.
-template <typename T>
-__device__ __forceinline__ void mu_issue(const RhsArgs<T> &A, unsigned blk, int rfirst, int j,
-                                         int lane)
-{
-    const int hw = 4 * (lane & 1), el = (lane >> 1) & 3, nd8 = lane >> 3;
-    const int e = min(rfirst + el, A.nelem - 1);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int i = 2 * j + h;
-        dma_lds<4>((const char *)(A.mu_e + e + (size_t)A.nelem * (8 * i + nd8)) + hw, blk + i * 256);
-    }
-}
-
-// FP64 mu_e copies of one iteration for runs of two elements (the cluster
-// order, where elements pair up as e, e+1 on a box mesh): rows 2j and 2j+1 of
+// mu_e copies of one iteration: rows 2j and 2j+1 of
 // the block of the run of elements e0, e1 (j = iteration within its run).
 // The block is node-major and element-fastest: lane L moves half L&1 of
 // mu_e(e_{(L/2)&1}, 16i + L/4) of row i.
@@ -1043,28 +1136,9 @@ __device__ __forceinline__ void mu_issue2(const RhsArgs<T> &A, unsigned blk, int
     }
 }
 
-// LPS copies of element e into the ring slot at LDS address slot (viscous
-// wave): row r, lane L moves 16-byte piece (64r+L)%6 of the projection record
-// of the node at lexicographic position (64r+L)/6, whose element-local index
-// ik[r] it holds (c: the element's connectivity row); then tau_stab(e) as two
-// 4-byte halves (lanes 0 and 1; the other lanes repeat them)
-template <typename T, int PJ_ROWS, int PJ_AT, int TAU_AT>
-__device__ __forceinline__ void lps_issue(const RhsArgs<T> &A, unsigned slot, const int *c,
-                                          const int (&ik)[PJ_ROWS], int e, int lane)
-{
-#pragma unroll
-    for (int r = 0; r < PJ_ROWS; ++r) {
-        const int piece = (64 * r + lane) % 6;
-        const int n = c[ik[r]];
-        dma_lds<16>(A.prj + kProjRec * (size_t)n + 2 * piece, slot + PJ_AT + r * 1024);
-    }
-    dma_lds<4>((const char *)(A.tau + e) + 4 * (lane & 1), slot + TAU_AT);
-}
-
-// reads ring slot sl into registers: He, gpvol, the conserved fields and mu_e
-// of node a (lexicographic position pa)
+// reads ring slot sl into registers: He, gpvol and the conserved fields of node a (lexicographic position pa)
 template <int P, typename T, bool G16>
-__device__ __forceinline__ void split_read(const unsigned char *sl, int a, int pa, bool visc,
+__device__ __forceinline__ void split_read(const unsigned char *sl, int a, int pa,
                                            T He[3][3], T &vol, SplitState<P, T> &x)
 {
     using L = SplitLDS<P, T, G16>;
@@ -1081,23 +1155,6 @@ __device__ __forceinline__ void split_read(const unsigned char *sl, int a, int p
     x.cq[1] = st[2 * NN + pa];
     x.cq[2] = st[3 * NN + pa];
     x.cE = st[4 * NN + pa];
-    if constexpr (!L::MUBLK)
-        if (visc) x.mue = ((const T *)(sl + L::GEO + L::ST))[a];
-}
-
-// residual records of element e (split_rw values per node: the five
-// residuals, and a zero when padded; lexicographic node order) from their
-// dense copy in LDS, 16 contiguous bytes per lane
-template <int P, typename T>
-__device__ __forceinline__ void split_store(const RhsArgs<T> &A, const void *dense, int e, int lane)
-{
-    constexpr int RW = split_rw<T>();
-    constexpr int NN = (P + 1) * (P + 1) * (P + 1), CH = RW * NN * (int)sizeof(T) / 16;
-    using U4 = unsigned __attribute__((ext_vector_type(4)));
-    const U4 *src = (const U4 *)dense;
-    U4 *o = (U4 *)(A.out + (size_t)e * RW * NN);
-#pragma unroll
-    for (int q = lane; q < CH; q += 64) o[q] = src[q];
 }
 
 // The two-wave kernel.  The staged nodal fields and the viscous fluxes are
@@ -1132,23 +1189,16 @@ __device__ __forceinline__ void split_store(const RhsArgs<T> &A, const void *den
             DIV1 += w1;                                                                    \
         }                                                                                  \
     } while (0)
-// CL: brick-local assembly (FP64).  The block walks element clusters, one
-// after the other; the viscous wave adds each element's residual records into
+// The block walks element clusters, one after the other; the viscous wave adds each element's residual records into
 // an LDS accumulator per cluster-local node instead of storing them, and after
 // a cluster's last element finishes its interior nodes (mass inverse and
 // stage combine, as k_gather_update) and stores one partial record per
 // surface node.  mu_e runs are then pairs of elements.
-// LPS: the viscous wave evaluates full_diff_stab_ijk (elem_stab.f90:207-438)
-// instead of full_diffusion_ijk: the stabilising terms -c_lps tau_e (Proj -
-// grad) enter the fluxes, nu_e and kappa_e multiply the gradients at each
-// point before the weak divergence, and the projections (node records) and
-// tau_e come through the ring with the element's other inputs.
-template <int P, typename T, bool G16, bool CL = false, bool LPS = false>
-__global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_SPLIT_WAVES_F32) void k_rhs_split(RhsArgs<T> A)
+template <int P, typename T, bool G16>
+__global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
 {
-    using L = SplitLDS<P, T, G16, CL ? 2 : SODHIP_SPLIT_RUN, LPS>;
-    static_assert(!CL || (sizeof(T) == 8 && P == 3), "cluster assembly: FP64, p=3");
-    static_assert(!LPS || (sizeof(T) == 8 && P == 3 && !CL), "LPS: FP64, p=3, element order");
+    using L = SplitLDS<P, T, G16>;
+    static_assert(sizeof(T) == 8 && P == 3, "cluster assembly: FP64, p=3");
     using V2 = T __attribute__((ext_vector_type(2)));
     // node records of REC values: 112 bytes in FP64, an odd multiple of 16,
     // so that 16 lanes reading 16 consecutive records with 16-byte reads hit
@@ -1158,7 +1208,7 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
     // the handed-over viscous residuals (3 pairs per node), then the dense
     // residual records (RW values per node) followed by the line derivatives
     // of u and rho (6 pairs per node) from DREC on
-    constexpr int RW = split_rw<T>();
+    constexpr int RW = 5; // values per residual record
     constexpr int DREC = RW * NN / 2;
     static_assert(DREC + 6 * NN <= 64 * GREC / 2, "derivative records fit in s2");
     static_assert(NN == 64, "one lane per node");
@@ -1166,13 +1216,13 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
     __shared__ V2 s2[64 * GREC / 2];
     __shared__ __attribute__((aligned(16))) unsigned char ring[L::BYTES];
     const unsigned ring_lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)ring;
-    // cluster mode: the block's element order and local-node ranges, the
+    // the block's element order and local-node ranges, the
     // local-index rows of the last AH + 1 elements, the accumulator
     constexpr int G = kClusterG, CMAX = kClusterBlockMax, CR = AH + 1;
-    __shared__ int cel_s[CL ? CMAX * G : 1];
-    __shared__ int cb_s[CL ? 2 * CMAX : 1];
-    __shared__ __attribute__((aligned(16))) int cloc_s[CL ? CR * 64 : 1];
-    __shared__ double acc_s[CL ? 5 * kClusterLMax : 1];
+    __shared__ int cel_s[CMAX * G];
+    __shared__ int cb_s[2 * CMAX];
+    __shared__ __attribute__((aligned(16))) int cloc_s[CR * 64];
+    __shared__ double acc_s[5 * kClusterLMax];
     const unsigned cloc_lds =
         (unsigned)(uintptr_t)(__attribute__((address_space(3))) int *)cloc_s;
 
@@ -1181,69 +1231,51 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
     const bool act = true;
     const bool visc = role == 1;
 
-    constexpr int RUN = L::RUN, RSH = RUN == 4 ? 2 : 1;
+    constexpr int RUN = L::RUN, RSH = 1;
     // over runs of RUN elements, or over clusters
-    const ElemRange er = CL ? elem_range(A.ncl) : elem_range((A.nelem + RUN - 1) / RUN);
+    const ElemRange er = elem_range(A.ncl);
     if (er.begin >= er.end) return;
-    const int rlast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
     const int nunits = (er.end - er.begin + er.stride - 1) / er.stride;
-    const int nit = (CL ? G : RUN) * nunits;
-    if constexpr (CL) {
-        // a padding slot (-1) of a cluster evaluates its first element again
-        // and adds nothing
-        for (int i = threadIdx.x; i < nunits * G; i += 128) {
-            const long c = er.begin + (long)(i / G) * er.stride;
-            cel_s[i] = A.cel[c * G + i % G];
-        }
-        for (int i = threadIdx.x; i < nunits; i += 128) {
-            const long c = er.begin + (long)i * er.stride;
-            cb_s[2 * i] = A.cnb[c];
-            cb_s[2 * i + 1] = A.cnb[c + 1];
-        }
-        for (int i = threadIdx.x; i < 5 * kClusterLMax; i += 128) acc_s[i] = 0.0;
-        __syncthreads();
+    const int nit = G * nunits;
+    // a padding slot (-1) of a cluster evaluates its first element again
+    // and adds nothing
+    for (int i = threadIdx.x; i < nunits * G; i += 128) {
+        const long c = er.begin + (long)(i / G) * er.stride;
+        cel_s[i] = A.cel[c * G + i % G];
     }
+    for (int i = threadIdx.x; i < nunits; i += 128) {
+        const long c = er.begin + (long)i * er.stride;
+        cb_s[2 * i] = A.cnb[c];
+        cb_s[2 * i + 1] = A.cnb[c + 1];
+    }
+    for (int i = threadIdx.x; i < 5 * kClusterLMax; i += 128) acc_s[i] = 0.0;
+    __syncthreads();
     // element of iteration t.  Past the block's last run, and past nelem in
     // the last run, elements repeat: the copies stay unconditional and a
     // repeated element stores the same records again.  In cluster mode past
     // the block's last element the copies repeat that element.
     auto elem_of = [&](int t) {
-        if constexpr (CL) {
-            const int i = min(t, nit - 1);
-            const int e = cel_s[i];
-            return e >= 0 ? e : cel_s[i - i % G];
-        } else {
-            const long r = min((long)er.begin + (long)(t / RUN) * er.stride, (long)rlast);
-            return (int)min(r * RUN + t % RUN, (long)A.nelem - 1);
-        }
+        const int i = min(t, nit - 1);
+        const int e = cel_s[i];
+        return e >= 0 ? e : cel_s[i - i % G];
     };
-    const int elast = elem_of(nit - 1);
     // FP64 mu_e blocks: iteration t (t >= -2 RUN) copies its share of the
     // block of run t/RUN + 2 (floor); the block of run r is read from
     // iteration RUN r on
     auto mu_at = [&](int t) {
-        if constexpr (L::MUBLK) {
-            const int r = (t >> RSH) + 2;
-            const unsigned blk = ring_lds + L::MUB_AT + (r % 3) * L::MUB;
-            if constexpr (CL) {
-                mu_issue2<T>(A, blk, elem_of(r * RUN), elem_of(r * RUN + 1), t & (RUN - 1), lane);
-            } else {
-                const long g = min((long)er.begin + (long)r * er.stride, (long)rlast);
-                mu_issue<T>(A, blk, (int)(g * RUN), t & 3, lane);
-            }
-        }
+        const int r = (t >> RSH) + 2;
+        const unsigned blk = ring_lds + L::MUB_AT + (r % 3) * L::MUB;
+        mu_issue2<T>(A, blk, elem_of(r * RUN), elem_of(r * RUN + 1), t & (RUN - 1), lane);
     };
     auto mu_read = [&](int t, int node) {
         return ((const T *)(ring + L::MUB_AT + ((t >> RSH) % 3) * L::MUB))[node * RUN + (t & (RUN - 1))];
     };
-    // cluster mode: the local-index row of iteration t's element, copied by
+    // the local-index row of iteration t's element, copied by
     // the viscous wave with its share of that element's inputs
     auto cloc_issue = [&](int t) {
-        if constexpr (CL) {
-            const int i = min(t, nit - 1);
-            const long c = er.begin + (long)(i / G) * er.stride;
-            dma_lds<4>(A.cloc + ((size_t)c * G + i % G) * NN + lane, cloc_lds + (t % CR) * 256);
-        }
+        const int i = min(t, nit - 1);
+        const long c = er.begin + (long)(i / G) * er.stride;
+        dma_lds<4>(A.cloc + ((size_t)c * G + i % G) * NN + lane, cloc_lds + (t % CR) * 256);
     };
     auto slot_of = [&](int t) { return (t % AH) * L::SLOT; };
     auto crow_of = [&](int t) { return AH * L::SLOT + (t % L::CROWS) * L::CROW; };
@@ -1256,9 +1288,6 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
     // lexicographic positions nd and 32 + nd.
     auto lex = [&](int r) { return min(max(A.perm[r], 0), NN - 1); };
     int a, ia0, ia1;
-    // LPS: element-local index of the node whose projection piece lane
-    // copies in row r (lexicographic position (64r + lane)/6)
-    int ik[LPS ? L::PJ_ROWS : 1];
     {
         int *inv = (int *)s1;
         if (role == 0) inv[lex(lane)] = lane;
@@ -1266,17 +1295,8 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
         a = min(max(inv[lane], 0), NN - 1);
         ia0 = min(max(inv[nd], 0), NN - 1);
         ia1 = min(max(inv[32 + nd], 0), NN - 1);
-        if constexpr (LPS)
-#pragma unroll
-            for (int r = 0; r < L::PJ_ROWS; ++r)
-                ik[r] = min(max(inv[(64 * r + lane) / 6], 0), NN - 1);
         lds_barrier();
     }
-    auto lps_at = [&](int t, const int *c) {
-        if constexpr (LPS)
-            lps_issue<T, L::PJ_ROWS, L::PJ_AT, L::TAU_AT>(A, ring_lds + slot_of(t), c, ik,
-                                                           elem_of(t), lane);
-    };
     const int pa = lane;
     LineTab<P, T> lt;
     build_linetab<P, T>(a, A.dl, A.inv, A.gI, A.gJ, A.gK, lt);
@@ -1305,7 +1325,6 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
                                       elem_of(t + AH), n0, n1, lane);
             mu_at(t - AH);
             cloc_issue(t);
-            lps_at(t, c);
         } else
             split_issue<P, T, G16, 0>(A, ring_lds + slot_of(t), ring_lds + crow_of(t + AH), elem_of(t),
                                       elem_of(t + AH), n0, n1, lane);
@@ -1367,7 +1386,7 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
             lds_barrier(); // B1
             if (t != 0) finish();
             T He[3][3], vol;
-            split_read<P, T, G16>(ring + slot_of(t), a, pa, false, He, vol, cur);
+            split_read<P, T, G16>(ring + slot_of(t), a, pa, He, vol, cur);
             T rho, u[3], q[3], H, rhoH;
             {
                 double r, ud[3], pd, hd, Td, umag;
@@ -1512,19 +1531,17 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
         for (int k = 0; k < 3; ++k)
 #pragma unroll
             for (int o = 0; o < P; ++o) gnb[k][o] = lex(lt.off[k][o]) * GREC + 6 * k;
-        // cluster mode: adds iteration tt's dense records (s2, lexicographic
+        // adds iteration tt's dense records (s2, lexicographic
         // node order) into the accumulator at the element's local nodes (64
         // distinct local nodes per element: no two lanes collide)
         auto cl_accumulate = [&](int tt) {
-            if constexpr (CL) {
-                const int i = min(tt, nit - 1);
-                if (cel_s[i] < 0) return; // padding slot
-                const int sl = min(max(cloc_s[(tt % CR) * 64 + lane], 0), kClusterLMax - 1);
-                const T *d = (const T *)s2 + RW * lane;
-                double *ac = acc_s + 5 * sl;
+            const int i = min(tt, nit - 1);
+            if (cel_s[i] < 0) return; // padding slot
+            const int sl = min(max(cloc_s[(tt % CR) * 64 + lane], 0), kClusterLMax - 1);
+            const T *d = (const T *)s2 + RW * lane;
+            double *ac = acc_s + 5 * sl;
 #pragma unroll
-                for (int f = 0; f < 5; ++f) ac[f] += (double)d[f];
-            }
+            for (int f = 0; f < 5; ++f) ac[f] += (double)d[f];
         };
         // cluster mode, after the last element of the cluster of iteration tt:
         // interior working nodes get R = fact * sum * invMl and the stage
@@ -1532,67 +1549,56 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
         // elements in the same ascending order), surface working nodes one
         // partial record; the accumulator is cleared for the next cluster
         auto cl_flush = [&](int tt) {
-            if constexpr (CL) {
-                const int k = min(tt, nit - 1) / G;
-                const int base = cb_s[2 * k], lim = cb_s[2 * k + 1];
-                const size_t np = (size_t)A.npoin;
-                for (int l = base + lane; l < lim; l += 64) {
-                    double v[5];
-                    double *ac = acc_s + 5 * (l - base);
+            const int k = min(tt, nit - 1) / G;
+            const int base = cb_s[2 * k], lim = cb_s[2 * k + 1];
+            const size_t np = (size_t)A.npoin;
+            for (int l = base + lane; l < lim; l += 64) {
+                double v[5];
+                double *ac = acc_s + 5 * (l - base);
+#pragma unroll
+                for (int f = 0; f < 5; ++f) {
+                    v[f] = ac[f];
+                    ac[f] = 0.0;
+                }
+                const int kind = A.ckind[l];
+                if (kind == 1) {
+                    double *r = A.rec + 5 * (size_t)l;
+#pragma unroll
+                    for (int f = 0; f < 5; ++f) r[f] = v[f];
+                } else if (kind == 0) {
+                    const size_t n = (size_t)A.cnode[l];
+                    const size_t k3[5] = {n, n, n + np, n + 2 * np, n};
+                    const double *y1v[5] = {A.y1r, A.y1q, A.y1q, A.y1q, A.y1E};
+                    double *yv[5] = {A.yr, A.yq, A.yq, A.yq, A.yE};
+                    double *rv[5] = {A.Rm, A.Rq, A.Rq, A.Rq, A.Re};
+                    double *xv[5] = {A.nxr, A.nxq, A.nxq, A.nxq, A.nxE};
+                    const double m = A.invMl[n];
+                    double b[5], y[5];
 #pragma unroll
                     for (int f = 0; f < 5; ++f) {
-                        v[f] = ac[f];
-                        ac[f] = 0.0;
+                        b[f] = A.rd1 ? y1v[f][k3[f]] : 0.0;
+                        y[f] = A.rdy ? yv[f][k3[f]] : 0.0;
                     }
-                    const int kind = A.ckind[l];
-                    if (kind == 1) {
-                        double *r = A.rec + 5 * (size_t)l;
 #pragma unroll
-                        for (int f = 0; f < 5; ++f) r[f] = v[f];
-                    } else if (kind == 0) {
-                        const size_t n = (size_t)A.cnode[l];
-                        const size_t k3[5] = {n, n, n + np, n + 2 * np, n};
-                        const double *y1v[5] = {A.y1r, A.y1q, A.y1q, A.y1q, A.y1E};
-                        double *yv[5] = {A.yr, A.yq, A.yq, A.yq, A.yE};
-                        double *rv[5] = {A.Rm, A.Rq, A.Rq, A.Rq, A.Re};
-                        double *xv[5] = {A.nxr, A.nxq, A.nxq, A.nxq, A.nxE};
-                        const double m = A.invMl[n];
-                        double b[5], y[5];
-#pragma unroll
-                        for (int f = 0; f < 5; ++f) {
-                            b[f] = A.rd1 ? y1v[f][k3[f]] : 0.0;
-                            y[f] = A.rdy ? yv[f][k3[f]] : 0.0;
+                    for (int f = 0; f < 5; ++f) {
+                        const double r = (A.fact * v[f]) * m;
+                        const double z = A.lam1 * b[f] + A.lams * y[f] + A.gdt * r;
+                        yv[f][k3[f]] = z;
+                        if (A.nxr) {
+                            const double zero = 0.0, nls = 0.0;
+                            xv[f][k3[f]] = A.nx_l1 * z + nls * zero + A.nx_gdt * r;
                         }
-#pragma unroll
-                        for (int f = 0; f < 5; ++f) {
-                            const double r = (A.fact * v[f]) * m;
-                            const double z = A.lam1 * b[f] + A.lams * y[f] + A.gdt * r;
-                            yv[f][k3[f]] = z;
-                            if (A.nxr) {
-                                const double zero = 0.0, nls = 0.0;
-                                xv[f][k3[f]] = A.nx_l1 * z + nls * zero + A.nx_gdt * r;
-                            }
-                            if (A.Rm) rv[f][k3[f]] = r;
-                        }
+                        if (A.Rm) rv[f][k3[f]] = r;
                     }
                 }
             }
         };
         for (int t = 0; t < nit; ++t) {
-            wait_vm<(AH - 1) * (L::NOPS1 + (CL ? 1 : 0))>();
+            wait_vm<(AH - 1) * (L::NOPS1 + 1)>();
             lds_barrier(); // B1
             T He[3][3], vol;
-            split_read<P, T, G16>(ring + slot_of(t), a, pa, true, He, vol, cur);
-            if constexpr (L::MUBLK) cur.mue = mu_read(t, a);
-            // LPS: the node's projection record and tau_e, read before B2 (the
-            // copies of element t + AH then start into this slot)
-            double pj[LPS ? kProjRec : 1], taus = 0.0;
-            if constexpr (LPS) {
-                const double *pr = (const double *)(ring + slot_of(t) + L::PJ_AT) + kProjRec * pa;
-#pragma unroll
-                for (int j = 0; j < kProjRec; ++j) pj[j] = pr[j];
-                taus = *(const double *)(ring + slot_of(t) + L::TAU_AT);
-            }
+            split_read<P, T, G16>(ring + slot_of(t), a, pa, He, vol, cur);
+ cur.mue = mu_read(t, a);
             T rho, u[3], Tk, muf;
             const T mue = cur.mue;
             {
@@ -1607,26 +1613,20 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
                 if (act) s1[(own + 10) >> 1] = V2{Tk, T(0)};
             }
             lds_barrier(); // B2
-            // cluster mode: the previous element's records go into the
+            // the previous element's records go into the
             // accumulator before its local-index row is overwritten below
-            if constexpr (CL)
-                if (t != 0) cl_accumulate(t - 1);
+            if (t != 0) cl_accumulate(t - 1);
             {
                 const int *c = (const int *)(ring + crow_of(t + AH));
                 split_issue<P, T, G16, 1>(A, ring_lds + slot_of(t), ring_lds + crow_of(t + 2 * AH),
                                           elem_of(t + AH), elem_of(t + 2 * AH), c[ia0], c[ia1], lane);
                 mu_at(t);
                 cloc_issue(t + AH);
-                lps_at(t + AH, c);
             }
             // residual records of the previous element, completed in s2 by the
             // convection wave: their stores complete while this element runs
             // (read here, before this wave's flux records overwrite s2)
-            if constexpr (CL) {
-                if (t != 0 && t % G == 0) cl_flush(t - 1);
-            } else if (t != 0) {
-                split_store<P, T>(A, s2, elem_of(t - 1), lane);
-            }
+            if (t != 0 && t % G == 0) cl_flush(t - 1);
             // grad T from the T lines; grad u and grad rho from the line
             // derivatives handed over by the convection wave
             T dT[3];
@@ -1657,91 +1657,31 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
                 gt[i] = He[i][0] * dT[0] + He[i][1] * dT[1] + He[i][2] * dT[2];
             }
             // contravariant fluxes G_k(F) = gpvol sum_d He(d,k) F_d into the flux record
-            if constexpr (LPS) {
-                // full_diff_stab_ijk's fluxes at the point (mu_sgs = 0), in
-                // the arithmetic of k_diff_stab; record per k: mass, energy,
-                // (unused), momentum 1..3
-                const double rhon = rho, mufl = muf, musgs = 0.0;
-                const double twoThirds = 2.0 / 3.0;
-                const double divU = gU[0][0] + gU[1][1] + gU[2][2];
-                const double nu_e = A.c_rho * mue / rhon;
-                const double mu_fgp = mufl + rhon * musgs;
-                const double kappa_e = mufl * A.Cp / A.Pr + A.c_ener * mue * A.Cp / A.Pr +
-                                       A.Cp * rhon * musgs / 0.9;
-                const double cl = -A.c_lps * taus;
-                // projected tensor rows from its upper triangle t11 t12 t13 t22 t23 t33
-                const int at[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
-                double F[5][3];
+            const T mut = muf + mue;
+            const T divU = gU[0][0] + gU[1][1] + gU[2][2];
+            const T tdiv = muf * T(2.0 / 3.0) * divU;
+            T tau[3][3];
 #pragma unroll
-                for (int i = 0; i < 3; ++i)
+            for (int i = 0; i < 3; ++i)
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        double tt2 = gU[i][d] + gU[d][i];
-                        if (i == d) tt2 = tt2 - twoThirds * divU;
-                        F[1 + i][d] = cl * (pj[at[3 * i + d]] - tt2) * rhon;
-                    }
+                for (int j = 0; j < 3; ++j) tau[i][j] = mut * (gU[i][j] + gU[j][i]);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    F[4][d] = cl * (pj[9 + d] - gt[d]) * rhon * A.Cp / A.Pr;
-                    F[0][d] = cl * (pj[6 + d] - gR[d]);
+            for (int i = 0; i < 3; ++i) tau[i][i] -= tdiv;
+            const int g = pa * GREC;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const T h0 = vol * He[0][k], h1 = vol * He[1][k], h2 = vol * He[2][k];
+                T gr[3], tuk = 0;
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    gr[r] = h0 * tau[r][0] + h1 * tau[r][1] + h2 * tau[r][2];
+                    tuk += gr[r] * u[r]; // tau is symmetric: contravariant (tau u)_k
                 }
-                double tauU[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        tauU[i] = tauU[i] + (mu_fgp + mue) * (gU[i][j] + gU[j][i]) * u[j];
-                        double tv = (mu_fgp + mue) * (gU[i][j] + gU[j][i]);
-                        if (i == j) tv = tv - mu_fgp * twoThirds * divU;
-                        F[1 + i][j] = F[1 + i][j] + tv;
-                    }
-                    tauU[i] = tauU[i] - mu_fgp * twoThirds * divU * u[i];
-                }
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    F[4][d] = F[4][d] + kappa_e * gt[d] + tauU[d];
-                    F[0][d] = F[0][d] + nu_e * gR[d];
-                }
-                const int g = pa * GREC;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    double Gf[5];
-#pragma unroll
-                    for (int f = 0; f < 5; ++f)
-                        Gf[f] = vol * (He[0][k] * F[f][0] + He[1][k] * F[f][1] + He[2][k] * F[f][2]);
-                    if (act) {
-                        s2[(g + 6 * k + 0) >> 1] = V2{Gf[0], Gf[4]};
-                        s2[(g + 6 * k + 2) >> 1] = V2{T(0), Gf[1]};
-                        s2[(g + 6 * k + 4) >> 1] = V2{Gf[2], Gf[3]};
-                    }
-                }
-            } else {
-                const T mut = muf + mue;
-                const T divU = gU[0][0] + gU[1][1] + gU[2][2];
-                const T tdiv = muf * T(2.0 / 3.0) * divU;
-                T tau[3][3];
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) tau[i][j] = mut * (gU[i][j] + gU[j][i]);
-#pragma unroll
-                for (int i = 0; i < 3; ++i) tau[i][i] -= tdiv;
-                const int g = pa * GREC;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const T h0 = vol * He[0][k], h1 = vol * He[1][k], h2 = vol * He[2][k];
-                    T gr[3], tuk = 0;
-#pragma unroll
-                    for (int r = 0; r < 3; ++r) {
-                        gr[r] = h0 * tau[r][0] + h1 * tau[r][1] + h2 * tau[r][2];
-                        tuk += gr[r] * u[r]; // tau is symmetric: contravariant (tau u)_k
-                    }
-                    if (act) {
-                        s2[(g + 6 * k + 0) >> 1] = V2{h0 * gR[0] + h1 * gR[1] + h2 * gR[2],
-                                                    h0 * gt[0] + h1 * gt[1] + h2 * gt[2]};
-                        s2[(g + 6 * k + 2) >> 1] = V2{tuk, gr[0]};
-                        s2[(g + 6 * k + 4) >> 1] = V2{gr[1], gr[2]};
-                    }
+                if (act) {
+                    s2[(g + 6 * k + 0) >> 1] = V2{h0 * gR[0] + h1 * gR[1] + h2 * gR[2],
+                                                h0 * gt[0] + h1 * gt[1] + h2 * gt[2]};
+                    s2[(g + 6 * k + 2) >> 1] = V2{tuk, gr[0]};
+                    s2[(g + 6 * k + 4) >> 1] = V2{gr[1], gr[2]};
                 }
             }
             // this wave alone reads s2 next: its LDS instructions execute in order
@@ -1778,27 +1718,16 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
             if (act) {
-                if constexpr (LPS) {
-                    // nu_e and kappa_e are inside the fluxes
-                    s2[3 * pa] = V2{W6[0], W6[3]};
-                    s2[3 * pa + 1] = V2{W6[4], W6[5]};
-                    s2[3 * pa + 2] = V2{W6[1], T(0)};
-                } else {
-                    s2[3 * pa] = V2{nu_e * W6[0], W6[3]};
-                    s2[3 * pa + 1] = V2{W6[4], W6[5]};
-                    s2[3 * pa + 2] = V2{W6[2] + kappa * W6[1], T(0)};
-                }
+                s2[3 * pa] = V2{nu_e * W6[0], W6[3]};
+                s2[3 * pa + 1] = V2{W6[4], W6[5]};
+                s2[3 * pa + 2] = V2{W6[2] + kappa * W6[1], T(0)};
             }
         }
         // the last element's records, completed by the convection wave
         lds_barrier();
         lds_barrier();
-        if constexpr (CL) {
-            cl_accumulate(nit - 1);
-            cl_flush(nit - 1);
-        } else {
-            split_store<P, T>(A, s2, elast, lane);
-        }
+        cl_accumulate(nit - 1);
+        cl_flush(nit - 1);
     }
     // no copy may still be writing this block's LDS when it retires
     wait_vm<0>();
@@ -1810,7 +1739,7 @@ __global__ __launch_bounds__(128, sizeof(T) == 8 ? SODHIP_SPLIT_WAVES : SODHIP_S
 
 // Launches the operators' element kernel.  bpc: the stage's blocks-per-CU setting
 // (16: the kernel's own launch shape; others scale the units a block takes).
-template <int P, typename T, bool CONV, bool VISC, bool CONS>
+template <int P, typename T, bool CONV, int VISC, bool CONS>
 static void launch_rhs_p(sodhip_ctx ctx, RhsArgs<T> A, int bpc)
 {
     const UnitShape us = unit_shape<P, T>(ctx, A.nelem, bpc);
@@ -1829,11 +1758,11 @@ static int launch_rhs(sodhip_ctx ctx, int porder, bool conv, bool diff, bool con
 #define SODHIP_RHS_CASE(PP)                                                                \
     case PP:                                                                               \
         if (conv && diff && cons)                                                          \
-            launch_rhs_p<PP, T, true, true, true>(ctx, A, bpc);                            \
+            launch_rhs_p<PP, T, true, 1, true>(ctx, A, bpc);                            \
         else if (conv && !diff && !cons)                                                   \
-            launch_rhs_p<PP, T, true, false, false>(ctx, A, bpc);                          \
+            launch_rhs_p<PP, T, true, 0, false>(ctx, A, bpc);                          \
         else if (!conv && diff && !cons)                                                   \
-            launch_rhs_p<PP, T, false, true, false>(ctx, A, bpc);                          \
+            launch_rhs_p<PP, T, false, 1, false>(ctx, A, bpc);                          \
         else                                                                               \
             return set_error(SODHIP_ERR_UNSUPPORTED, "unsupported operator combination");  \
         break;
@@ -1878,43 +1807,6 @@ static int check_common(sodhip_ctx ctx, int porder, int nelem, int npoin, const 
     SODHIP_REQUIRE(nelem > 0 && npoin > 0 && connec, "invalid mesh arguments");
     return SODHIP_OK;
 }
-
-// full_convec_ijk's element records only (5 values per element-node, unscaled,
-// at e*nnode + perm[a] of out), for stage drivers that add more terms to the
-// same records before one gather
-template <typename T>
-int conv_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *He, const T *gpvol,
-                  const T *dl, const int *inv, const int *gI, const int *gJ, const int *gK,
-                  const T *u, const T *q, const T *rho, const T *pr, const T *E, T *out)
-{
-    RhsArgs<T> A{};
-    A.nelem = m->nelem;
-    A.npoin = m->npoin;
-    A.EN = (size_t)m->nelem * nnode_of(porder);
-    A.connecT = m->connecT;
-    A.perm = m->perm;
-    A.He = He;
-    A.gpvol = gpvol;
-    A.dl = dl;
-    A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
-    A.u = u;
-    A.q = q;
-    A.rho = rho;
-    A.pr = pr;
-    A.E = E;
-    A.out = out;
-    int tok = prof_begin(ctx, 0);
-    const int rc = launch_rhs<T>(ctx, porder, true, false, false, A);
-    prof_end(ctx, tok);
-    return rc;
-}
-template int conv_elements<double>(sodhip_ctx, int, const MeshCache *, const double *,
-                                   const double *, const double *, const int *, const int *,
-                                   const int *, const int *, const double *, const double *,
-                                   const double *, const double *, const double *, double *);
 
 template <typename T>
 static int full_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const int *connec,
@@ -2142,74 +2034,75 @@ int rhs_cluster_stage(sodhip_ctx ctx, const MeshCache *m, const ClusterTables *c
     const int grid = (int)(8 * per);
     int tok = prof_begin(ctx, 0);
     if (A.geo16)
-        k_rhs_split<3, T, true, true><<<grid, 128, 0, ctx->stream>>>(A);
+        k_rhs_split<3, T, true><<<grid, 128, 0, ctx->stream>>>(A);
     else
-        k_rhs_split<3, T, false, true><<<grid, 128, 0, ctx->stream>>>(A);
+        k_rhs_split<3, T, false><<<grid, 128, 0, ctx->stream>>>(A);
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());
     return SODHIP_OK;
 }
 
-// blocks of 128 threads of kernel k resident on one CU (at least 1)
-template <typename K> static int lps_resident(K k)
+// The LPS operators' element kernels (LpsArgs, common.hpp): the fused stage's
+// convection and stabilised viscous operator from the conserved state (`stage`),
+// the drop-in stabilised operator, or the projections' records.
+int lps_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const LpsArgs &L, LpsKernel what)
 {
-    int r = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, k, 128, 0) != hipSuccess) r = 1;
-    return std::max(r, 1);
-}
-
-int rhs_lps_elements(sodhip_ctx ctx, const MeshCache *m, const double *He, const double *gpvol,
-                     const double *dl, const int *inv, const int *gI, const int *gJ, const int *gK,
-                     const double *rho, const double *q, const double *E, const double *mu_e,
-                     const double *prj, const double *tau, double gamma, double Rgas, double Cp,
-                     double Pr, double mu_factor, double c_rho, double c_ener, double c_lps,
-                     double *out)
-{
-    using T = double;
-    RhsArgs<T> A{};
+    RhsArgs<double> A{};
     A.nelem = m->nelem;
     A.npoin = m->npoin;
-    A.EN = (size_t)m->nelem * 64;
+    A.EN = (size_t)m->nelem * nnode_of(porder);
     A.connecT = m->connecT;
     A.perm = m->perm;
-    A.He = He;
-    A.gpvol = gpvol;
-    A.dl = dl;
-    A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
-    A.cr = rho;
-    A.cq = q;
-    A.cE = E;
-    A.mu_e = mu_e;
-    A.gamma = gamma;
-    A.Rgas = Rgas;
-    A.mu_factor = mu_factor;
-    A.p_ref = 0.0;
-    A.Cp = Cp;
-    A.Pr = Pr;
-    A.c_rho = c_rho;
-    A.c_ener = c_ener;
-    A.prj = prj;
-    A.tau = tau;
-    A.c_lps = c_lps;
-    A.out = out;
-    A.geo16 = ctx->stage_geo16 && ((uintptr_t)He % 16 == 0) && ((uintptr_t)gpvol % 16 == 0);
-    // the grid is a whole number of rounds of the blocks a CU holds at once:
-    // the LPS mode's LDS leaves room for 3, where the plain kernel has 4 and
-    // the stage's blocks-per-CU setting is tuned for it (16 blocks per CU
-    // would leave a third of a round: 1.35 ms against 1.30 ms at 64^3)
-    static const int res16 = lps_resident(k_rhs_split<3, T, true, false, true>);
-    static const int res4 = lps_resident(k_rhs_split<3, T, false, false, true>);
-    const int res = A.geo16 ? res16 : res4;
-    const int grid = elem_grid(ctx, m->nelem, std::max(res, ctx->stage_bpc / res * res));
-    int tok = prof_begin(ctx, 0);
-    if (A.geo16)
-        k_rhs_split<3, T, true, false, true><<<grid, 128, 0, ctx->stream>>>(A);
-    else
-        k_rhs_split<3, T, false, false, true><<<grid, 128, 0, ctx->stream>>>(A);
-    prof_end(ctx, tok);
+    A.He = L.He;
+    A.gpvol = L.gpvol;
+    A.dl = L.dl;
+    A.inv = L.inv;
+    A.rho = L.rho;
+    A.u = L.u;
+    A.Tem = L.Tem;
+    A.rho_n = L.rho_n;
+    A.mu_fluid = L.mu_fluid;
+    A.mu_e = L.mu_e;
+    A.mu_sgs = L.mu_sgs;
+    A.cr = L.cr;
+    A.cq = L.cq;
+    A.cE = L.cE;
+    A.gamma = L.gamma;
+    A.Rgas = L.Rgas;
+    A.mu_factor = L.mu_factor;
+    A.Cp = L.Cp;
+    A.Pr = L.Pr;
+    A.c_rho = L.c_rho;
+    A.c_ener = L.c_ener;
+    A.c_lps = L.c_lps;
+    A.tau = L.tau;
+    A.prj = L.prj;
+    A.pMass = L.pMass;
+    A.pEner = L.pEner;
+    A.pMX = L.pMX;
+    A.pMY = L.pMY;
+    A.pMZ = L.pMZ;
+    A.out = L.out;
+    A.geo16 = (what != LpsKernel::stage || ctx->stage_geo16) && ((uintptr_t)A.He % 16 == 0) &&
+              ((uintptr_t)A.gpvol % 16 == 0);
+    const int bpc = what == LpsKernel::stage ? ctx->stage_bpc : 16;
+#define SODHIP_LPS_CASE(PP)                                                                \
+    case PP:                                                                               \
+        if (what == LpsKernel::stage)                                                      \
+            launch_rhs_p<PP, double, true, 2, true>(ctx, A, bpc);                          \
+        else if (what == LpsKernel::stab)                                                  \
+            launch_rhs_p<PP, double, false, 2, false>(ctx, A, bpc);                        \
+        else                                                                               \
+            launch_rhs_p<PP, double, false, 3, false>(ctx, A, bpc);                        \
+        break;
+    switch (porder) {
+        SODHIP_LPS_CASE(2)
+        SODHIP_LPS_CASE(3)
+        SODHIP_LPS_CASE(4)
+    default:
+        return set_error(SODHIP_ERR_UNSUPPORTED, "porder %d not supported (2..4)", porder);
+    }
+#undef SODHIP_LPS_CASE
     SODHIP_TRY_HIP(hipGetLastError());
     return SODHIP_OK;
 }

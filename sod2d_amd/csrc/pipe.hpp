@@ -48,6 +48,9 @@ template <int N> __device__ __forceinline__ void wait_vm()
 // this wave's LDS reads have returned: a copy may overwrite what they read
 __device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+// the value is formed by here (the compiler may not move its computation further on)
+template <typename U> __device__ __forceinline__ void pin(U &x) { asm volatile("" : "+v"(x)); }
+
 // LDS address of a __shared__ array
 template <typename U> __device__ __forceinline__ unsigned lds_addr(U *p)
 {
