@@ -13,10 +13,8 @@
 namespace sodhip {
 
 // comp_tau (elem_stab.f90:589-616): tau_e = max over the element's nodes of
-// h (fact_c c + |u|), h = helem_k (c_species_stab / p); one thread per
-// element over the reference's element-fastest connec, the nodes visited an
-// i-line at a time (build_alex) with all loads of a line issued together
-// (fmax is exact).
+// h (fact_c c + |u|), h = helem_k (c_species_stab / p), over tiles of 16 elements
+// (device.hpp), all loads of an i-line issued together (fmax is exact).
 __global__ __launch_bounds__(256) void k_comp_tau(int nelem, int nnode, int porder,
                                                   const int *__restrict__ connec,
                                                   const int *__restrict__ perm,
@@ -26,33 +24,37 @@ __global__ __launch_bounds__(256) void k_comp_tau(int nelem, int nnode, int pord
                                                   double c_species_stab, double fact_c,
                                                   double *__restrict__ tau)
 {
+    __shared__ double sh[64];
     __shared__ int alex[125];
     build_alex(perm, nnode, alex);
-    const int e = xcd_block() * blockDim.x + threadIdx.x;
-    if (e >= nelem) return;
-    const double h = helem_k[e] * (c_species_stab / (double)porder);
-    const int KA = porder + 1;
-    double taul = 0.0;
-    for (int l0 = 0; l0 < nnode; l0 += KA) {
-        int n[5];
+    const int KA = porder + 1, nl = KA * KA;
+    const TileRange tr = tile_range(nelem);
+    for (int t = tr.first; t < tr.end; t += tr.stride) {
+        const int el = t * kTile + (threadIdx.x & 15), e = min(el, nelem - 1);
+        const double h = helem_k[e] * (c_species_stab / (double)porder);
+        double taul = 0.0;
+        for (int l = threadIdx.x >> 4; l < nl; l += 16) {
+            int n[5];
 #pragma unroll
-        for (int j = 0; j < 5; ++j)
-            n[j] = connec[e + (size_t)nelem * alex[min(l0 + min(j, KA - 1), nnode - 1)]] - 1;
-        double u0[5], u1[5], u2[5], cs[5];
+            for (int j = 0; j < 5; ++j)
+                n[j] = connec[e + (size_t)nelem * alex[l * KA + min(j, KA - 1)]] - 1;
+            double u0[5], u1[5], u2[5], cs[5];
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            u0[j] = u[n[j]];
-            u1[j] = u[n[j] + (size_t)npoin];
-            u2[j] = u[n[j] + 2 * (size_t)npoin];
-            cs[j] = csound[n[j]];
+            for (int j = 0; j < 5; ++j) {
+                u0[j] = u[n[j]];
+                u1[j] = u[n[j] + (size_t)npoin];
+                u2[j] = u[n[j] + 2 * (size_t)npoin];
+                cs[j] = csound[n[j]];
+            }
+#pragma unroll
+            for (int j = 0; j < 5; ++j) {
+                const double aux1 = fact_c * cs[j] + sqrt(u0[j] * u0[j] + u1[j] * u1[j] + u2[j] * u2[j]);
+                taul = fmax(taul, h * aux1);
+            }
         }
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            const double aux1 = fact_c * cs[j] + sqrt(u0[j] * u0[j] + u1[j] * u1[j] + u2[j] * u2[j]);
-            taul = fmax(taul, h * aux1);
-        }
+        taul = tile_max(taul, sh);
+        if (threadIdx.x < kTile && el < nelem) tau[e] = taul;
     }
-    tau[e] = taul;
 }
 
 // Node-ordered assemblies.  Node n's slots row[n]..row[n+1]-1 are taken four
@@ -226,7 +228,7 @@ extern "C" int sodhip_comp_tau_f64(sodhip_ctx ctx, int porder, int nelem, int np
     MeshCache *m = nullptr;
     int rc = get_mesh(ctx, porder, nelem, npoin, connec, &m);
     if (rc) return rc;
-    k_comp_tau<<<tpe_grid(nelem), 256, 0, ctx->stream>>>(
+    k_comp_tau<<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>(
         nelem, nn, porder, connec, m->perm, csound, u, npoin, helem_k, c_species_stab,
         flag_drop_c_in_envit ? 0.0 : 1.0, tau);
     SODHIP_TRY_HIP(hipGetLastError());

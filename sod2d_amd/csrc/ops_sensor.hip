@@ -206,14 +206,13 @@ __global__ __launch_bounds__(kRedThreads) void k_rho_min(int npoin_w, const int 
     if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
-// smart_visc_spectral_imex (mod_entropy_viscosity.f90:113-227), one thread per
-// element over the reference's element-fastest connec, mu_e and mue_l (for a
-// node position the lanes of a wave read and write consecutive entries):
-// mue_l <- incoming mu_e; beta_e = max over the nodes of rho helem_k (cmax/p)
+// smart_visc_spectral_imex (mod_entropy_viscosity.f90:113-227) over tiles of 16
+// elements (device.hpp): mue_l <- incoming mu_e; beta_e = max over the nodes of rho helem_k (cmax/p)
 // (|u| + fact c); mu_e = cglob min(ce rho |Reta|/norm (helem_k/p)^2, beta_e).
 // norm: 1, or the max of the partials (max |eta - mean|), or the min of the
-// partials (min rho), folded per block.  The nodes are visited an i-line at a
-// time (build_alex) with all loads of a line issued together.
+// partials (min rho), folded per block.  All loads of an i-line are issued
+// together; density and residual stay in registers between the maximum and the
+// write.
 struct ImexArgs {
     int nelem, nnode, porder;
     const int *connec, *perm;
@@ -237,60 +236,60 @@ __global__ __launch_bounds__(256) void k_visc_imex(ImexArgs A)
             v = A.norm_min ? fmin(v, A.part[i]) : fmax(v, A.part[i]);
         norm = A.norm_min ? block_min(v, sh) : block_max(v, sh);
     }
-    const int e = xcd_block() * blockDim.x + threadIdx.x;
-    if (e >= A.nelem) return;
     const size_t NE = (size_t)A.nelem;
     const double *u1 = A.u + A.npoin, *u2 = A.u + 2 * (size_t)A.npoin;
-    const double hk = A.helem_k[e], cp = A.cmax / (double)A.porder;
-    const int KA = A.porder + 1;
-    double betae = 0.0;
-    for (int l0 = 0; l0 < A.nnode; l0 += KA) {
-        size_t ea[5];
-        int n[5];
-        double mu[5], v0[5], v1[5], v2[5], cs[5], rh[5];
+    const double cp = A.cmax / (double)A.porder;
+    const int KA = A.porder + 1, nl = KA * KA;
+    const TileRange tr = tile_range(A.nelem);
+    for (int t = tr.first; t < tr.end; t += tr.stride) {
+        const int el = t * kTile + (threadIdx.x & 15), e = min(el, A.nelem - 1);
+        const double hk = A.helem_k[e];
+        double betae = 0.0;
+        double rh[kTileLines][5], re[kTileLines][5];
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            ea[j] = e + NE * alex[min(l0 + min(j, KA - 1), A.nnode - 1)];
-            n[j] = A.connec[ea[j]] - 1;
-            mu[j] = A.mu_e[ea[j]];
+        for (int r = 0; r < kTileLines; ++r) {
+            const int l = (threadIdx.x >> 4) + 16 * r;
+            if (l >= nl) break;
+            size_t ea[5];
+            int n[5];
+            double mu[5], v0[5], v1[5], v2[5], cs[5];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) {
+                ea[j] = e + NE * alex[l * KA + min(j, KA - 1)];
+                n[j] = A.connec[ea[j]] - 1;
+                mu[j] = A.mu_e[ea[j]];
+            }
+#pragma unroll
+            for (int j = 0; j < 5; ++j) {
+                v0[j] = A.u[n[j]];
+                v1[j] = u1[n[j]];
+                v2[j] = u2[n[j]];
+                cs[j] = A.csound[n[j]];
+                rh[r][j] = A.rho[n[j]];
+                re[r][j] = A.Reta[n[j]];
+            }
+#pragma unroll
+            for (int j = 0; j < 5; ++j) {
+                if (j < KA && el < A.nelem) A.mue_l[ea[j]] = mu[j];
+                const double speed =
+                    sqrt(v0[j] * v0[j] + v1[j] * v1[j] + v2[j] * v2[j]) + A.fact_low_mach * cs[j];
+                betae = fmax(betae, (rh[r][j] * hk) * cp * speed);
+            }
         }
+        betae = tile_max(betae, sh);
+        if (el >= A.nelem) continue;
+        const double hp = hk / (double)A.porder;
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            v0[j] = A.u[n[j]];
-            v1[j] = u1[n[j]];
-            v2[j] = u2[n[j]];
-            cs[j] = A.csound[n[j]];
-            rh[j] = A.rho[n[j]];
-        }
+        for (int r = 0; r < kTileLines; ++r) {
+            const int l = (threadIdx.x >> 4) + 16 * r;
+            if (l >= nl) break;
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            if (j < KA) A.mue_l[ea[j]] = mu[j];
-            const double speed =
-                sqrt(v0[j] * v0[j] + v1[j] * v1[j] + v2[j] * v2[j]) + A.fact_low_mach * cs[j];
-            betae = fmax(betae, (rh[j] * hk) * cp * speed);
-        }
-    }
-    const double hp = hk / (double)A.porder;
-    for (int l0 = 0; l0 < A.nnode; l0 += KA) {
-        size_t ea[5];
-        int n[5];
-        double rh[5], re[5];
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            ea[j] = e + NE * alex[min(l0 + min(j, KA - 1), A.nnode - 1)];
-            n[j] = A.connec[ea[j]] - 1;
-        }
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            rh[j] = A.rho[n[j]];
-            re[j] = A.Reta[n[j]];
-        }
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            if (j >= KA) break;
-            const double R1 = rh[j] * fabs(re[j]) / norm;
-            const double Ve = A.ce * R1 * (hp * hp);
-            A.mu_e[ea[j]] = A.cglob * fmin(Ve, betae);
+            for (int j = 0; j < 5; ++j) {
+                if (j >= KA) break;
+                const double R1 = rh[r][j] * fabs(re[r][j]) / norm;
+                const double Ve = A.ce * R1 * (hp * hp);
+                A.mu_e[e + NE * alex[l * KA + j]] = A.cglob * fmin(Ve, betae);
+            }
         }
     }
 }
@@ -321,9 +320,8 @@ __global__ __launch_bounds__(256) void k_ducros_node(int npoin, const double *__
     nq[n + P2] = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
 }
 
-// the element pass: one thread per element over the reference's
-// element-fastest connec, helem and mu_e, the nodes visited an i-line at a
-// time (build_alex) with all loads of a line issued together
+// the element pass, over tiles of 16 elements (device.hpp), all loads of an i-line
+// issued together
 __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder, int npoin,
                                                 const int *__restrict__ connec,
                                                 const int *__restrict__ perm,
@@ -333,33 +331,36 @@ __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder
 {
     __shared__ int alex[125];
     build_alex(perm, nnode, alex);
-    const int e = xcd_block() * blockDim.x + threadIdx.x;
-    if (e >= nelem) return;
     const size_t P1 = (size_t)npoin, P2 = 2 * (size_t)npoin;
-    const int KA = porder + 1;
-    for (int l0 = 0; l0 < nnode; l0 += KA) {
-        size_t t[5];
-        int n[5];
+    const int KA = porder + 1, nl = KA * KA;
+    const TileRange tr = tile_range(nelem);
+    for (int tile = tr.first; tile < tr.end; tile += tr.stride) {
+        const int e = tile * kTile + (threadIdx.x & 15);
+        if (e >= nelem) continue;
+        for (int l = threadIdx.x >> 4; l < nl; l += 16) {
+            size_t t[5];
+            int n[5];
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            t[j] = (size_t)alex[min(l0 + min(j, KA - 1), nnode - 1)] * nelem + e;
-            n[j] = connec[t[j]] - 1;
-        }
-        double phi[5], d2[5], um[5], he[5], mu[5];
+            for (int j = 0; j < 5; ++j) {
+                t[j] = (size_t)alex[l * KA + min(j, KA - 1)] * nelem + e;
+                n[j] = connec[t[j]] - 1;
+            }
+            double phi[5], d2[5], um[5], he[5], mu[5];
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            phi[j] = nq[n[j]];
-            d2[j] = nq[n[j] + P1];
-            um[j] = nq[n[j] + P2];
-            he[j] = helem[t[j]];
-            mu[j] = mu_e[t[j]];
-        }
+            for (int j = 0; j < 5; ++j) {
+                phi[j] = nq[n[j]];
+                d2[j] = nq[n[j] + P1];
+                um[j] = nq[n[j] + P2];
+                he[j] = helem[t[j]];
+                mu[j] = mu_e[t[j]];
+            }
 #pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            if (j >= KA) break;
-            const double rr = 1.0 * um[j] / he[j];
-            const double phi2 = d2[j] / (d2[j] + rr * rr + DBL_EPSILON);
-            mu_e[t[j]] = mu[j] * (fmax(phi[j] - dmin, 0.0) * phi2 + dmin);
+            for (int j = 0; j < 5; ++j) {
+                if (j >= KA) break;
+                const double rr = 1.0 * um[j] / he[j];
+                const double phi2 = d2[j] / (d2[j] + rr * rr + DBL_EPSILON);
+                mu_e[t[j]] = mu[j] * (fmax(phi[j] - dmin, 0.0) * phi2 + dmin);
+            }
         }
     }
 }
@@ -675,7 +676,7 @@ extern "C" int sodhip_smart_visc_spectral_imex_f64(
     A.norm_min = high_mach ? 1 : 0;
     A.mu_e = mu_e;
     A.mue_l = mue_l;
-    k_visc_imex<<<tpe_grid(nelem), 256, 0, ctx->stream>>>(A);
+    k_visc_imex<<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>(A);
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());
     return SODHIP_OK;
@@ -701,7 +702,7 @@ extern "C" int sodhip_ducros_visc_limit_f64(sodhip_ctx ctx, int porder, int nele
     double *nq = (double *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 2);
     k_ducros_node<<<(npoin + 255) / 256, 256, 0, ctx->stream>>>(npoin, u, divU, vorti, Ml, nq);
-    k_ducros<<<tpe_grid(nelem), 256, 0, ctx->stream>>>(nelem, nnode_of(porder), porder, npoin,
+    k_ducros<<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>(nelem, nnode_of(porder), porder, npoin,
                                                        connec, m->perm, nq, helem, ducros_min_val,
                                                        mu_e);
     prof_end(ctx, tok);
