@@ -271,28 +271,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             if constexpr (!CONS) x.musgs = A.mu_sgs ? A.mu_sgs[eg] : T(0);
         }
     };
-    // the dense residual records of unit u (in `area`) to its block of A.out:
-    // read into registers, then stored SB contiguous bytes per lane
-    constexpr int SB = gcd16(RW * NL * (int)sizeof(T)), CH = RW * NL * (int)sizeof(T) / SB,
-                  NC = (CH + NT - 1) / NT;
-    using U4 = unsigned __attribute__((ext_vector_type(4)));
-    using U2 = unsigned __attribute__((ext_vector_type(2)));
-    using SV = std::conditional_t<SB == 16, U4, std::conditional_t<SB == 8, U2, unsigned>>;
-    auto rec_read = [&](SV v[NC]) {
-#pragma unroll
-        for (int i = 0; i < NC; ++i) v[i] = ((const SV *)area)[min(lane + i * NT, CH - 1)];
-    };
-    auto rec_store = [&](const SV v[NC], int u) {
-        SV *o = (SV *)(A.out + (size_t)u * RW * NL);
-        if (NE == 1 || (u + 1) * NE <= A.nelem) {
-#pragma unroll
-            for (int i = 0; i < NC; ++i)
-                if (lane + i * NT < CH) o[lane + i * NT] = v[i];
-        } else { // the odd last element of a unit of two
-            const T *s = area;
-            for (int i = lane; i < RW * NN; i += NT) ((T *)o)[i] = s[i];
-        }
-    };
+    using O = RecOut<P, T, RW>; // residual records
 
     In cur, nxt;
     GeoAt at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, unit(er.begin), geo_at, wl, wv);
@@ -317,10 +296,10 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 for (int i = 0; i < 3; ++i) He[i][j] = hp[i + 3 * j];
         }
         const T vol = ((const T *)(geo + Q::HEA + at.gv))[ln.sub * NN + ln.a];
-        SV out[NC];
-        rec_read(out);
+        typename O::V out[O::NC];
+        O::read(out, area, lane);
         lds_done();
-        if (prev >= 0) rec_store(out, prev);
+        if (prev >= 0) O::store(out, area, A.out, prev, A.nelem, lane);
         load(nxt, u2, slot);
         int pn[L::PJ ? L::PI : 1];
         if constexpr (L::PJ) {
@@ -732,176 +711,208 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         cur = nxt;
     }
     lds_barrier();
-    SV out[NC];
-    rec_read(out);
-    if (prev >= 0) rec_store(out, prev);
+    typename O::V out[O::NC];
+    O::read(out, area, lane);
+    if (prev >= 0) O::store(out, area, A.out, prev, A.nelem, lane);
     // no copy may still be writing this block's LDS when it retires
     wait_vm<0>();
 }
 
-// generic_scalar_convec_ijk (elem_convec.f90:472-594):
-// Re = gpvol [ 1/2 (div f + eta div u) + 1/2 u.grad(eta) ]
-// FUSEF: the flux is f = u * eta, formed in registers instead of read (the
-// time loop's f_eta = u(:,:,1) * eta(:,1) of the same two arrays)
-template <int P, typename T, bool FUSEF>
-__global__ __launch_bounds__(EG<P>::NT) void k_scalar_convec(RhsArgs<T> A, const T *__restrict__ f,
-                                                             const T *__restrict__ eta)
+// The first-derivative operators on the element pipeline, by OP:
+//   SFUSED, SFLUX  generic_scalar_convec_ijk (elem_convec.f90:472-594):
+//     gpvol [ 1/2 (div f + eta div u) + 1/2 u.grad(eta) ], with f = u eta formed in
+//     registers (the time loop's f_eta = u(:,:,1) * eta(:,1) of the same two arrays)
+//     or read;
+//   DIV, CURL, DIVCURL  eval_divergence (mod_operators.f90:485-570) and
+//     compute_vorticity (mod_operators.f90:684-775) at each GLL point.  With g_ik =
+//     du_i/dxi_k the line derivatives and grad u(i,j) = sum_k He(j,k) g_ik: gpvol *
+//     div u, and eps_ijk du_j/dx_k (the reference's leviCivi sum, minus the curl).
+// Records of RW values per element-node at e*NN + perm[a].
+//
+// What bounds it: memory.  The 80 bytes of geometry per element-node are most of
+// what is read; copied through LDS they are read once and in order, where each lane
+// read its own 72 bytes of He at a stride of 72 (MEASURED).
+enum class GradOp { SFUSED, SFLUX, DIV, CURL, DIVCURL };
+
+// waves per SIMD asked of the compiler: as many as run without spilling
+template <int P, typename T, GradOp OP> constexpr int grad_waves()
 {
-    constexpr int NN = EG<P>::NN, NT = EG<P>::NT;
-    __shared__ T s[7 * NT]; // eta, u(3), f(3)
-    const int lane = threadIdx.x;
-    const bool act = lane < NN;
-    const int a = act ? lane : 0;
-    LineTab<P, T> lt;
-    build_linetab<P, T>(a, A.dl, A.inv, A.gI, A.gJ, A.gK, lt);
-    const int pa = min(max(A.perm[a], 0), NN - 1);
-    struct In {
-        T et, u[3], fv[3], He[9], vol;
+    return sizeof(T) == 8 && (P == 4 || OP == GradOp::SFLUX) ? 3 : 4;
+}
+
+template <int P, typename T, GradOp OP>
+__global__ __launch_bounds__((EP<P, T>::NTB), (grad_waves<P, T, OP>())) void k_grad(RhsArgs<T> A, const T *__restrict__ f,
+                                                            const T *__restrict__ eta)
+{
+    using Q = EP<P, T>;
+    using V2 = T __attribute__((ext_vector_type(2)));
+    constexpr bool SC = OP == GradOp::SFUSED || OP == GradOp::SFLUX, FLUX = OP == GradOp::SFLUX;
+    constexpr bool DIV = OP == GradOp::DIV || OP == GradOp::DIVCURL,
+                   CURL = OP == GradOp::CURL || OP == GradOp::DIVCURL;
+    constexpr int NN = Q::NN, NL = Q::NL, NT = Q::NT, NE = Q::NE, NW = Q::NW, G = Q::G;
+    constexpr int RW = SC ? 1 : (DIV ? 1 : 0) + (CURL ? 3 : 0);
+    // nodal records u1 u2 | u3 eta | f1 f2 | f3 -, at a stride of an odd number of
+    // pairs, so that 16 consecutive records start in 16 different banks
+    constexpr int REC = FLUX ? 10 : 6;
+    __shared__ __attribute__((aligned(16))) T area_s[G * REC * NT];
+    __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * Q::GEO];
+    __shared__ int conn_s[G * 2 * NT];
+    const int sb = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    T *const area = area_s + sb * REC * NT;
+    unsigned char *const geo = geo_s + sb * Q::GEO;
+    int *const conn = conn_s + sb * 2 * NT;
+    const unsigned geo_at = lds_addr(geo_s) + sb * Q::GEO;
+    const unsigned conn_at = lds_addr(conn_s) + sb * 2 * NT * 4;
+    const int lane = threadIdx.x % NT, wl = lane & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(lane >> 6);
+
+    const int nunits = (A.nelem + NE - 1) / NE;
+    const UnitRange er = unit_range((nunits + G - 1) / G, A.run, A.wide);
+    auto unit = [&](int g) { return min(g * G + sb, nunits - 1); };
+    if (er.begin >= er.end) return;
+    const int ulast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
+    const LexLane<P, T, false> ln(lane, A.dl, A.inv, A.perm);
+    const size_t EN = (size_t)A.nelem * NN, np = (size_t)A.npoin;
+    auto conn_issue = [&](int u, int slot) {
+        const size_t i = (size_t)u * NL + lane;
+        dma_lds<4>(A.connecT + (i < EN ? i : EN - 1), conn_at + (slot * NT + wv * 64) * 4);
     };
-    auto load = [&](In &x, int e) {
-        const size_t ea = (size_t)e * NN + a;
-        const int n = act ? A.connecT[ea] : 0;
-        x.et = eta[n];
+    struct In {
+        T et, u[3], fv[3];
+    };
+    auto load = [&](In &x, int slot) {
+        const int n = conn[slot * NT + ln.sub * NN + ln.a];
+        if constexpr (SC) x.et = eta[n];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            x.u[d] = A.u[n + (size_t)A.npoin * d];
-            x.fv[d] = FUSEF ? x.u[d] * x.et : f[n + (size_t)A.npoin * d];
+            x.u[d] = A.u[n + np * d];
+            if constexpr (FLUX) x.fv[d] = f[n + np * d];
         }
-        const T *hp = A.He + 9 * ea;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) x.He[i] = hp[i];
-        x.vol = A.gpvol[ea];
     };
-    const ElemRange er = elem_range(A.nelem);
-    if (er.begin >= er.end) return;
-    const int elast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
+    using O = RecOut<P, T, RW>;
+
     In cur, nxt;
-    load(cur, er.begin);
-    for (int e = er.begin; e < er.end; e += er.stride) {
-        load(nxt, min(e + er.stride, elast));
-        if (act) {
-            s[a] = cur.et;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                s[(1 + d) * NT + a] = cur.u[d];
-                s[(4 + d) * NT + a] = cur.fv[d];
-            }
-        }
+    GeoAt at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, unit(er.begin), geo_at, wl, wv);
+    conn_issue(unit(er.begin), 0);
+    conn_issue(unit(min(er.begin + er.stride, ulast)), 1);
+    wait_vm<0>();
+    lds_barrier();
+    load(cur, 0);
+    int slot = 1, prev = -1;
+    for (int g = er.begin; g < er.end; g += er.stride, slot ^= 1) {
+        const int u = unit(g), u2 = unit(min(g + er.stride, ulast)),
+                  u3 = unit(min(g + 2 * er.stride, ulast));
+        wait_vm<0>();
         lds_barrier();
-        T gE[3] = {0, 0, 0}, divU = 0, divF = 0;
+        T He[3][3];
+        {
+            const T *hp = (const T *)(geo + at.he) + 9 * (ln.sub * NN + ln.a);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) He[i][j] = hp[i + 3 * j];
+        }
+        const T vol = ((const T *)(geo + Q::HEA + at.gv))[ln.sub * NN + ln.a];
+        typename O::V out[O::NC];
+        O::read(out, area, lane);
+        lds_done();
+        if (prev >= 0) O::store(out, area, A.out, prev, A.nelem, lane);
+        load(nxt, slot);
+        unit_sync<NW>();
+        at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
+        conn_issue(u3, slot ^ 1);
+        prev = g * G + sb < nunits ? u : -1;
+
+        const T *v = cur.u;
+        T fo[3] = {0, 0, 0};
+        if constexpr (SC)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) fo[d] = FLUX ? cur.fv[d] : v[d] * cur.et;
+        const int own = lane * REC;
+        *(V2 *)(area + own) = V2{v[0], v[1]};
+        *(V2 *)(area + own + 2) = V2{v[2], SC ? cur.et : T(0)};
+        if constexpr (FLUX) {
+            *(V2 *)(area + own + 4) = V2{fo[0], fo[1]};
+            area[own + 6] = fo[2];
+        }
+        unit_sync<NW>();
+
+        // multiply-adds by name: SFUSED and SFLUX give the same bits whichever of two
+        // products the compiler would contract
+        T gE[3] = {0, 0, 0}, divU = 0, divF = 0, gu[3][3] = {}; // gu[i][j] = du_i/dx_j
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const T c0 = lt.ds[k];
-            T de = c0 * cur.et, du[3], df[3];
+            const T c0 = ln.ds[k];
+            T de = SC ? c0 * cur.et : T(0), du[3], df[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                du[d] = c0 * cur.u[d];
-                df[d] = c0 * cur.fv[d];
+                du[d] = c0 * v[d];
+                df[d] = c0 * fo[d];
             }
 #pragma unroll
             for (int o = 0; o < P; ++o) {
-                const int b = lt.off[k][o];
-                const T c = lt.d[k][o];
-                de += c * s[b];
+                const T *b = area + ln.nb[k][o] * REC;
+                const T c = ln.d[k][o];
+                const V2 x01 = *(const V2 *)b, x2e = *(const V2 *)(b + 2);
+                const T x[3] = {x01.x, x01.y, x2e.x};
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    du[d] += c * s[(1 + d) * NT + b];
-                    df[d] += c * s[(4 + d) * NT + b];
+                for (int d = 0; d < 3; ++d) du[d] = fma(c, x[d], du[d]);
+                if constexpr (SC) {
+                    de = fma(c, x2e.y, de);
+                    T y[3];
+                    if constexpr (FLUX) {
+                        const V2 f01 = *(const V2 *)(b + 4);
+                        y[0] = f01.x;
+                        y[1] = f01.y;
+                        y[2] = b[6];
+                    } else {
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) y[d] = x[d] * x2e.y;
+                    }
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) df[d] = fma(c, y[d], df[d]);
                 }
             }
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                const T h = cur.He[i + 3 * k]; // He(i,k)
-                gE[i] += h * de;
-                divU += h * du[i];
-                divF += h * df[i];
+                if constexpr (SC) {
+                    gE[i] = fma(He[i][k], de, gE[i]);
+                    divU = fma(He[i][k], du[i], divU);
+                    divF = fma(He[i][k], df[i], divF);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) gu[i][j] += He[j][k] * du[i];
+                }
             }
         }
-        T r = T(0.5) * (divF + cur.et * divU);
+        T r[RW];
+        if constexpr (SC) {
+            T t = T(0.5) * fma(cur.et, divU, divF);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) r += T(0.5) * (cur.u[i] * gE[i]);
-        if (act) A.out[(size_t)e * NN + pa] = cur.vol * r;
-        cur = nxt;
-        lds_barrier();
-    }
-}
-
-// eval_divergence (mod_operators.f90:485-570) and compute_vorticity
-// (mod_operators.f90:684-775) at each GLL point.  With g_ik = du_i/dxi_k the
-// line derivatives and grad u(i,j) = sum_k He(j,k) g_ik: the divergence record
-// is gpvol * div u, the vorticity record eps_ijk du_j/dx_k (the reference's
-// leviCivi sum, minus the curl).  Records of DIV + 3 CURL values per
-// element-node at e*NN + perm[a].
-template <int P, typename T, bool DIV, bool CURL>
-__global__ __launch_bounds__(EG<P>::NT) void k_div_curl(RhsArgs<T> A)
-{
-    constexpr int NN = EG<P>::NN, NT = EG<P>::NT, NF = (DIV ? 1 : 0) + (CURL ? 3 : 0);
-    __shared__ T s[3 * NT]; // u(3)
-    const int lane = threadIdx.x;
-    const bool act = lane < NN;
-    const int a = act ? lane : 0;
-    LineTab<P, T> lt;
-    build_linetab<P, T>(a, A.dl, A.inv, A.gI, A.gJ, A.gK, lt);
-    const int pa = min(max(A.perm[a], 0), NN - 1);
-    struct In {
-        T u[3], He[9], vol;
-    };
-    auto load = [&](In &x, int e) {
-        const size_t ea = (size_t)e * NN + a;
-        const int n = act ? A.connecT[ea] : 0;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) x.u[d] = A.u[n + (size_t)A.npoin * d];
-        const T *hp = A.He + 9 * ea;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) x.He[i] = hp[i];
-        x.vol = DIV ? A.gpvol[ea] : T(0);
-    };
-    const ElemRange er = elem_range(A.nelem);
-    if (er.begin >= er.end) return;
-    const int elast = er.begin + (er.end - 1 - er.begin) / er.stride * er.stride;
-    In cur, nxt;
-    load(cur, er.begin);
-    for (int e = er.begin; e < er.end; e += er.stride) {
-        load(nxt, min(e + er.stride, elast));
-        if (act) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) s[d * NT + a] = cur.u[d];
-        }
-        lds_barrier();
-        T g[3][3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const T c0 = lt.ds[k];
-            T du[3] = {c0 * cur.u[0], c0 * cur.u[1], c0 * cur.u[2]};
-#pragma unroll
-            for (int o = 0; o < P; ++o) {
-                const int b = lt.off[k][o];
-                const T c = lt.d[k][o];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) du[d] += c * s[d * NT + b];
-            }
-#pragma unroll
-            for (int d = 0; d < 3; ++d) g[d][k] = du[d];
-        }
-        T gu[3][3]; // gu[i][j] = du_i/dx_j
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                gu[i][j] = cur.He[j] * g[i][0] + cur.He[j + 3] * g[i][1] + cur.He[j + 6] * g[i][2];
-        if (act) {
-            T *o = A.out + NF * ((size_t)e * NN + pa);
-            int f = 0;
-            if constexpr (DIV) o[f++] = cur.vol * (gu[0][0] + gu[1][1] + gu[2][2]);
+            for (int i = 0; i < 3; ++i) t = fma(T(0.5), v[i] * gE[i], t);
+            r[0] = vol * t;
+        } else {
+            int n = 0;
+            if constexpr (DIV) r[n++] = vol * (gu[0][0] + gu[1][1] + gu[2][2]);
             if constexpr (CURL) {
-                o[f++] = gu[1][2] - gu[2][1];
-                o[f++] = gu[2][0] - gu[0][2];
-                o[f++] = gu[0][1] - gu[1][0];
+                r[n++] = gu[1][2] - gu[2][1];
+                r[n++] = gu[2][0] - gu[0][2];
+                r[n++] = gu[0][1] - gu[1][0];
             }
         }
+#pragma unroll
+        for (int i = 0; i < RW; ++i) pin(r[i]);
+        unit_sync<NW>();
+#pragma unroll
+        for (int i = 0; i < RW; ++i) area[ln.rec * RW + i] = r[i];
         cur = nxt;
-        lds_barrier();
     }
+    lds_barrier();
+    typename O::V out[O::NC];
+    O::read(out, area, lane);
+    if (prev >= 0) O::store(out, area, A.out, prev, A.nelem, lane);
+    // no copy may still be writing this block's LDS when it retires
+    wait_vm<0>();
 }
 
 // curlU(n,:) /= lelpn(n) over the working nodes (compute_vorticity's makeConti)
@@ -1160,35 +1171,12 @@ __device__ __forceinline__ void split_read(const unsigned char *sl, int a, int p
 // The two-wave kernel.  The staged nodal fields and the viscous fluxes are
 // node-major records, so one 16-byte LDS read returns two fields of a
 // neighbour and the field offsets are immediates of the read instruction:
-//   node record (12 values): u1 u2 | u3 rho | p H | rhoH q1 | q2 q3 | T -
+//   node record (10 values): u1 u2 | u3 rho | p H | T - | padding
 //   flux record (18 values): for k = 1..3, G_k of (grad rho, grad T, tau u,
 //                            tau_1., tau_2., tau_3.)
-//
-// SPLIT_PAIR: line derivatives D0, D1 and W-weighted line sums DIV0, DIV1 of
-// the field pair at record offset OFF (convection wave).
-#define SPLIT_PAIR(OFF, OWN0, OWN1, D0, D1, DIV0, DIV1)                                    \
-    do {                                                                                   \
-        const T o0_ = (OWN0), o1_ = (OWN1);                                                \
-        DIV0 = 0;                                                                          \
-        DIV1 = 0;                                                                          \
-        _Pragma("unroll") for (int k = 0; k < 3; ++k)                                      \
-        {                                                                                  \
-            T v0 = lt.ds[k] * o0_, v1 = lt.ds[k] * o1_;                                    \
-            T w0 = Wo[k] * o0_, w1 = Wo[k] * o1_;                                          \
-            _Pragma("unroll") for (int o = 0; o < P; ++o)                                  \
-            {                                                                              \
-                const V2 x = LD2(nb[k][o] + (OFF));                                        \
-                v0 += lt.d[k][o] * x.x;                                                    \
-                v1 += lt.d[k][o] * x.y;                                                    \
-                w0 += Wx[k][o] * x.x;                                                      \
-                w1 += Wx[k][o] * x.y;                                                      \
-            }                                                                              \
-            D0[k] = v0;                                                                    \
-            D1[k] = v1;                                                                    \
-            DIV0 += w0;                                                                    \
-            DIV1 += w1;                                                                    \
-        }                                                                                  \
-    } while (0)
+// Both operators are evaluated as k_rhs evaluates them (the FP64 stage's K and z
+// coefficients, the same sums in the same order), so that this assembly and the
+// node-ordered one differ by the order of a surface node's terms only.
 // The block walks element clusters, one after the other; the viscous wave adds each element's residual records into
 // an LDS accumulator per cluster-local node instead of storing them, and after
 // a cluster's last element finishes its interior nodes (mass inverse and
@@ -1200,10 +1188,10 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
     using L = SplitLDS<P, T, G16>;
     static_assert(sizeof(T) == 8 && P == 3, "cluster assembly: FP64, p=3");
     using V2 = T __attribute__((ext_vector_type(2)));
-    // node records of REC values: 112 bytes in FP64, an odd multiple of 16,
-    // so that 16 lanes reading 16 consecutive records with 16-byte reads hit
-    // distinct banks (96-byte records would pair them up); 144-byte flux records
-    constexpr int NN = L::NN, REC = sizeof(T) == 8 ? 14 : 12, GREC = 18, AH = L::AH;
+    // node records of REC values: 80 bytes, an odd multiple of 16, so that 16
+    // lanes reading 16 consecutive records with 16-byte reads hit distinct
+    // banks; 144-byte flux records
+    constexpr int NN = L::NN, REC = 10, GREC = 18, AH = L::AH;
     // s2 holds, in turn: the viscous flux records (GREC values per node) and
     // the handed-over viscous residuals (3 pairs per node), then the dense
     // residual records (RW values per node) followed by the line derivatives
@@ -1332,11 +1320,6 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
     }
     SplitState<P, T> cur;
 
-    // reciprocals of the gas constant and of Pr (one rounding apart from the
-    // divisions of the reference's expressions)
-    const double rRgas = 1.0 / A.Rgas;
-    const T cp_pr = A.Cp / A.Pr;
-    double rinv = 0.0;
     auto prim = [&](const SplitState<P, T> &c, double &r, double ud[3], double &pd, double &hd,
                     double &Td, double &umag) {
         r = c.cr;
@@ -1350,8 +1333,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
         const double eint = c.cE * ri - 0.5 * umag;
         pd = r * (A.gamma - 1.0) * eint;
         hd = (A.gamma / (A.gamma - 1.0)) * pd * ri;
-        Td = pd * ri * rRgas;
-        rinv = ri;
+        Td = pd * ri / A.Rgas;
     };
         // indices are even value offsets into the records
 #define LD1(i) (s1[(i) >> 1].x)
@@ -1387,24 +1369,19 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
             if (t != 0) finish();
             T He[3][3], vol;
             split_read<P, T, G16>(ring + slot_of(t), a, pa, He, vol, cur);
-            T rho, u[3], q[3], H, rhoH;
+            T rho, u[3], p, H;
             {
                 double r, ud[3], pd, hd, Td, umag;
                 prim(cur, r, ud, pd, hd, Td, umag);
                 rho = T(r);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    u[d] = T(ud[d]);
-                    q[d] = T(cur.cq[d]);
-                }
+                for (int d = 0; d < 3; ++d) u[d] = T(ud[d]);
+                p = T(pd - A.p_ref);
                 H = T(hd + 0.5 * umag);
-                rhoH = T(r * (hd + 0.5 * umag));
                 if (act) {
                     s1[(own + 0) >> 1] = V2{u[0], u[1]};
                     s1[(own + 2) >> 1] = V2{u[2], rho};
-                    s1[(own + 4) >> 1] = V2{T(pd - A.p_ref), H};
-                    s1[(own + 6) >> 1] = V2{rhoH, q[0]};
-                    s1[(own + 8) >> 1] = V2{q[1], q[2]};
+                    s1[(own + 4) >> 1] = V2{p, H};
                 }
             }
             lds_barrier(); // B2
@@ -1414,102 +1391,70 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                                           elem_of(t + AH), elem_of(t + 2 * AH), c[ia0], c[ia1], lane);
             }
 
-            T Rm = 0, Rq[3] = {0, 0, 0}, Re = 0;
-            T Ut[3];
+            T Rq[3] = {0, 0, 0}, Re = 0;
+            T Ut[3], divU = 0;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) Ut[k] = He[0][k] * u[0] + He[1][k] * u[1] + He[2][k] * u[2];
-            // velocity and density lines: contravariant line weights W_k(m),
-            // div(u_i u), div u, q_k d/dxi_k u_i and d/dxi_k rho
-            T Wo[3], Wx[3][P];
-            T divUw = 0, drho[3];
-            {
-                T Qt[3], divFuu[3] = {0, 0, 0};
+            for (int k = 0; k < 3; ++k) {
+                Ut[k] = He[0][k] * u[0] + He[1][k] * u[1] + He[2][k] * u[2];
+                divU += lt.ds[k] * Ut[k];
+            }
+            // velocity and density lines: the coefficients K_k(m), the momentum
+            // sums, div u, div q + u.grad rho, and the line derivatives for the
+            // viscous wave
+            const T a0 = divU;
+            T s = T(2) * rho * a0, Kx[3][P];
 #pragma unroll
-                for (int k = 0; k < 3; ++k) Qt[k] = He[0][k] * q[0] + He[1][k] * q[1] + He[2][k] * q[2];
+            for (int k = 0; k < 3; ++k) {
+                const T c0 = lt.ds[k];
+                T du[3], dr = c0 * rho, rq[3] = {0, 0, 0}, dvu = 0, dvq = 0;
 #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const T c0 = lt.ds[k];
-                    T du[3];
+                for (int i = 0; i < 3; ++i) du[i] = c0 * u[i];
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) du[i] = c0 * u[i];
-                    T dr = c0 * rho;
-                    Wo[k] = c0 * Ut[k];
-                    divUw += Wo[k];
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) divFuu[i] += Wo[k] * u[i];
-#pragma unroll
-                    for (int o = 0; o < P; ++o) {
-                        const T c = lt.d[k][o];
-                        const V2 x01 = LD2(nb[k][o] + 0), x2r = LD2(nb[k][o] + 2);
-                        const T ub[3] = {x01.x, x01.y, x2r.x};
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) du[i] += c * ub[i];
-                        dr += c * x2r.y;
-                        const T w = c * (He[0][k] * ub[0] + He[1][k] * ub[1] + He[2][k] * ub[2]);
-                        Wx[k][o] = w;
-                        divUw += w;
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) divFuu[i] += w * ub[i];
-                    }
-                    drho[k] = dr;
-                    s2[DREC + 6 * pa + 2 * k] = V2{du[0], du[1]};
-                    s2[DREC + 6 * pa + 2 * k + 1] = V2{du[2], dr};
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) Rq[i] += Qt[k] * du[i];
+                for (int o = 0; o < P; ++o) {
+                    const T c = lt.d[k][o];
+                    const V2 x01 = LD2(nb[k][o] + 0), x2r = LD2(nb[k][o] + 2);
+                    dr += c * x2r.y;
+                    const T ut = He[0][k] * x01.x + He[1][k] * x01.y + He[2][k] * x2r.x;
+                    const T z = c * (Ut[k] + ut), K = z * (rho + x2r.y);
+                    Kx[k][o] = K;
+                    dvu += c * ut;
+                    dvq += z * x2r.y;
+                    rq[0] += K * x01.x;
+                    rq[1] += K * x01.y;
+                    rq[2] += K * x2r.x;
+                    du[0] += c * x01.x;
+                    du[1] += c * x01.y;
+                    du[2] += c * x2r.x;
                 }
 #pragma unroll
-                for (int i = 0; i < 3; ++i) Rq[i] = T(0.25) * (Rq[i] + rho * divFuu[i]);
+                for (int i = 0; i < 3; ++i) Rq[i] += rq[i];
+                divU += dvu;
+                s += dvq;
+                s2[DREC + 6 * pa + 2 * k] = V2{du[0], du[1]};
+                s2[DREC + 6 * pa + 2 * k + 1] = V2{du[2], dr};
             }
             lds_barrier(); // B3
-            {
-                const T urho = Ut[0] * drho[0] + Ut[1] * drho[1] + Ut[2] * drho[2];
-                Rm += T(0.5) * urho;
+            // pressure gradient and the enthalpy's sum
+            T dp[3];
 #pragma unroll
-                for (int i = 0; i < 3; ++i) Rq[i] += T(0.25) * u[i] * urho;
-                Re += T(0.25) * H * urho;
-            }
-            // field pairs (p, H), (rho H, q1), (q2, q3): line derivative d and
-            // W-weighted line sum div = div(s u) of both fields
-            T divQ = 0;
-            auto grad_i = [&](int i, const T d[3]) { return He[i][0] * d[0] + He[i][1] * d[1] + He[i][2] * d[2]; };
-            auto utd = [&](const T d[3]) { return Ut[0] * d[0] + Ut[1] * d[1] + Ut[2] * d[2]; };
-            {
-                T dp[3], dH[3], dv0, dv1;
-                SPLIT_PAIR(4, LD1(own + 4), H, dp, dH, dv0, dv1);
+            for (int k = 0; k < 3; ++k) {
+                T re = 0;
+                dp[k] = lt.ds[k] * p;
 #pragma unroll
-                for (int i = 0; i < 3; ++i) Rq[i] += grad_i(i, dp);
-                T qt = 0;
+                for (int o = 0; o < P; ++o) {
+                    const V2 x = LD2(nb[k][o] + 4);
+                    re += Kx[k][o] * x.y;
+                    dp[k] += lt.d[k][o] * x.x;
+                }
+                Re += re;
+            }
+            const T B = s + rho * (divU + T(4) * a0);
+            pend[0] = vol * (T(0.5) * (s + rho * divU));
 #pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    qt += (He[0][k] * q[0] + He[1][k] * q[1] + He[2][k] * q[2]) * dH[k];
-                Re += T(0.25) * (qt + rho * dv1);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            {
-                T dRH[3], dq0[3], dv0, dv1;
-                SPLIT_PAIR(6, rhoH, q[0], dRH, dq0, dv0, dv1);
-                Re += T(0.25) * (utd(dRH) + dv0);
-                divQ += grad_i(0, dq0);
-                Rq[0] += T(0.25) * (utd(dq0) + dv1);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            {
-                T dq1[3], dq2[3], dv0, dv1;
-                SPLIT_PAIR(8, q[1], q[2], dq1, dq2, dv0, dv1);
-                divQ += grad_i(1, dq1);
-                Rq[1] += T(0.25) * (utd(dq1) + dv0);
-                divQ += grad_i(2, dq2);
-                Rq[2] += T(0.25) * (utd(dq2) + dv1);
-            }
-            Rm += T(0.5) * (divQ + rho * divUw);
-#pragma unroll
-            for (int i = 0; i < 3; ++i) Rq[i] += T(0.25) * (u[i] * divQ + q[i] * divUw);
-            Re += T(0.25) * (H * divQ + rhoH * divUw);
-            pend[0] = Rm * vol;
-            pend[1] = Rq[0] * vol;
-            pend[2] = Rq[1] * vol;
-            pend[3] = Rq[2] * vol;
-            pend[4] = Re * vol;
+            for (int i = 0; i < 3; ++i)
+                pend[1 + i] = vol * (T(0.25) * (Rq[i] + u[i] * B) +
+                                     (He[i][0] * dp[0] + He[i][1] * dp[1] + He[i][2] * dp[2]));
+            pend[4] = vol * (T(0.25) * (Re + H * B));
         }
         // the last element's records
         lds_barrier();
@@ -1610,7 +1555,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                 Tk = T(Td);
                 const double mfe = A.mu_factor_e ? A.mu_factor_e[elem_of(t)] : A.mu_factor;
                 muf = T(sutherland<double>(mfe, Td));
-                if (act) s1[(own + 10) >> 1] = V2{Tk, T(0)};
+                if (act) s1[(own + 6) >> 1] = V2{Tk, T(0)};
             }
             lds_barrier(); // B2
             // the previous element's records go into the
@@ -1634,7 +1579,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
             for (int k = 0; k < 3; ++k) {
                 T vt = lt.ds[k] * Tk;
 #pragma unroll
-                for (int o = 0; o < P; ++o) vt += lt.d[k][o] * LD1(nb[k][o] + 10);
+                for (int o = 0; o < P; ++o) vt += lt.d[k][o] * LD1(nb[k][o] + 6);
                 dT[k] = vt;
             }
             lds_barrier(); // B3
@@ -1694,26 +1639,27 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                 const int g = pa * GREC;
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    const T c0 = lt.ds[k];
                     const V2 o01 = GL2(g + 6 * k), o23 = GL2(g + 6 * k + 2), o45 = GL2(g + 6 * k + 4);
-                    T v[6] = {c0 * o01.x, c0 * o01.y, c0 * o23.x, c0 * o23.y, c0 * o45.x, c0 * o45.y};
+                    const T own6[6] = {o01.x, o01.y, o23.x, o23.y, o45.x, o45.y};
+#pragma unroll
+                    for (int f = 0; f < 6; ++f) W6[f] += lt.ds[k] * own6[f];
+                }
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
 #pragma unroll
                     for (int o = 0; o < P; ++o) {
                         const T c = tt[k][o];
                         const V2 x01 = GL2(gnb[k][o]), x23 = GL2(gnb[k][o] + 2), x45 = GL2(gnb[k][o] + 4);
-                        v[0] += c * x01.x;
-                        v[1] += c * x01.y;
-                        v[2] += c * x23.x;
-                        v[3] += c * x23.y;
-                        v[4] += c * x45.x;
-                        v[5] += c * x45.y;
+                        W6[0] += c * x01.x;
+                        W6[1] += c * x01.y;
+                        W6[2] += c * x23.x;
+                        W6[3] += c * x23.y;
+                        W6[4] += c * x45.x;
+                        W6[5] += c * x45.y;
                     }
-#pragma unroll
-                    for (int f = 0; f < 6; ++f) W6[f] += v[f];
-                }
             }
-            const T nu_e = A.c_rho * mue * T(rinv);
-            const T kappa = (muf + A.c_ener * mue) * cp_pr;
+            const T nu_e = A.c_rho * mue / rho;
+            const T kappa = muf * A.Cp / A.Pr + A.c_ener * mue * A.Cp / A.Pr;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
@@ -1732,7 +1678,6 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
     // no copy may still be writing this block's LDS when it retires
     wait_vm<0>();
 #undef LD1
-#undef SPLIT_PAIR
 #undef LD2
 #undef GL2
 }
@@ -2120,6 +2065,16 @@ template int rhs_fused_elements<float>(sodhip_ctx, int, const MeshCache *, const
                                        double, double, const double *, double, double, double,
                                        float *);
 
+template <int P, typename T, GradOp OP>
+static void launch_grad_p(sodhip_ctx ctx, RhsArgs<T> A, const T *f = nullptr, const T *eta = nullptr)
+{
+    const UnitShape us = unit_shape<P, T>(ctx, A.nelem);
+    A.run = us.run;
+    A.wide = us.wide;
+    A.geo16 = ((uintptr_t)A.He % 16 == 0) && ((uintptr_t)A.gpvol % 16 == 0);
+    k_grad<P, T, OP><<<us.grid, EP<P, T>::NTB, 0, ctx->stream>>>(A, f, eta);
+}
+
 template <typename T>
 static int scalar_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const int *connec,
                          const T *He, const T *gpvol, const T *dl, const int *inv, const int *gI,
@@ -2150,13 +2105,12 @@ static int scalar_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const
     A.gK = gK;
     A.u = u;
     A.out = (T *)ctx->scratch.ptr;
-    const int grid = elem_grid(ctx, nelem, 128);
     int tok = prof_begin(ctx, 3);
-#define SODHIP_SC(PP)                                                                       \
-    if (q)                                                                                  \
-        k_scalar_convec<PP, T, false><<<grid, EG<PP>::NT, 0, ctx->stream>>>(A, q, eta);     \
-    else                                                                                    \
-        k_scalar_convec<PP, T, true><<<grid, EG<PP>::NT, 0, ctx->stream>>>(A, q, eta);
+#define SODHIP_SC(PP)                                              \
+    if (q)                                                         \
+        launch_grad_p<PP, T, GradOp::SFLUX>(ctx, A, q, eta);       \
+    else                                                           \
+        launch_grad_p<PP, T, GradOp::SFUSED>(ctx, A, q, eta);
     switch (porder) {
     case 2: SODHIP_SC(2) break;
     case 3: SODHIP_SC(3) break;
@@ -2211,7 +2165,7 @@ static int div_curl(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
-    A.gpvol = gpvol;
+    A.gpvol = gpvol ? gpvol : He; // not used by the vorticity
     A.dl = dl;
     A.inv = inv;
     A.gI = gI;
@@ -2219,21 +2173,17 @@ static int div_curl(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
     A.gK = gK;
     A.u = u;
     A.out = (T *)ctx->scratch.ptr;
-    const int grid = elem_grid(ctx, nelem, 128);
     int tok = prof_begin(ctx, 3);
-#define SODHIP_DC(PP, DV, CU) \
-    k_div_curl<PP, T, DV, CU><<<grid, EG<PP>::NT, 0, ctx->stream>>>(A)
-#define SODHIP_DC_P(PP)                                                        \
-    if (divU && curlU) SODHIP_DC(PP, true, true);                              \
-    else if (divU) SODHIP_DC(PP, true, false);                                 \
-    else SODHIP_DC(PP, false, true);
+#define SODHIP_DC_P(PP)                                                       \
+    if (divU && curlU) launch_grad_p<PP, T, GradOp::DIVCURL>(ctx, A);         \
+    else if (divU) launch_grad_p<PP, T, GradOp::DIV>(ctx, A);                 \
+    else launch_grad_p<PP, T, GradOp::CURL>(ctx, A);
     switch (porder) {
     case 2: SODHIP_DC_P(2) break;
     case 3: SODHIP_DC_P(3) break;
     case 4: SODHIP_DC_P(4) break;
     }
 #undef SODHIP_DC_P
-#undef SODHIP_DC
     SODHIP_TRY_HIP(hipGetLastError());
     T *c0 = curlU, *c1 = curlU ? curlU + npoin : nullptr, *c2 = curlU ? curlU + 2 * (size_t)npoin : nullptr;
     if (divU && curlU)

@@ -217,4 +217,33 @@ template <int P, typename T, bool TRANS> struct LexLane {
     }
 };
 
+// A unit's records of RW values per node, written to LDS densely in the record order
+// (LexLane::rec), go to out (elements back to back) as whole vectors: read into
+// registers, then stored SB contiguous bytes per lane.
+template <int P, typename T, int RW> struct RecOut {
+    using Q = EP<P, T>;
+    static constexpr int SB = gcd16(RW * Q::NL * (int)sizeof(T)), CH = RW * Q::NL * (int)sizeof(T) / SB,
+                         NC = (CH + Q::NT - 1) / Q::NT;
+    using U4 = unsigned __attribute__((ext_vector_type(4)));
+    using U2 = unsigned __attribute__((ext_vector_type(2)));
+    using V = std::conditional_t<SB == 16, U4, std::conditional_t<SB == 8, U2, unsigned>>;
+    static __device__ __forceinline__ void read(V (&v)[NC], const T *area, int lane)
+    {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[i] = ((const V *)area)[min(lane + i * Q::NT, CH - 1)];
+    }
+    static __device__ __forceinline__ void store(const V (&v)[NC], const T *area, T *out, int u,
+                                                 int nelem, int lane)
+    {
+        V *o = (V *)(out + (size_t)u * RW * Q::NL);
+        if (Q::NE == 1 || (u + 1) * Q::NE <= nelem) {
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                if (lane + i * Q::NT < CH) o[lane + i * Q::NT] = v[i];
+        } else { // the odd last element of a unit of two
+            for (int i = lane; i < RW * Q::NN; i += Q::NT) ((T *)o)[i] = area[i];
+        }
+    }
+};
+
 } // namespace sodhip

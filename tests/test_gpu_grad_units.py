@@ -1,0 +1,90 @@
+"""Entropy convection, divergence and vorticity at the edges of their kernel's units:
+element counts that leave the last unit or group of units partly empty, and geometry
+arrays that do not start on a 16-byte boundary, against the oracle.
+
+Tolerances: FP64 sums of about 9 (p+1) products with relative error 2^-53 each stay
+below 1e-13 of the result's 2-norm; FP32 (2^-24) below 2e-5."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import make_case, relerr
+
+pytestmark = pytest.mark.gpu
+
+# element counts 1, 2, 5, 7 (units of two, groups of two and four) and 63
+BOXES = [(1, 1, 1), (2, 1, 1), (5, 1, 1), (7, 1, 1), (7, 3, 3)]
+
+
+def _shifted(x, elems):
+    """A device copy of x that starts `elems` values past an allocation's start."""
+    import torch
+    buf = torch.zeros(x.numel() + elems + 8, dtype=x.dtype, device="cuda")
+    out = buf[elems:elems + x.numel()]
+    out.copy_(x)
+    return out
+
+
+@pytest.mark.parametrize("p", [2, 3, 4])
+@pytest.mark.parametrize("box", BOXES)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gradient_operators_at_unit_edges(p, box, shift):
+    import torch
+    from oracle import oracle as O
+    from sod2d_amd import case, device as D
+    from sod2d_amd._lib import check, lib
+
+    g = make_case(p, box, periodic=False, jitter=0.05, lengths=(1.0, 1.1, 0.9))
+    m, T = g.mesh, g.tables
+    n = m.npoin
+    rng = np.random.default_rng(60 + p)
+    u = np.asfortranarray(rng.normal(0, 0.3, (n, 3)))
+    eta = rng.normal(size=n)
+    f = np.asfortranarray(rng.normal(size=(n, 3)))
+    lelpn = case.elem_per_node(m.connec, n)
+    up = D.to_dev
+    He, gv = _shifted(up(g.He), shift), _shifted(up(g.gpvol), shift)
+    dl, connec, lw, le = up(T.dlxigp_ip), up(m.connec), up(m.lpoin_w), up(lelpn)
+    tabs = [up(x) for x in (T.invAtoIJK, T.gmshAtoI, T.gmshAtoJ, T.gmshAtoK)]
+    du, de, df = up(u), up(eta), up(f)
+    out = lambda k: torch.full((k * n,), 7.0, dtype=torch.float64, device="cuda")  # noqa: E731
+    R, R0, div, curl, div2, curl2 = out(1), out(1), out(1), out(3), out(1), out(3)
+    scal = (m.nelem, n, connec, None, None, He, gv, dl, None, *tabs)
+    D.generic_scalar_convec_ijk(*scal, df, de, du, R, True, -1.0)
+    D.generic_scalar_convec_ijk(*scal, None, de, du, R0, True, -1.0)
+    D.eval_divergence(m.nelem, n, connec, He, gv, dl, *tabs, du, div)
+    D.compute_vorticity(m.nelem, n, m.npoin_w, lw, connec, le, He, dl, *tabs, du, curl)
+    D.div_curl(m.nelem, n, m.npoin_w, lw, connec, le, He, gv, dl, *tabs, du, div2, curl2)
+
+    # FP32: the entry point of the C interface
+    f32 = torch.float32
+    He4, gv4 = _shifted(up(g.He).to(f32), shift), _shifted(up(g.gpvol).to(f32), shift)
+    s4 = [x.to(f32).contiguous() for x in (dl, df, de, du)]
+    R4 = torch.full((n,), 7.0, dtype=f32, device="cuda")
+    ctx = D.Context(0)
+    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    torch.cuda.synchronize()
+    check(lib().sodhip_generic_scalar_convec_ijk_f32(
+        ctx.h, p, m.nelem, n, ptr(connec), ptr(He4), ptr(gv4), ptr(s4[0]), *map(ptr, tabs),
+        ptr(s4[1]), ptr(s4[2]), ptr(s4[3]), ptr(R4), 1, C.c_float(-1.0)), "scalar_convec_f32")
+    torch.cuda.synchronize()
+
+    OT = O.Tables(p)
+    w = m.lpoin_w - 1
+    fo = lambda a: np.asarray(a).ravel(order="F")  # noqa: E731
+    ref = O.generic_scalar_convec_ijk(OT, m.connec, g.He, g.gpvol, f, eta, u, None, True, -1.0)
+    ref0 = O.generic_scalar_convec_ijk(OT, m.connec, g.He, g.gpvol,
+                                       np.asfortranarray(u * eta[:, None]), eta, u, None, True, -1.0)
+    odiv = O.eval_divergence(OT, m.connec, g.He, g.gpvol, u)
+    ocurl = O.compute_vorticity(OT, m.connec, m.lpoin_w, lelpn, g.He, u)
+    assert relerr(R.cpu().numpy(), ref) < 1e-13
+    assert relerr(R0.cpu().numpy(), ref0) < 1e-13
+    assert relerr(div.cpu().numpy(), odiv) < 1e-13
+    got = curl.cpu().numpy().reshape(3, n).T
+    assert relerr(fo(got[w]), fo(ocurl[w])) < 1e-13
+    assert torch.equal(div, div2) and torch.equal(curl, curl2)
+    r = lambda a: np.asfortranarray(np.asarray(a, dtype=np.float32).astype(np.float64))  # noqa: E731
+    ref4 = O.generic_scalar_convec_ijk(OT, m.connec, r(g.He), r(g.gpvol), r(f), r(eta), r(u), None,
+                                       True, -1.0)
+    assert relerr(R4.cpu().numpy(), ref4) < 2e-5
