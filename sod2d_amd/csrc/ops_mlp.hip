@@ -613,26 +613,25 @@ __global__ __launch_bounds__(256, 2) void k_surrogate(SurArgs A)
 }
 
 // smart_visc_spectral (the plain sensor, p = 3) on the listed elements, one
-// wave per element; the same arithmetic as k_smart_visc_ch.  With nfall set,
+// wave per element; the same arithmetic as k_smart_visc.  With nfall set,
 // block 0 also copies the count there.
 __global__ __launch_bounds__(64) void k_smart_visc_list(SensorArgs A, const int *__restrict__ list,
                                                         int *__restrict__ nfall)
 {
     constexpr int P = 3, NN = 64;
-    __shared__ double ml[NN];
-    const int a = threadIdx.x;
+    __shared__ double buf[3][NN];
+    const int at = threadIdx.x; // node in line order
     const int cnt = list[0];
-    if (nfall && blockIdx.x == 0 && a == 0) *nfall = cnt;
+    if (nfall && blockIdx.x == 0 && at == 0) *nfall = cnt;
     if ((int)blockIdx.x >= cnt) return;
-    int src[27];
-    filter_sources<P>(a, A.inv, src);
+    const int a = min(max(A.inv[at] - 1, 0), NN - 1);
+    const FilterLane<P> fl(at);
     double norm = 1.0;
     if (A.pmax) {
         norm = 0.0;
-        for (int i = a; i < A.nparts; i += 64) norm = fmax(norm, A.pmax[i]);
+        for (int i = at; i < A.nparts; i += 64) norm = fmax(norm, A.pmax[i]);
         norm = wmax(norm);
     }
-    const double w[3] = {0.25, 0.5, 0.25};
     for (int i = blockIdx.x; i < cnt; i += gridDim.x) {
         const int e = list[1 + i];
         const int n = A.connecT[(size_t)e * NN + a];
@@ -644,15 +643,13 @@ __global__ __launch_bounds__(64) void k_smart_visc_list(SensorArgs A, const int 
         const double R1 = rho * fabs(A.Reta[n]) / norm;
         const double h = A.helem[e + (size_t)A.nelem * a];
         const double v = A.cglob * fmin(A.ce * R1 * (h * h), be);
-        ml[a] = v;
-        __syncthreads();
-        double acc = 0.0;
+        double acc = v;
 #pragma unroll
-        for (int l = 0; l < 3; ++l)
-#pragma unroll
-            for (int m = 0; m < 3; ++m)
-#pragma unroll
-                for (int nn = 0; nn < 3; ++nn) acc += w[l] * w[m] * w[nn] * ml[src[9 * l + 3 * m + nn]];
+        for (int k = 0; k < 3; ++k) {
+            buf[k][at] = acc;
+            __syncthreads();
+            acc = filter_line(buf[k][fl.n[k][0]], acc, buf[k][fl.n[k][1]]);
+        }
         const size_t g = e + (size_t)A.nelem * a;
         A.mue_l[g] = v;
         A.mu_e[g] = acc;

@@ -14,6 +14,7 @@
 
 #include "common.hpp"
 #include "device.hpp"
+#include "pipe.hpp"
 #include "sensor.hpp"
 
 namespace sodhip {
@@ -365,110 +366,160 @@ __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder
     }
 }
 
-// Chunked variant: the workgroup (NT = roundup((p+1)^3, 64) lanes, one or two
-// waves) walks CH consecutive elements at a time so that the element-fastest
-// arrays helem(nelem,nnode), mue_l and mu_e move as whole 128-byte lines: the
-// CH x NN block is read and written through LDS with thread t holding (node
-// t/CH, element t%CH), while the per-element arithmetic keeps lane = node.
-template <int P, int CH, typename S = double>
-__global__ __launch_bounds__(SG<P>::NT) void k_smart_visc_ch(SensorArgsT<S> A)
+// max over each row of 16 lanes, by DPP rotations
+__device__ __forceinline__ double row_max(double v)
 {
-    constexpr int N1 = SG<P>::N1, NN = SG<P>::NN, NT = SG<P>::NT, NW = NT / 64;
-    constexpr int BLK = CH * NN, ROWS = (BLK + NT - 1) / NT;
-    __shared__ double lb[BLK]; // helem, then mue_l, of the chunk: [c][a]
-    __shared__ double ob[BLK]; // mu_e of the chunk
-    __shared__ double wmax[NW];
-    const int lane = threadIdx.x, wl = lane & 63, wv = lane >> 6;
-    const bool act = lane < NN;
-    const int a = act ? lane : 0;
+    auto ror = [](double x, auto n) {
+        constexpr int ctrl = 0x120 + decltype(n)::value;
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), ctrl, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), ctrl, 0xf, 0xf, false);
+        return __hiloint2double(hi, lo);
+    };
+    v = fmax(v, ror(v, std::integral_constant<int, 8>{}));
+    v = fmax(v, ror(v, std::integral_constant<int, 4>{}));
+    v = fmax(v, ror(v, std::integral_constant<int, 2>{}));
+    return fmax(v, ror(v, std::integral_constant<int, 1>{}));
+}
+// ... and over the wave
+__device__ __forceinline__ double wave_max(double v)
+{
+    v = row_max(v);
+    v = fmax(v, __shfl_xor(v, 16, 64));
+    return fmax(v, __shfl_xor(v, 32, 64));
+}
+
+// smart_visc_spectral over chunks of CH = 16 consecutive elements, so that the
+// element-fastest arrays helem(nelem,nnode), mue_l and mu_e move as whole 128-byte
+// lines through LDS (thread t holds node t/CH of element t%CH).  In between, lanes
+// hold nodes in line order (I fastest), as the operators' kernels do: a gather then
+// touches a quarter of the cache lines that it touches in gmsh order.  Groups of NT
+// lanes (one wave; two at p=4) take NE elements at a time (two at p=2), and every
+// group's share of the chunk, E rounds, is in flight at once.
+//
+// What bounds it: waits on L2 for the gathers of six node fields (the vector memory
+// units stall on lines in flight 0.7 of the time, whatever the occupancy).  48 bytes
+// per element-node and the node fields once would take 145 us of a large copy's rate at
+// 262k elements, p=3; it takes 284 us, 404 with one wave per chunk in gmsh order, which
+// also read the filter's 27 sources one by one and rows of 64 doubles whose 16
+// elements share a bank pair.  48k elements, p=4: 167 -> 131 us; 152k, p=2: 155 -> 68 us;
+// 512 elements, p=3 (32 waves): 28 -> 8.5 us.  The filter is three line passes of two
+// LDS reads, and rows are padded to an odd number of doubles.
+template <int P> struct SensorShape {
+    static constexpr int NN = SG<P>::NN, NT = SG<P>::NT, NW = NT / 64, CH = 16;
+    static constexpr int NE = P == 2 ? 2 : 1, G = 4, NTB = G * NT; // groups, threads
+    static constexpr int E = CH / (G * NE), ROW = NN | 1;
+};
+
+template <int P, typename S>
+__global__ __launch_bounds__(SensorShape<P>::NTB, 4) void k_smart_visc(SensorArgsT<S> A)
+{
+    using Q = SensorShape<P>;
+    constexpr int NN = Q::NN, NT = Q::NT, NW = Q::NW, CH = Q::CH, NE = Q::NE, E = Q::E, ROW = Q::ROW;
+    constexpr int BLK = CH * NN, ROWS = (BLK + Q::NTB - 1) / Q::NTB;
+    __shared__ double lb[CH * ROW], ob[CH * ROW];
+    __shared__ double wmax[NW > 1 ? Q::G * NW * E : 1];
+    const int grp = threadIdx.x / NT, lane = threadIdx.x % NT, wl = threadIdx.x & 63;
+    const bool act = lane < NE * NN;
+    const int sub = act ? lane / NN : 0, at = act ? lane - sub * NN : 0;
+    const int a = min(max(A.inv[at] - 1, 0), NN - 1);
+    const FilterLane<P> fl(at);
     double norm = 1.0;
     if (A.pmax) { // every wave folds all partial maxima itself
         norm = 0.0;
         for (int i = wl; i < A.nparts; i += 64) norm = fmax(norm, A.pmax[i]);
-#pragma unroll
-        for (int s = 32; s > 0; s >>= 1) norm = fmax(norm, __shfl_xor(norm, s, 64));
+        norm = wave_max(norm);
     }
-    int src[27];
-    filter_sources<P>(a, A.inv, src);
-    const double w[3] = {0.25, 0.5, 0.25};
-    // XCD-aware: the blocks of one XCD walk chunks of one contiguous eighth
-    const int per = gridDim.x >> 3, xcd = blockIdx.x & 7, rk = blockIdx.x >> 3;
-    const int span = (A.nelem + 7) >> 3;
-    const int xb = xcd * span, xe = min(A.nelem, xb + span);
-    const int nch = xe > xb ? (xe - xb + CH - 1) / CH : 0;
-    if (rk >= nch) return;
-    struct In {
-        double u0, u1, u2, T, rho, Reta, hk;
-    };
-    auto load = [&](In &x, int e) {
-        const int n = act ? A.connecT[(size_t)e * NN + a] : 0;
-        x.u0 = A.u[n];
-        x.u1 = A.u[n + A.npoin];
-        x.u2 = A.u[n + 2 * (size_t)A.npoin];
-        x.T = A.Tem[n];
-        x.rho = A.rho[n];
-        x.Reta = A.Reta[n];
-        x.hk = A.helem_k[e];
-    };
-    In cur, nxt;
-    load(cur, xb + rk * CH);
-    for (int ci = rk; ci < nch; ci += per) {
-        const int c0 = xb + ci * CH, cn = min(CH, xe - c0);
-        const int cnext = ci + per < nch ? xb + (ci + per) * CH : c0 + cn - 1;
-        // helem of the chunk, whole lines (elements past the range re-read the last)
+    const size_t np = (size_t)A.npoin;
+    const TileRange tr = tile_range(A.nelem);
+    if (tr.first >= tr.end) return;
+    // element of round r in the chunk, and its place in LDS
+    auto slot = [&](int r) { return (r * Q::G + grp) * NE + sub; };
+    auto elem = [&](int tile, int r) { return min(tile * CH + slot(r), A.nelem - 1); };
+    int n[E];
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const int t = r * NT + lane;
-            if (t < BLK) {
-                const int an = t / CH, c = t % CH;
-                lb[c * NN + an] = A.helem[(c0 + min(c, cn - 1)) + (size_t)A.nelem * an];
+    for (int r = 0; r < E; ++r) n[r] = A.connecT[(size_t)elem(tr.first, r) * NN + a];
+    for (int tile = tr.first; tile < tr.end; tile += tr.stride) {
+        const int c0 = tile * CH, cn = min(CH, A.nelem - c0);
+        double u0[E], u1[E], u2[E], T[E], rho[E], re[E], hk[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            u0[r] = A.u[n[r]];
+            u1[r] = A.u[n[r] + np];
+            u2[r] = A.u[n[r] + 2 * np];
+            T[r] = A.Tem[n[r]];
+            rho[r] = A.rho[n[r]];
+            re[r] = A.Reta[n[r]];
+            hk[r] = A.helem_k[elem(tile, r)];
+        }
+        // helem of the chunk (elements past the last re-read it)
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            const int t = i * Q::NTB + threadIdx.x;
+            if (t < BLK) lb[t % CH * ROW + t / CH] = A.helem[c0 + min(t % CH, cn - 1) + (size_t)A.nelem * (t / CH)];
+        }
+        const int tnext = tile + tr.stride < tr.end ? tile + tr.stride : tile;
+#pragma unroll
+        for (int r = 0; r < E; ++r) n[r] = A.connecT[(size_t)elem(tnext, r) * NN + a];
+        double be[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const double aux2 = sqrt(u0[r] * u0[r] + u1[r] * u1[r] + u2[r] * u2[r]);
+            const double aux3 = A.fact_low_mach * sqrt(A.Rgas * A.gamma * T[r]);
+            const double b = act ? (rho[r] * hk[r]) * (A.cmax / (double)P) * (aux2 + aux3) : 0.0;
+            if constexpr (NE == 2) {
+                const double b0 = wave_max(sub == 0 ? b : 0.0), b1 = wave_max(sub == 1 ? b : 0.0);
+                be[r] = sub == 0 ? b0 : b1;
+            } else {
+                be[r] = wave_max(b);
+                if constexpr (NW > 1)
+                    if (wl == 0) wmax[(grp * NW + lane / 64) * E + r] = be[r];
             }
         }
         lds_barrier();
-        for (int c = 0; c < cn; ++c) {
-            const int e = c0 + c;
-            load(nxt, c + 1 < cn ? e + 1 : cnext);
-            const double aux2 = sqrt(cur.u0 * cur.u0 + cur.u1 * cur.u1 + cur.u2 * cur.u2);
-            const double aux3 = A.fact_low_mach * sqrt(A.Rgas * A.gamma * cur.T);
-            double be = act ? (cur.rho * cur.hk) * (A.cmax / (double)P) * (aux2 + aux3) : 0.0;
+        double ml[E];
 #pragma unroll
-            for (int s = 32; s > 0; s >>= 1) be = fmax(be, __shfl_xor(be, s, 64));
+        for (int r = 0; r < E; ++r) {
             if constexpr (NW > 1) {
-                if (wl == 0) wmax[wv] = be;
-                lds_barrier();
-                be = wmax[0];
 #pragma unroll
-                for (int w2 = 1; w2 < NW; ++w2) be = fmax(be, wmax[w2]);
+                for (int w = 0; w < NW; ++w) be[r] = fmax(be[r], wmax[(grp * NW + w) * E + r]);
             }
-            const double nrm = A.norm_i ? A.norm_i[A.elem_inst[e]] : norm;
-            const double R1 = cur.rho * fabs(cur.Reta) / nrm;
-            const double h = lb[c * NN + a];
+            const double nrm = A.norm_i ? A.norm_i[A.elem_inst[elem(tile, r)]] : norm;
+            const double R1 = rho[r] * fabs(re[r]) / nrm;
+            const double h = lb[slot(r) * ROW + a];
             const double Ve = A.ce * R1 * (h * h);
-            const double ml = A.cglob * fmin(Ve, be);
-            if (act) lb[c * NN + a] = ml; // the lane's own h slot
-            lds_barrier();
-            double acc = 0.0;
-#pragma unroll
-            for (int l = 0; l < 3; ++l)
-#pragma unroll
-                for (int m = 0; m < 3; ++m)
-#pragma unroll
-                    for (int nn = 0; nn < 3; ++nn)
-                        acc += w[l] * w[m] * w[nn] * lb[c * NN + src[9 * l + 3 * m + nn]];
-            if (act) ob[c * NN + a] = acc;
-            cur = nxt;
+            ml[r] = A.cglob * fmin(Ve, be[r]);
         }
+        // the three line passes, lb -> ob -> lb, in line order (a group's own rows)
+        double v[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) v[r] = ml[r];
+        unit_sync<NW>();
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            double *const buf = k == 1 ? ob : lb;
+            if (act)
+#pragma unroll
+                for (int r = 0; r < E; ++r) buf[slot(r) * ROW + at] = v[r];
+            unit_sync<NW>();
+#pragma unroll
+            for (int r = 0; r < E; ++r)
+                v[r] = filter_line(buf[slot(r) * ROW + fl.n[k][0]], v[r], buf[slot(r) * ROW + fl.n[k][1]]);
+        }
+        unit_sync<NW>();
+        if (act)
+#pragma unroll
+            for (int r = 0; r < E; ++r) {
+                lb[slot(r) * ROW + a] = ml[r];
+                ob[slot(r) * ROW + a] = v[r];
+            }
         lds_barrier();
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const int t = r * NT + lane;
-            if (t < BLK) {
-                const int an = t / CH, c = t % CH;
-                if (c < cn) {
-                    const size_t g = (c0 + c) + (size_t)A.nelem * an;
-                    A.mue_l[g] = lb[c * NN + an];
-                    A.mu_e[g] = ob[c * NN + an];
-                }
+        for (int i = 0; i < ROWS; ++i) {
+            const int t = i * Q::NTB + threadIdx.x;
+            if (t < BLK && t % CH < cn) {
+                const size_t g = c0 + t % CH + (size_t)A.nelem * (t / CH);
+                A.mue_l[g] = lb[t % CH * ROW + t / CH];
+                A.mu_e[g] = ob[t % CH * ROW + t / CH];
             }
         }
         lds_barrier(); // the next chunk overwrites lb and ob
@@ -574,10 +625,11 @@ static int smart_visc(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoi
     A.elem_inst = norm_i ? ens->elem_inst : nullptr;
     A.mu_e = mu_e;
     A.mue_l = mue_l;
+    const int grid = tile_grid(nelem, ctx->num_cu);
     switch (porder) {
-    case 2: k_smart_visc_ch<2, 16, T><<<elem_grid(ctx, (nelem + 15) / 16, 8), 64, 0, ctx->stream>>>(A); break;
-    case 3: k_smart_visc_ch<3, 16, T><<<elem_grid(ctx, (nelem + 15) / 16, 8), 64, 0, ctx->stream>>>(A); break;
-    case 4: k_smart_visc_ch<4, 16, T><<<elem_grid(ctx, (nelem + 15) / 16, 8), SG<4>::NT, 0, ctx->stream>>>(A); break;
+    case 2: k_smart_visc<2, T><<<grid, SensorShape<2>::NTB, 0, ctx->stream>>>(A); break;
+    case 3: k_smart_visc<3, T><<<grid, SensorShape<3>::NTB, 0, ctx->stream>>>(A); break;
+    case 4: k_smart_visc<4, T><<<grid, SensorShape<4>::NTB, 0, ctx->stream>>>(A); break;
     }
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());

@@ -45,33 +45,29 @@ __device__ __forceinline__ int convert_ijk(int g, int P)
     return g + 1; // 2..P -> 3..P+1
 }
 
-// The 27 element-local sources of node a's filter value: the node at
-// geometric offset (l-1, m-1, n-1) of a, reflected at the element boundary by
-// convertIJK, in the reference's (l, m, n) loop order.
-template <int P>
-__device__ __forceinline__ void filter_sources(int a, const int *inv, int src[27])
+// The 3x3x3 filter is the product of three line filters (weights 1/4, 1/2, 1/4, the
+// neighbours at geometric offset -1 and +1 reflected at the element boundary by
+// convertIJK).  at: position of the lane's node in line order (I fastest, the
+// order of inv), n[k]: the positions of its two neighbours along line k.
+template <int P> struct FilterLane {
+    int n[3][2];
+    __device__ __forceinline__ explicit FilterLane(int at)
+    {
+        constexpr int N1 = SG<P>::N1;
+        const int own[3] = {at % N1, at / N1 % N1, at / (N1 * N1)};
+        const int stride[3] = {1, N1, N1 * N1};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int g = geo_of(own[k] + 1, N1);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                n[k][s] = at + (convert_ijk(g + 2 * s - 1, P) - 1 - own[k]) * stride[k];
+        }
+    }
+};
+__device__ __forceinline__ double filter_line(double lo, double own, double hi)
 {
-    constexpr int N1 = SG<P>::N1, NN = SG<P>::NN;
-    int I = 1, J = 1, K = 1;
-    for (int k = 0; k < N1; ++k)
-        for (int j = 0; j < N1; ++j)
-            for (int i = 0; i < N1; ++i)
-                if (inv[i + N1 * (j + N1 * k)] - 1 == a) {
-                    I = i + 1;
-                    J = j + 1;
-                    K = k + 1;
-                }
-    const int ii = geo_of(I, N1), jj = geo_of(J, N1), kk = geo_of(K, N1);
-#pragma unroll
-    for (int l = 0; l < 3; ++l)
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-#pragma unroll
-            for (int n = 0; n < 3; ++n) {
-                const int ci = convert_ijk(ii + l - 1, P) - 1, cj = convert_ijk(jj + m - 1, P) - 1,
-                          ck = convert_ijk(kk + n - 1, P) - 1;
-                src[9 * l + 3 * m + n] = min(max(inv[ci + N1 * (cj + N1 * ck)] - 1, 0), NN - 1);
-            }
+    return 0.25 * (lo + hi) + 0.5 * own; // the products are exact
 }
 
 // blocks of the entropy normalisation's reductions: its partial maxima take

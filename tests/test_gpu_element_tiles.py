@@ -67,3 +67,52 @@ def test_tile_edges(p, box):
     ref = O.adapt_dt_cfl(p, m.connec, g.helem, f["u"], cs, 0.5, 0.4, f["mu_fluid"], f["mu_sgs"],
                          f["mu_e"], f["rho"])
     assert abs(dt.value - ref) <= 1e-13 * ref
+
+
+@pytest.mark.parametrize("p", [2, 3, 4])
+@pytest.mark.parametrize("box", [(1, 1, 1), (5, 3, 1), (4, 2, 2), (17, 1, 1), (11, 3, 1)])
+def test_sensor_chunk_edges(p, box):
+    """smart_visc_spectral over chunks of 16 elements: the maximum and the filter are
+    formed in FP64 (positive weights, fewer than 40 roundings: 1e-13); the FP32
+    interface rounds the result once (2^-24: 2e-7)."""
+    import torch
+    from oracle import oracle as O
+    from sod2d_amd import device as D
+    from sod2d_amd._lib import check, lib
+
+    g = make_case(p, box, periodic=False, jitter=0.05, lengths=(1.0, 1.1, 0.9))
+    m, T = g.mesh, g.tables
+    n, ne, nn = m.npoin, m.nelem, T.nnode
+    r = np.random.default_rng(40 + p)
+    f = dict(Reta=r.normal(0, 1.0, n) * 10.0 ** r.uniform(-2, 4, n), rho=r.uniform(0.9, 1.1, n),
+             u=np.asfortranarray(r.normal(0, 0.3, (n, 3))), Tem=r.uniform(0.9, 1.1, n),
+             eta=r.normal(size=n), h=g.helem_l, hk=g.helem)
+    OT = O.Tables(p)
+    up = D.to_dev
+    connec, lw, inv = up(m.connec), up(m.lpoin_w), up(T.invAtoIJK)
+    prm = D.visc_params(287.0)
+    for dt, tol in ((torch.float64, 1e-13), (torch.float32, 2e-7)):
+        d = {k: up(v).to(dt) for k, v in f.items()}
+        mu, ml = (torch.full((ne * nn,), 7.0, dtype=dt, device="cuda") for _ in range(2))
+        if dt == torch.float64:
+            D.smart_visc_spectral(ne, n, m.npoin_w, connec, lw, d["Reta"], None, None, None, None,
+                                  None, 1.4, d["rho"], d["u"], None, d["Tem"], d["eta"], d["h"],
+                                  d["hk"], None, mu, inv, None, None, None, ml, prm)
+            o = f
+        else:
+            ctx = D.Context(0)
+            ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+            torch.cuda.synchronize()
+            check(lib().sodhip_smart_visc_spectral_f32(
+                ctx.h, p, ne, n, m.npoin_w, ptr(connec), ptr(lw), ptr(d["Reta"]), C.c_float(1.4),
+                ptr(d["rho"]), ptr(d["u"]), ptr(d["Tem"]), ptr(d["eta"]), ptr(d["h"]),
+                ptr(d["hk"]), ptr(inv), C.byref(prm), ptr(mu), ptr(ml)), "smart_visc f32")
+            o = {k: np.asfortranarray(np.asarray(v, np.float32).astype(np.float64))
+                 for k, v in f.items()}
+        torch.cuda.synchronize()
+        omu, oml = O.smart_visc_spectral(OT, m.connec, m.lpoin_w, o["Reta"],
+                                         float(np.float32(1.4)) if dt == torch.float32 else 1.4,
+                                         o["rho"], o["u"], o["Tem"], o["eta"], o["h"], o["hk"],
+                                         O.visc_params(287.0), fz((ne, nn)))
+        assert relerr(ml.cpu().numpy(), oml.ravel(order="F")) < tol
+        assert relerr(mu.cpu().numpy(), omu.ravel(order="F")) < tol
