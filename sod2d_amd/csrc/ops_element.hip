@@ -115,20 +115,20 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
 //
 // What bounds it: the convection moves 8 GB between L1 and L2 at 553k elements, p=3
 // (5 GB of them from HBM) and waits for them most of the time; it runs at about
-// 5 TB/s of HBM traffic against 5.7 TB/s of a large copy.  The viscous operator adds
-// the element-fastest mu arrays (64 lines per element and array), the kernel of both
-// operators LDS reads (51 of 16 bytes per lane at p=4) and FP64 arithmetic.  Against
+// 5 TB/s of HBM traffic against 5.7 TB/s of a large copy.  The kernel of both
+// operators adds LDS reads (51 of 16 bytes per lane at p=4) and FP64 arithmetic.  Against
 // one element per workgroup in gmsh lane order with W-weighted sums, and geometry
 // in 4-byte rows at odd p=4 elements (kernel times, one box):
-//   p=3 FP64, 553k elements: convection 1.64 -> 1.25 ms, viscous 1.94 -> 1.54 ms
+//   p=3 FP64, 553k elements: convection 1.64 -> 1.25 ms, viscous 1.94 -> 1.28 ms
 //   p=4 FP64,  63k elements: convection 0.77 -> 0.34 ms, viscous 0.80 -> 0.34 ms
 //   p=4 FP32,  46k elements: convection 0.30 -> 0.15 ms, viscous 0.36 -> 0.18 ms
 //   both, fused stage: p=4 FP64, 48k elements 1.57 -> 0.30 ms (it spilled 124
 //   registers; 0.42 ms with q and rho H as fields of their own); p=2 FP64, 152k elements
-//   0.47 -> 0.15 ms; p=3 FP64, 262k elements 0.83 -> 0.76 ms and p=3 with FP32
+//   0.47 -> 0.15 ms; p=3 FP64, 262k elements 0.83 -> 0.64 ms and p=3 with FP32
 //   operators, 87k elements 0.21 -> 0.17 ms against two waves per element, one per
-//   operator, that hand over through LDS.  At p=3 FP64 the vector ALU is busy 42 %
-//   and LDS 38 % of the time with two waves per SIMD.
+//   operator, that hand over through LDS.  The group's viscosities come together
+//   (mu_issue): with every lane reading its own the p=3 kernels touched 64 lines per
+//   element and array and took 0.76 ms (fused) and 1.54 ms (viscous).
 //   LPS: p=4, 41k elements, convection and stabilised operator 0.77 (two kernels, the
 //   second adding to the first one's records) -> 0.40 ms, projections 0.36 -> 0.20 ms;
 //   p=3, 111k elements, 0.55 (two waves per element) -> 0.34 ms and 0.41 -> 0.27 ms;
@@ -186,6 +186,12 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     __shared__ __attribute__((aligned(16))) T area_s[G * L::AREA];
     __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * GEO];
     __shared__ int conn_s[G * 2 * NT];
+    // viscosities of the group's elements, [array][node][element]; by turns in two
+    // places where no barrier separates their reads from the next copies
+    constexpr bool MUS = FLUX && G > 1;
+    constexpr int NMU = CONS ? 1 : 2, MUB = MUS ? (NN * G * (int)sizeof(T) + 255) / 256 * 256 : 0;
+    constexpr int MUN = NW > 1 ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) unsigned char mu_s[MUS ? MUN * NMU * MUB : 4];
     // this thread's unit of the group, and its LDS
     const int sb = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
     T *const area = area_s + sb * L::AREA;
@@ -208,6 +214,22 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     auto conn_issue = [&](int u, int slot) {
         const size_t i = (size_t)u * NL + lane;
         dma_lds<4>(A.connecT + (i < EN ? i : EN - 1), conn_at + (slot * NT + wv * 64) * 4);
+    };
+    // The element-fastest (nelem, nnode) viscosities of group g, G neighbours at a time:
+    // the lanes of one row copy 256 bytes of [node][element], 4 each
+    auto mu_issue = [&](int g, int slot) {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+#pragma unroll
+        for (int r0 = 0; r0 < MUB / 256; r0 += Q::NTB / 64) {
+            const int r = r0 + wave, b = r * 256 + 4 * wl;
+            if (MUB / 256 % (Q::NTB / 64) != 0 && r >= MUB / 256) break;
+            const int node = min(b / (G * (int)sizeof(T)), NN - 1), in = b % (G * (int)sizeof(T));
+            const size_t at = (size_t)min(g * G + in / (int)sizeof(T), A.nelem - 1) + (size_t)A.nelem * node;
+            const unsigned to = lds_addr(mu_s) + slot % MUN * NMU * MUB + r * 256;
+            dma_lds<4>((const char *)(A.mu_e + at) + in % (int)sizeof(T), to);
+            if constexpr (!CONS)
+                if (A.mu_sgs) dma_lds<4>((const char *)(A.mu_sgs + at) + in % (int)sizeof(T), to + MUB);
+        }
     };
     __shared__ T tcol[L::TLDS ? 3 * P * Q::NT : 1];
     if constexpr (L::TLDS)
@@ -265,7 +287,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             if constexpr (LPS) x.n = n;
         }
         if constexpr (LPS) x.tau = A.tau[min(u * NE + ln.sub, A.nelem - 1)];
-        if constexpr (FLUX) {
+        if constexpr (FLUX && !MUS) {
             const size_t eg = (size_t)min(u * NE + ln.sub, A.nelem - 1) + (size_t)A.nelem * ln.a;
             x.mue = A.mu_e[eg];
             if constexpr (!CONS) x.musgs = A.mu_sgs ? A.mu_sgs[eg] : T(0);
@@ -277,6 +299,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     GeoAt at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, unit(er.begin), geo_at, wl, wv);
     conn_issue(unit(er.begin), 0);
     conn_issue(unit(min(er.begin + er.stride, ulast)), 1);
+    if constexpr (MUS) mu_issue(er.begin, 0);
     wait_vm<0>();
     lds_barrier();
     load(cur, unit(er.begin), 0);
@@ -296,6 +319,11 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 for (int i = 0; i < 3; ++i) He[i][j] = hp[i + 3 * j];
         }
         const T vol = ((const T *)(geo + Q::HEA + at.gv))[ln.sub * NN + ln.a];
+        if constexpr (MUS) {
+            const T *m = (const T *)(mu_s + (slot ^ 1) % MUN * NMU * MUB) + ln.a * G + sb;
+            cur.mue = m[0];
+            if constexpr (!CONS) cur.musgs = A.mu_sgs ? m[MUB / sizeof(T)] : T(0);
+        }
         typename O::V out[O::NC];
         O::read(out, area, lane);
         lds_done();
@@ -307,6 +335,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             for (int i = 0; i < L::PI; ++i) pn[i] = conn[(slot ^ 1) * NT + pj_node[i * NT + lane]];
         }
         unit_sync<NW>();
+        if constexpr (MUS) mu_issue(min(g + er.stride, ulast), slot);
         if constexpr (L::PJ) {
 #pragma unroll
             for (int i = 0; i < L::PI; ++i) {
@@ -731,7 +760,9 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
 //
 // What bounds it: memory.  The 80 bytes of geometry per element-node are most of
 // what is read; copied through LDS they are read once and in order, where each lane
-// read its own 72 bytes of He at a stride of 72 (MEASURED).
+// read its own 72 bytes of He at a stride of 72: entropy convection 432 -> 356 us
+// (262k elements, p=3; 335 us at a large copy's rate), 250 -> 145 us (48k, p=4) and
+// 143 -> 102 us (152k, p=2); DIVCURL 220 -> 127 us (41k, p=4).
 enum class GradOp { SFUSED, SFLUX, DIV, CURL, DIVCURL };
 
 // waves per SIMD asked of the compiler: as many as run without spilling
