@@ -119,8 +119,8 @@ template <typename T> __device__ __forceinline__ T sutherland(T mu_factor, T Tk)
 // operators adds LDS reads (51 of 16 bytes per lane at p=4) and FP64 arithmetic.  Against
 // one element per workgroup in gmsh lane order with W-weighted sums, and geometry
 // in 4-byte rows at odd p=4 elements (kernel times, one box):
-//   p=3 FP64, 553k elements: convection 1.64 -> 1.25 ms, viscous 1.94 -> 1.28 ms
-//   p=4 FP64,  63k elements: convection 0.77 -> 0.34 ms, viscous 0.80 -> 0.34 ms
+//   p=3 FP64, 553k elements: convection 1.64 -> 1.14 ms, viscous 1.94 -> 1.28 ms
+//   p=4 FP64,  63k elements: convection 0.77 -> 0.32 ms, viscous 0.80 -> 0.34 ms
 //   p=4 FP32,  46k elements: convection 0.30 -> 0.15 ms, viscous 0.36 -> 0.18 ms
 //   both, fused stage: p=4 FP64, 48k elements 1.57 -> 0.30 ms (it spilled 124
 //   registers; 0.42 ms with q and rho H as fields of their own); p=2 FP64, 152k elements
@@ -138,7 +138,18 @@ template <int P, typename T, bool CONV, int VISC, bool CONS> struct ElemLDS {
     using Q = EP<P, T>;
     // nodal records (values), flux records and residual records share one area
     // of one stride, so that a line neighbour has one LDS offset
-    static constexpr int REC = VISC == 3 ? 12 : VISC ? 18 : 10, AREA = REC * Q::NT;
+    // A group's units take their nodes together, line by line over the group's
+    // elements (a gather's consecutive lanes then follow an i-line through G
+    // neighbours and share its cache lines), where nothing but gathers and geometry is
+    // read: the drop-in convection takes 1.14 instead of 1.25 ms (p=3, 553k elements)
+    // and 321 instead of 336 us (p=4, 63k), the projections 266 instead of 269 us.  The
+    // two barriers that this costs are not paid back in the kernels with a viscous flux:
+    // 1.27 against 1.28 ms drop-in, and the fused stage 665 against 640 us (p=3, 262k)
+    // and 312 against 300 us (p=4, 48k).  The areas of a group's units start 16 banks
+    // apart.
+    static constexpr bool JOINT = Q::G > 1 && (VISC == 0 || VISC == 3);
+    static constexpr int REC = VISC == 3 ? 12 : VISC ? 18 : 10,
+                         AREA = REC * Q::NT + (JOINT ? 64 / (int)sizeof(T) : 0);
     // at p=4 the transposed coefficients of both operators' kernel do not fit in
     // the registers beside the rest: they stay in LDS, one column per lane
     static constexpr bool TLDS = CONV && VISC && P == 4;
@@ -253,16 +264,31 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     auto ld2 = [&](int i) { return *(const V2 *)(area + i); };
     auto st2 = [&](int i, T x, T y) { *(V2 *)(area + i) = V2{x, y}; };
 
-    // inputs of one unit at the lane's node (loaded one unit ahead)
+    // The node whose inputs this thread reads (one group of units ahead) and stages
+    constexpr bool JOINT = L::JOINT;
+    int gu = sb, gl = lane, ga = ln.a; // unit of the group, record, node
+    if constexpr (JOINT) {
+        constexpr int N1 = Q::N1, PAD = NT - NN;
+        const int t = threadIdx.x, line = t / (G * N1), r = t % (G * N1);
+        gu = r / N1;
+        gl = line * N1 + r % N1;
+        if (PAD > 0 && line >= N1 * N1) { // threads without a node fill the padding
+            gu = (t - G * NN) / PAD;
+            gl = NN + (t - G * NN) % PAD;
+        }
+        ga = min(max(A.inv[gl < NN ? gl : 0] - 1, 0), NN - 1);
+    }
+    T *const garea = area_s + gu * L::AREA + gl * REC;
+    const int *const gconn = conn_s + gu * 2 * NT + (JOINT ? ga : ln.sub * NN + ln.a);
     struct In {
         double cr, cq[3], cE;                     // conserved state (CONS)
         T rho, u[3], q[3], pr, E, Tem, rhon, muf; // primitive inputs (drop-in)
         T mue, musgs;
-        double tau; // LPS
-        int n;
+        double tau; // LPS, own unit
+        int n;      // own node
     };
-    auto load = [&](In &x, int u, int slot) {
-        const int n = conn[slot * NT + ln.sub * NN + ln.a];
+    auto load = [&](In &x, int g, int slot) {
+        const int n = gconn[slot * NT];
         if constexpr (CONS) {
             x.cr = A.cr[n];
             x.cq[0] = A.cq[n];
@@ -284,11 +310,12 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 x.rhon = A.rho_n[n];
                 x.muf = A.mu_fluid[n];
             }
-            if constexpr (LPS) x.n = n;
+            if constexpr (LPS) x.n = conn[slot * NT + ln.sub * NN + ln.a];
         }
-        if constexpr (LPS) x.tau = A.tau[min(u * NE + ln.sub, A.nelem - 1)];
+        const int e = min(unit(g) * NE + ln.sub, A.nelem - 1);
+        if constexpr (LPS) x.tau = A.tau[e];
         if constexpr (FLUX && !MUS) {
-            const size_t eg = (size_t)min(u * NE + ln.sub, A.nelem - 1) + (size_t)A.nelem * ln.a;
+            const size_t eg = (size_t)e + (size_t)A.nelem * ln.a;
             x.mue = A.mu_e[eg];
             if constexpr (!CONS) x.musgs = A.mu_sgs ? A.mu_sgs[eg] : T(0);
         }
@@ -302,7 +329,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     if constexpr (MUS) mu_issue(er.begin, 0);
     wait_vm<0>();
     lds_barrier();
-    load(cur, unit(er.begin), 0);
+    load(cur, er.begin, 0);
     int slot = 1, prev = -1;
     for (int g = er.begin; g < er.end; g += er.stride, slot ^= 1) {
         const int u = unit(g), u2 = unit(min(g + er.stride, ulast)),
@@ -328,13 +355,13 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         O::read(out, area, lane);
         lds_done();
         if (prev >= 0) O::store(out, area, A.out, prev, A.nelem, lane);
-        load(nxt, u2, slot);
+        load(nxt, min(g + er.stride, ulast), slot);
         int pn[L::PJ ? L::PI : 1];
         if constexpr (L::PJ) {
 #pragma unroll
             for (int i = 0; i < L::PI; ++i) pn[i] = conn[(slot ^ 1) * NT + pj_node[i * NT + lane]];
         }
-        unit_sync<NW>();
+        unit_sync<JOINT ? 2 : NW>(); // (of a group: every unit's records have been read)
         if constexpr (MUS) mu_issue(min(g + er.stride, ulast), slot);
         if constexpr (L::PJ) {
 #pragma unroll
@@ -359,6 +386,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         // ---------------- stage
         T rho, v[3], q[3] = {0, 0, 0}, H = 0, rhoH = 0, p = 0, Tk = 0, muf = 0, rhon = 0, musgs = 0;
         const T mue = FLUX ? cur.mue : T(0);
+        if constexpr (FLUX && !CONS) musgs = cur.musgs;
         if constexpr (CONS) {
             const double r = cur.cr, ri = 1.0 / r;
             double ud[3], umag = 0.0;
@@ -401,21 +429,41 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             if constexpr (FLUX) {
                 rhon = cur.rhon;
                 muf = cur.muf;
-                musgs = cur.musgs;
             }
         }
         // (lanes without a node write records of their own past the unit's: a
         // condition here would let the compiler sink the arithmetic behind it)
         const int own = lane * REC;
-        st2(own, v[0], v[1]);
-        st2(own + 2, v[2], rho);
-        if constexpr (CONV) st2(own + 4, p, H);
+        auto put = [&](int i, T x, T y) { *(V2 *)(garea + i) = V2{x, y}; };
+        put(0, v[0], v[1]);
+        put(2, v[2], rho);
+        if constexpr (CONV) put(4, p, H);
         if constexpr (CONV && !RHOU) {
-            st2(own + 6, rhoH, q[0]);
-            st2(own + 8, q[1], q[2]);
+            put(6, rhoH, q[0]);
+            put(8, q[1], q[2]);
         }
-        if constexpr (VISC != 0) area[own + TEM] = Tk;
-        unit_sync<NW>();
+        if constexpr (VISC != 0) garea[TEM] = Tk;
+        unit_sync<JOINT ? 2 : NW>();
+        if constexpr (JOINT) { // back to the lane's own node
+            const V2 x01 = ld2(own), x2r = ld2(own + 2);
+            v[0] = x01.x;
+            v[1] = x01.y;
+            v[2] = x2r.x;
+            rho = x2r.y;
+            if constexpr (CONV) {
+                const V2 xpH = ld2(own + 4);
+                p = xpH.x;
+                H = xpH.y;
+            }
+            if constexpr (CONV && !RHOU) {
+                const V2 xHq = ld2(own + 6), xqq = ld2(own + 8);
+                rhoH = xHq.x;
+                q[0] = xHq.y;
+                q[1] = xqq.x;
+                q[2] = xqq.y;
+            }
+            if constexpr (VISC != 0) Tk = area[own + TEM];
+        }
 
         // ---------------- lines
         T Rm = 0, Rq[3] = {0, 0, 0}, Re = 0;
