@@ -641,6 +641,21 @@ int sodhip_rk_stage_f64(sodhip_ctx ctx, int porder, int nelem, int npoin, int np
                         const double *q1, const double *E1, double *rho, double *q, double *E,
                         double *Rmass, double *Rmom, double *Rener);
 
+/* sodhip_rk_stage_f64 with R evaluated at the state (rho_at, q_at, E_at) instead of
+ * the one it overwrites, e.g. stage 1 at y1: y <- lam1*y1 + lams*y + gam*dt*R(y1)
+ * without a copy of y1 to y first.  rho_at, q_at and E_at may be rho1, q1 and E1,
+ * or rho, q and E. */
+int sodhip_rk_stage_from_f64(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_w,
+                             const int *connec, const int *lpoin_w, int op_precision,
+                             const void *He, const void *gpvol, const void *dlxigp_ip,
+                             const int *invAtoIJK, const int *gmshAtoI, const int *gmshAtoJ,
+                             const int *gmshAtoK, const void *mu_e, const double *invMl,
+                             const sodhip_stage_params *prm, double dt, double lam1, double lams,
+                             double gam, const double *rho1, const double *q1, const double *E1,
+                             double *rho, double *q, double *E, double *Rmass, double *Rmom,
+                             double *Rener, const double *rho_at, const double *q_at,
+                             const double *E_at);
+
 /* sodhip_rk_stage_f64 for the last stage of a step at fixed dt, fused with the
  * first stage of the next step of the reference sequencing: besides the new
  * state y (rho, q, E), stores y_next = 1 * y + 0 * 0 + gam_next * dt * R over

@@ -107,6 +107,8 @@ _SIGS = {
     "sodhip_entropy_residual_f64": (I, [P, I, I, P, D, D, P, P, P]),
     "sodhip_rk_stage_f64": (I, [P, I, I, I, I, P, P, I] + [P] * 9
                             + [C.POINTER(StageParams), D, D, D, D] + [P] * 9),
+    "sodhip_rk_stage_from_f64": (I, [P, I, I, I, I, P, P, I] + [P] * 9
+                                 + [C.POINTER(StageParams), D, D, D, D] + [P] * 12),
     "sodhip_rk_stage_next_f64": (I, [P, I, I, I, I, P, P, I] + [P] * 9
                                  + [C.POINTER(StageParams), D, D, D, D] + [P] * 9
                                  + [D, P, P, P]),

@@ -232,7 +232,8 @@ int rhs_cluster_stage(sodhip_ctx ctx, const MeshCache *m, const ClusterTables *c
                       const double *invMl, double fact, double dt, double lam1, double lams,
                       double gam, const double *rho1, const double *q1, const double *E1,
                       double *rho, double *q, double *E, double *Rmass, double *Rmom,
-                      double *Rener, const NextStage *next, double *rec);
+                      double *Rener, const NextStage *next, const double *const st[3],
+                      double *rec);
 // gather/update of one stage from element records of rw (5 or 6) values
 // (ops_stage.hip)
 template <typename TS>

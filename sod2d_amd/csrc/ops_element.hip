@@ -1990,7 +1990,8 @@ int rhs_cluster_stage(sodhip_ctx ctx, const MeshCache *m, const ClusterTables *c
                       const double *invMl, double fact, double dt, double lam1, double lams,
                       double gam, const double *rho1, const double *q1, const double *E1,
                       double *rho, double *q, double *E, double *Rmass, double *Rmom,
-                      double *Rener, const NextStage *next, double *rec)
+                      double *Rener, const NextStage *next, const double *const st[3],
+                      double *rec)
 {
     using T = double;
     RhsArgs<T> A{};
@@ -2006,9 +2007,9 @@ int rhs_cluster_stage(sodhip_ctx ctx, const MeshCache *m, const ClusterTables *c
     A.gI = gI;
     A.gJ = gJ;
     A.gK = gK;
-    A.cr = rho;
-    A.cq = q;
-    A.cE = E;
+    A.cr = st[0];
+    A.cq = st[1];
+    A.cE = st[2];
     A.mu_e = mu_e;
     A.gamma = gamma;
     A.Rgas = Rgas;

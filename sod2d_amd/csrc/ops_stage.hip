@@ -282,7 +282,7 @@ template int gather_update<double>(sodhip_ctx, const MeshCache *, int, int, cons
                                    double *, double *, const NextStage *);
 
 // One fused stage on the mesh tables m (with its working incidence built) and
-// the record scratch scr of scr_bytes
+// the record scratch scr of scr_bytes; the RHS is evaluated at the state st
 template <typename T>
 static int rk_stage_on(sodhip_ctx ctx, int porder, const MeshCache *m, int npoin, int npoin_w,
                        const int *lpoin_w, const T *He, const T *gpvol, const T *dl,
@@ -290,8 +290,9 @@ static int rk_stage_on(sodhip_ctx ctx, int porder, const MeshCache *m, int npoin
                        const double *invMl, const sodhip_stage_params *prm, double dt,
                        double lam1, double lams, double gam, const double *rho1, const double *q1,
                        const double *E1, double *rho, double *q, double *E, double *Rmass,
-                       double *Rmom, double *Rener, const NextStage *next, void *scr_mem,
-                       size_t scr_bytes, const ClusterTables *cl)
+                       double *Rmom, double *Rener, const NextStage *next,
+                       const double *const st[3], void *scr_mem, size_t scr_bytes,
+                       const ClusterTables *cl)
 {
     const size_t EN = (size_t)m->nelem * nnode_of(porder);
     if constexpr (sizeof(T) == 8) {
@@ -308,7 +309,7 @@ static int rk_stage_on(sodhip_ctx ctx, int porder, const MeshCache *m, int npoin
                                        prm->mu_factor, prm->mu_factor_e, prm->c_rho,
                                        prm->c_ener, prm->p_ref, invMl,
                                        prm->fact, dt, lam1, lams, gam, rho1, q1, E1, rho, q, E,
-                                       Rmass, Rmom, Rener, next, rec);
+                                       Rmass, Rmom, Rener, next, st, rec);
             if (rc) return rc;
             return gather_update_on<double>(ctx, npoin, cl->ns, cl->snode, cl->srow, cl->ssrc,
                                             rec, 5, invMl, prm->fact, dt, lam1, lams, gam, rho1,
@@ -321,7 +322,7 @@ static int rk_stage_on(sodhip_ctx ctx, int porder, const MeshCache *m, int npoin
         return set_error(SODHIP_ERR_ARG, "the stage needs %zu bytes of record scratch, %zu available",
                          rw * EN * sizeof(T), scr_bytes);
     T *scr = (T *)scr_mem;
-    int rc = rhs_fused_elements<T>(ctx, porder, m, He, gpvol, dl, inv, gI, gJ, gK, rho, q, E, mu_e,
+    int rc = rhs_fused_elements<T>(ctx, porder, m, He, gpvol, dl, inv, gI, gJ, gK, st[0], st[1], st[2], mu_e,
                                    prm->gamma_gas, prm->Rgas, prm->Cp, prm->Pr, prm->mu_factor, prm->mu_factor_e,
                                    prm->c_rho, prm->c_ener, prm->p_ref, scr);
     if (rc) return rc;
@@ -337,7 +338,8 @@ static int rk_stage(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
                     const T *mu_e, const double *invMl, const sodhip_stage_params *prm, double dt,
                     double lam1, double lams, double gam, const double *rho1, const double *q1,
                     const double *E1, double *rho, double *q, double *E, double *Rmass,
-                    double *Rmom, double *Rener, const NextStage *next = nullptr)
+                    double *Rmom, double *Rener, const NextStage *next = nullptr,
+                    const double *const *from = nullptr)
 {
     MeshCache *m = nullptr;
     int rc = get_mesh(ctx, porder, nelem, npoin, connec, &m);
@@ -353,9 +355,10 @@ static int rk_stage(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
     }
     const size_t need = cl ? (size_t)cl->nloc * 5 * sizeof(double) : rw * EN * sizeof(T);
     if ((rc = ensure_buf(ctx->scratch, need))) return rc;
+    const double *const at[3] = {from ? from[0] : rho, from ? from[1] : q, from ? from[2] : E};
     return rk_stage_on<T>(ctx, porder, m, npoin, npoin_w, lpoin_w, He, gpvol, dl, inv, gI, gJ, gK,
                           mu_e, invMl, prm, dt, lam1, lams, gam, rho1, q1, E1, rho, q, E, Rmass,
-                          Rmom, Rener, next, ctx->scratch.ptr, ctx->scratch.bytes, cl);
+                          Rmom, Rener, next, at, ctx->scratch.ptr, ctx->scratch.bytes, cl);
 }
 
 // One classical RK4 stage (see k_gather_rk4): the fused RHS at the stage state
@@ -733,6 +736,41 @@ extern "C" int sodhip_rk_stage_next_f64(
     return set_error(SODHIP_ERR_ARG, "op_precision must be 8 or 4 (got %d)", op_precision);
 }
 
+extern "C" int sodhip_rk_stage_from_f64(
+    sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_w, const int *connec,
+    const int *lpoin_w, int op_precision, const void *He, const void *gpvol,
+    const void *dlxigp_ip, const int *invAtoIJK, const int *gmshAtoI, const int *gmshAtoJ,
+    const int *gmshAtoK, const void *mu_e, const double *invMl, const sodhip_stage_params *prm,
+    double dt, double lam1, double lams, double gam, const double *rho1, const double *q1,
+    const double *E1, double *rho, double *q, double *E, double *Rmass, double *Rmom,
+    double *Rener, const double *rho_at, const double *q_at, const double *E_at)
+{
+    SODHIP_REQUIRE(ctx && prm, "null argument");
+    SODHIP_REQUIRE(porder >= 2 && porder <= kMaxP, "porder %d not supported (2..4)", porder);
+    SODHIP_REQUIRE(nelem > 0 && npoin > 0 && npoin_w > 0 && npoin_w <= npoin,
+                   "invalid mesh sizes");
+    SODHIP_REQUIRE(connec && lpoin_w && He && gpvol && dlxigp_ip && invAtoIJK && gmshAtoI &&
+                       gmshAtoJ && gmshAtoK && mu_e && invMl && rho1 && q1 && E1 && rho && q && E,
+                   "null array argument");
+    SODHIP_REQUIRE(!!Rmass == !!Rmom && !!Rmom == !!Rener, "Rmass/Rmom/Rener: all or none");
+    SODHIP_REQUIRE(rho_at && q_at && E_at, "null state array");
+    SODHIP_TRY_HIP(hipSetDevice(ctx->device));
+    const double *const at[3] = {rho_at, q_at, E_at};
+    if (op_precision == 8)
+        return rk_stage<double>(ctx, porder, nelem, npoin, npoin_w, connec, lpoin_w,
+                                (const double *)He, (const double *)gpvol,
+                                (const double *)dlxigp_ip, invAtoIJK, gmshAtoI, gmshAtoJ, gmshAtoK,
+                                (const double *)mu_e, invMl, prm, dt, lam1, lams, gam, rho1, q1,
+                                E1, rho, q, E, Rmass, Rmom, Rener, nullptr, at);
+    if (op_precision == 4)
+        return rk_stage<float>(ctx, porder, nelem, npoin, npoin_w, connec, lpoin_w,
+                               (const float *)He, (const float *)gpvol, (const float *)dlxigp_ip,
+                               invAtoIJK, gmshAtoI, gmshAtoJ, gmshAtoK, (const float *)mu_e, invMl,
+                               prm, dt, lam1, lams, gam, rho1, q1, E1, rho, q, E, Rmass, Rmom,
+                               Rener, nullptr, at);
+    return set_error(SODHIP_ERR_ARG, "op_precision must be 8 or 4 (got %d)", op_precision);
+}
+
 extern "C" int sodhip_rk_stage_noalloc_f64(
     sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_w, const int *connec,
     const int *lpoin_w, int op_precision, const void *He, const void *gpvol,
@@ -764,6 +802,7 @@ extern "C" int sodhip_rk_stage_noalloc_f64(
     const MeshCache *m = nullptr;
     int rc = find_mesh(ctx, porder, nelem, npoin, connec, npoin_w, lpoin_w, &m);
     if (rc) return rc;
+    const double *const at[3] = {rho, q, E};
     // launch timing may create events: it is off for this call
     const bool prof = ctx->prof;
     ctx->prof = false;
@@ -772,14 +811,14 @@ extern "C" int sodhip_rk_stage_noalloc_f64(
                                  (const double *)gpvol, (const double *)dlxigp_ip, invAtoIJK,
                                  gmshAtoI, gmshAtoJ, gmshAtoK, (const double *)mu_e, invMl, prm,
                                  dt, lam1, lams, gam, rho1, q1, E1, rho, q, E, Rmass, Rmom, Rener,
-                                 nullptr, scr, kNoAllocScratchBytes,
+                                 nullptr, at, scr, kNoAllocScratchBytes,
                                  ctx->cluster_stage && porder == 3 ? m->clusters.get() : nullptr);
     else
         rc = rk_stage_on<float>(ctx, porder, m, npoin, npoin_w, lpoin_w, (const float *)He,
                                 (const float *)gpvol, (const float *)dlxigp_ip, invAtoIJK,
                                 gmshAtoI, gmshAtoJ, gmshAtoK, (const float *)mu_e, invMl, prm, dt,
                                 lam1, lams, gam, rho1, q1, E1, rho, q, E, Rmass, Rmom, Rener,
-                                nullptr, scr, kNoAllocScratchBytes, nullptr);
+                                nullptr, at, scr, kNoAllocScratchBytes, nullptr);
     ctx->prof = prof;
     return rc;
 }

@@ -1,0 +1,70 @@
+"""Time steps with a fresh stage 1 (parity=False), whose right-hand side is evaluated
+at level 1 (sodhip_rk_stage_from_f64) instead of at a copy of it, against the oracle.
+Per-step bar of the other time-loop tests (FP64 sums reassociate: 1e-12).  A stage
+from level 1 gives the bits of the stage in place on a copy of it, in both operator
+precisions."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import make_case, relerr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("p,n,clusters", [(2, 3, 0), (3, 3, 0), (3, 4, 1), (4, 2, 0)])
+@pytest.mark.parametrize("dt_mode", ["fixed", "adaptive"])
+def test_fresh_stage1(monkeypatch, p, n, clusters, dt_mode):
+    from oracle import oracle as O
+    from sod2d_amd.device import Context
+    from sod2d_amd.solver import TGVParams, TGVRun
+    g = make_case(p, n, periodic=True, lengths=(2 * np.pi,) * 3)
+    tp, to = TGVParams(), O.tgv_params()
+    ic = O.tgv_ic(g.mesh.coord, to)
+    if clusters:
+        monkeypatch.setenv("SODHIP_STAGE_CLUSTERS", "1")
+    ctx = Context(0)
+    monkeypatch.delenv("SODHIP_STAGE_CLUSTERS", raising=False)
+    run = TGVRun(p, geometry=g, params=tp, initial=ic, ctx=ctx, dt_mode=dt_mode, parity=False)
+    orc = O.TGVOracle(p, g, ic, to, parity=False, dt_mode=dt_mode, cfl=(tp.cfl_conv, tp.cfl_diff))
+    w = orc.lpoin_w - 1
+    for step in range(3):
+        run.step()
+        orc.step()
+        s = run.state()
+        for k in ("rho", "q", "E"):
+            assert relerr(s[k][w], getattr(orc, k)[1][w]) < 1e-12, (k, step)
+
+
+@pytest.mark.parametrize("p", [2, 3, 4])
+@pytest.mark.parametrize("precision", [8, 4])
+def test_stage_from_level1_is_the_stage_on_a_copy(p, precision):
+    import torch
+    from sod2d_amd._lib import check, lib
+    from sod2d_amd.device import _ptr
+    from sod2d_amd.solver import TGVRun
+    g = make_case(p, 3, periodic=True, lengths=(2 * np.pi,) * 3)
+    run = TGVRun(p, geometry=g, parity=False, dt_mode="fixed", op_precision=precision)
+    run.step()
+    y1 = [run.rho[1], run.q[1], run.E[1]]
+    R = [run.Rmass, run.Rmom, run.Rener]
+
+    def args(lam1, lams, y):
+        return (run.ctx.h, p, run.nelem, run.npoin, run.npoin_w, _ptr(run.connec),
+                _ptr(run.lpoin_w), precision, _ptr(run.He_op), _ptr(run.gpvol_op),
+                _ptr(run.dl_op), *[_ptr(x) for x in run.tabs], _ptr(run.mu_e_op),
+                _ptr(run.invMl), C.byref(run.sp), run.dt, lam1, lams, 0.25,
+                *[_ptr(x) for x in (*y1, *y, *R)])
+
+    ya = [x.clone() for x in y1]
+    check(lib().sodhip_rk_stage_f64(*args(0.0, 1.0, ya)), "rk_stage")
+    Ra = [x.clone() for x in R]
+    yb = [x.clone() for x in y1]
+    w = run.lpoin_w.long() - 1
+    for x in yb:  # what the stage overwrites is not read
+        x.view(-1, run.npoin)[:, w] = 7.0
+    check(lib().sodhip_rk_stage_from_f64(*args(1.0, 0.0, yb), *[_ptr(x) for x in y1]), "from")
+    torch.cuda.synchronize()
+    for a, b in zip((*ya, *Ra), (*yb, *R)):
+        assert torch.equal(a, b)
