@@ -128,8 +128,8 @@ struct sodhip_ctx_s {
     std::vector<std::unique_ptr<sodhip::MeshCache>> meshes;
     sodhip::DevBuf scratch;  // per element-node residual partials
     sodhip::DevBuf scratch2; // reduction partials of the step (the sensor's normalisation)
-    sodhip::DevBuf diag;     // reduction partials read back by the host (dt, diagnostics)
-    sodhip::DevBuf hostbuf;  // pinned staging (small reductions)
+    sodhip::DevBuf diag;     // reduction partials read back by the host (diagnostics)
+    sodhip::DevBuf hostbuf;  // pinned host memory that kernels write to (dt)
     bool prof = false;
     struct Pending {
         int kind;
@@ -156,6 +156,8 @@ namespace sodhip {
 
 // grows ctx->scratch to at least `bytes`
 int ensure_buf(DevBuf &b, size_t bytes);
+// the same for pinned host memory, which kernels address as the host does
+int ensure_host(DevBuf &b, size_t bytes);
 // mesh cache lookup/build for (connec, porder, nelem, npoin)
 int get_mesh(sodhip_ctx ctx, int porder, int nelem, int npoin, const int *connec,
              MeshCache **out);

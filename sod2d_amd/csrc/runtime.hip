@@ -46,6 +46,22 @@ int ensure_buf(DevBuf &b, size_t bytes)
     return SODHIP_OK;
 }
 
+int ensure_host(DevBuf &b, size_t bytes)
+{
+    if (b.bytes >= bytes && b.ptr) return SODHIP_OK;
+    if (b.ptr) SODHIP_TRY_HIP(hipHostFree(b.ptr));
+    b.ptr = nullptr;
+    b.bytes = 0;
+    const size_t want = std::max<size_t>(bytes, 4096);
+    hipError_t e = hipHostMalloc(&b.ptr, want, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        b.ptr = nullptr;
+        return set_error(SODHIP_ERR_ALLOC, "hipHostMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+    }
+    b.bytes = want;
+    return SODHIP_OK;
+}
+
 int diag_grid(sodhip_ctx ctx, int nelem, int blocks_per_cu)
 {
     const int g = std::min((nelem + 7) / 8 * 8, ctx->num_cu * blocks_per_cu);
