@@ -564,10 +564,10 @@ def main(argv=None):
                     == (16, 1, 256)), 5)})),
         },
         "roofline": {
-            "kernel": ("LPS stage (sodhip_rk_stage_lps_f64): k_rhs_split in LPS mode "
+            "kernel": ("LPS stage (sodhip_rk_stage_lps_f64): k_rhs in LPS mode "
                        "(convection and full_diff_stab_ijk) + k_gather_update, per stage; "
                        "full_proj_ijk (ms_projection) excluded" if a.lps else
-                       "fused RK stage: k_rhs_split (element) + k_gather_update (node)"),
+                       "fused RK stage: k_rhs (element) + k_gather_update (node)"),
             "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
             "algorithmic_bytes_per_stage": B,

@@ -167,7 +167,7 @@ int sodhip_copy_present(sodhip_ctx ctx, const void *src_host, void *dst_host, si
  * 3 other nodal kernels, 4 the LPS projections (full_proj_ijk's element
  * kernel and gather). */
 /* Launch shape of the fused RK stage on this context: blocks per CU of the
- * element kernel (1..64; with a grid-stride walk this sets the elements each
+ * element kernel (1..64; 16 is the library's own rule, other values scale the elements each
  * workgroup takes), whether the geometry moves through LDS in 16-byte lane
  * rows when He and gpvol are aligned for it (1) or in 4-byte rows (0), and
  * the gather/update block size (64, 128 or 256).  Defaults 16, 1, 256.  The

@@ -186,8 +186,6 @@ int eos_stage_sutherland(sodhip_ctx ctx, const MeshCache *m, double gamma_gas, d
 int prof_begin(sodhip_ctx ctx, int kind);
 void prof_end(sodhip_ctx ctx, int token);
 
-// XCD-aware grid: number of blocks for a grid-stride element loop
-int elem_grid(sodhip_ctx ctx, int nelem, int blocks_per_cu);
 // grid of the lane-per-node element loops (xcd_elems): a multiple of 8, at
 // most blocks_per_cu blocks per CU
 int diag_grid(sodhip_ctx ctx, int nelem, int blocks_per_cu = 32);

@@ -40,25 +40,6 @@ __device__ __forceinline__ XcdElems xcd_elems(int nelem)
     return {b + rk, min(nelem, b + span), per};
 }
 
-// max over the block of NW waves (one value per wave in sh[NW]); every lane
-// returns the maximum
-template <int NW> __device__ __forceinline__ double block_max_w(double v, double *sh)
-{
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v = fmax(v, __shfl_xor(v, s, 64));
-    if constexpr (NW == 1) {
-        return v;
-    } else {
-        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-        __syncthreads();
-        double m = sh[0];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) m = fmax(m, sh[w]);
-        __syncthreads();
-        return m;
-    }
-}
-
 // Node order of the per-element reductions and limiters: alex[l] is the node at
 // lexicographic position l of the element's (i, j, k) line indices (the inverse
 // of the mesh cache's perm), so that a group of P+1 consecutive positions is one

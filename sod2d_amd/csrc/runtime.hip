@@ -68,16 +68,6 @@ int diag_grid(sodhip_ctx ctx, int nelem, int blocks_per_cu)
     return std::max(8, g / 8 * 8);
 }
 
-int elem_grid(sodhip_ctx ctx, int nelem, int blocks_per_cu)
-{
-    // a multiple of 8 so that every XCD receives the same number of blocks
-    long g = (long)ctx->num_cu * blocks_per_cu;
-    long need = ((long)nelem + 7) / 8 * 8;
-    g = std::min(g, need);
-    g = std::max<long>(8, (g + 7) / 8 * 8);
-    return (int)g;
-}
-
 static void free_mesh(MeshCache *m)
 {
     if (!m) return;
