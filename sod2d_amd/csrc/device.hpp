@@ -57,9 +57,20 @@ __device__ __forceinline__ void build_alex(const int *__restrict__ perm, int nno
 // t / 16 on, one line at p=2 and p=3 and at most two at p=4.  (A thread per element
 // walked all its lines one after the other, and a mesh of 1,728 elements
 // occupied 7 of 256 CUs: 85 us for smart_visc_spectral_imex, now 11; at 41k elements
-// 119 us, now 94.)  Each XCD takes one
-// contiguous eighth of the tiles, whose shared nodes then sit in its L2.
-constexpr int kTile = 16, kTileLines = 2;
+// 119 us, now 92.)  Each XCD takes one
+// contiguous eighth of the tiles, whose shared nodes then sit in its L2.  The kernels
+// are instances per line length KA: with five nodes read per line at every order, the
+// index clamped, the tiles were slower than a thread per element on large meshes
+// (343k elements, p=2: CFL step 97 us per thread, 127 clamped, 82 now; 262k, p=3: 200,
+// 236 and 208 us; smart_visc_spectral_imex 142, 164, 124 and 232, 280, 224 us).
+constexpr int kTile = 16;
+// launches the kernel for KA = porder + 1 nodes per line (porder checked before)
+#define SODHIP_BY_LINE(porder, launch)                                                     \
+    do {                                                                                   \
+        if ((porder) == 2) launch(3);                                                      \
+        else if ((porder) == 3) launch(4);                                                 \
+        else launch(5);                                                                    \
+    } while (0)
 struct TileRange {
     int first, end, stride; // tiles
 };

@@ -15,6 +15,7 @@ namespace sodhip {
 // comp_tau (elem_stab.f90:589-616): tau_e = max over the element's nodes of
 // h (fact_c c + |u|), h = helem_k (c_species_stab / p), over tiles of 16 elements
 // (device.hpp), all loads of an i-line issued together (fmax is exact).
+template <int KA>
 __global__ __launch_bounds__(256) void k_comp_tau(int nelem, int nnode, int porder,
                                                   const int *__restrict__ connec,
                                                   const int *__restrict__ perm,
@@ -27,27 +28,27 @@ __global__ __launch_bounds__(256) void k_comp_tau(int nelem, int nnode, int pord
     __shared__ double sh[64];
     __shared__ int alex[125];
     build_alex(perm, nnode, alex);
-    const int KA = porder + 1, nl = KA * KA;
+    constexpr int nl = KA * KA;
     const TileRange tr = tile_range(nelem);
     for (int t = tr.first; t < tr.end; t += tr.stride) {
         const int el = t * kTile + (threadIdx.x & 15), e = min(el, nelem - 1);
         const double h = helem_k[e] * (c_species_stab / (double)porder);
         double taul = 0.0;
         for (int l = threadIdx.x >> 4; l < nl; l += 16) {
-            int n[5];
+            int n[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j)
-                n[j] = connec[e + (size_t)nelem * alex[l * KA + min(j, KA - 1)]] - 1;
-            double u0[5], u1[5], u2[5], cs[5];
+            for (int j = 0; j < KA; ++j)
+                n[j] = connec[e + (size_t)nelem * alex[l * KA + j]] - 1;
+            double u0[KA], u1[KA], u2[KA], cs[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
+            for (int j = 0; j < KA; ++j) {
                 u0[j] = u[n[j]];
                 u1[j] = u[n[j] + (size_t)npoin];
                 u2[j] = u[n[j] + 2 * (size_t)npoin];
                 cs[j] = csound[n[j]];
             }
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
+            for (int j = 0; j < KA; ++j) {
                 const double aux1 = fact_c * cs[j] + sqrt(u0[j] * u0[j] + u1[j] * u1[j] + u2[j] * u2[j]);
                 taul = fmax(taul, h * aux1);
             }
@@ -228,9 +229,13 @@ extern "C" int sodhip_comp_tau_f64(sodhip_ctx ctx, int porder, int nelem, int np
     MeshCache *m = nullptr;
     int rc = get_mesh(ctx, porder, nelem, npoin, connec, &m);
     if (rc) return rc;
-    k_comp_tau<<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>(
-        nelem, nn, porder, connec, m->perm, csound, u, npoin, helem_k, c_species_stab,
-        flag_drop_c_in_envit ? 0.0 : 1.0, tau);
+    const int grid = tile_grid(nelem, ctx->num_cu);
+#define SODHIP_TAU(KA)                                                                     \
+    k_comp_tau<KA><<<grid, 256, 0, ctx->stream>>>( \
+        nelem, nn, porder, connec, m->perm, csound, u, npoin, helem_k, c_species_stab, \
+        flag_drop_c_in_envit ? 0.0 : 1.0, tau)
+    SODHIP_BY_LINE(porder, SODHIP_TAU);
+#undef SODHIP_TAU
     SODHIP_TRY_HIP(hipGetLastError());
     return SODHIP_OK;
 }

@@ -225,6 +225,7 @@ struct ImexArgs {
     double *mu_e, *mue_l;
 };
 
+template <int KA>
 __global__ __launch_bounds__(256) void k_visc_imex(ImexArgs A)
 {
     __shared__ double sh[256];
@@ -240,28 +241,28 @@ __global__ __launch_bounds__(256) void k_visc_imex(ImexArgs A)
     const size_t NE = (size_t)A.nelem;
     const double *u1 = A.u + A.npoin, *u2 = A.u + 2 * (size_t)A.npoin;
     const double cp = A.cmax / (double)A.porder;
-    const int KA = A.porder + 1, nl = KA * KA;
+    constexpr int nl = KA * KA, LINES = (nl + 15) / 16;
     const TileRange tr = tile_range(A.nelem);
     for (int t = tr.first; t < tr.end; t += tr.stride) {
         const int el = t * kTile + (threadIdx.x & 15), e = min(el, A.nelem - 1);
         const double hk = A.helem_k[e];
         double betae = 0.0;
-        double rh[kTileLines][5], re[kTileLines][5];
+        double rh[LINES][KA], re[LINES][KA];
 #pragma unroll
-        for (int r = 0; r < kTileLines; ++r) {
+        for (int r = 0; r < LINES; ++r) {
             const int l = (threadIdx.x >> 4) + 16 * r;
             if (l >= nl) break;
-            size_t ea[5];
-            int n[5];
-            double mu[5], v0[5], v1[5], v2[5], cs[5];
+            size_t ea[KA];
+            int n[KA];
+            double mu[KA], v0[KA], v1[KA], v2[KA], cs[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                ea[j] = e + NE * alex[l * KA + min(j, KA - 1)];
+            for (int j = 0; j < KA; ++j) {
+                ea[j] = e + NE * alex[l * KA + j];
                 n[j] = A.connec[ea[j]] - 1;
                 mu[j] = A.mu_e[ea[j]];
             }
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
+            for (int j = 0; j < KA; ++j) {
                 v0[j] = A.u[n[j]];
                 v1[j] = u1[n[j]];
                 v2[j] = u2[n[j]];
@@ -270,8 +271,8 @@ __global__ __launch_bounds__(256) void k_visc_imex(ImexArgs A)
                 re[r][j] = A.Reta[n[j]];
             }
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                if (j < KA && el < A.nelem) A.mue_l[ea[j]] = mu[j];
+            for (int j = 0; j < KA; ++j) {
+                if (el < A.nelem) A.mue_l[ea[j]] = mu[j];
                 const double speed =
                     sqrt(v0[j] * v0[j] + v1[j] * v1[j] + v2[j] * v2[j]) + A.fact_low_mach * cs[j];
                 betae = fmax(betae, (rh[r][j] * hk) * cp * speed);
@@ -281,12 +282,11 @@ __global__ __launch_bounds__(256) void k_visc_imex(ImexArgs A)
         if (el >= A.nelem) continue;
         const double hp = hk / (double)A.porder;
 #pragma unroll
-        for (int r = 0; r < kTileLines; ++r) {
+        for (int r = 0; r < LINES; ++r) {
             const int l = (threadIdx.x >> 4) + 16 * r;
             if (l >= nl) break;
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                if (j >= KA) break;
+            for (int j = 0; j < KA; ++j) {
                 const double R1 = rh[r][j] * fabs(re[r][j]) / norm;
                 const double Ve = A.ce * R1 * (hp * hp);
                 A.mu_e[e + NE * alex[l * KA + j]] = A.cglob * fmin(Ve, betae);
@@ -323,6 +323,7 @@ __global__ __launch_bounds__(256) void k_ducros_node(int npoin, const double *__
 
 // the element pass, over tiles of 16 elements (device.hpp), all loads of an i-line
 // issued together
+template <int KA>
 __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder, int npoin,
                                                 const int *__restrict__ connec,
                                                 const int *__restrict__ perm,
@@ -333,22 +334,22 @@ __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder
     __shared__ int alex[125];
     build_alex(perm, nnode, alex);
     const size_t P1 = (size_t)npoin, P2 = 2 * (size_t)npoin;
-    const int KA = porder + 1, nl = KA * KA;
+    constexpr int nl = KA * KA;
     const TileRange tr = tile_range(nelem);
     for (int tile = tr.first; tile < tr.end; tile += tr.stride) {
         const int e = tile * kTile + (threadIdx.x & 15);
         if (e >= nelem) continue;
         for (int l = threadIdx.x >> 4; l < nl; l += 16) {
-            size_t t[5];
-            int n[5];
+            size_t t[KA];
+            int n[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                t[j] = (size_t)alex[l * KA + min(j, KA - 1)] * nelem + e;
+            for (int j = 0; j < KA; ++j) {
+                t[j] = (size_t)alex[l * KA + j] * nelem + e;
                 n[j] = connec[t[j]] - 1;
             }
-            double phi[5], d2[5], um[5], he[5], mu[5];
+            double phi[KA], d2[KA], um[KA], he[KA], mu[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
+            for (int j = 0; j < KA; ++j) {
                 phi[j] = nq[n[j]];
                 d2[j] = nq[n[j] + P1];
                 um[j] = nq[n[j] + P2];
@@ -356,8 +357,7 @@ __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder
                 mu[j] = mu_e[t[j]];
             }
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                if (j >= KA) break;
+            for (int j = 0; j < KA; ++j) {
                 const double rr = 1.0 * um[j] / he[j];
                 const double phi2 = d2[j] / (d2[j] + rr * rr + DBL_EPSILON);
                 mu_e[t[j]] = mu[j] * (fmax(phi[j] - dmin, 0.0) * phi2 + dmin);
@@ -728,7 +728,11 @@ extern "C" int sodhip_smart_visc_spectral_imex_f64(
     A.norm_min = high_mach ? 1 : 0;
     A.mu_e = mu_e;
     A.mue_l = mue_l;
-    k_visc_imex<<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>(A);
+#define SODHIP_IMEX(KA) \
+    k_visc_imex<KA><<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>( \
+        A)
+    SODHIP_BY_LINE(porder, SODHIP_IMEX);
+#undef SODHIP_IMEX
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());
     return SODHIP_OK;
@@ -754,9 +758,12 @@ extern "C" int sodhip_ducros_visc_limit_f64(sodhip_ctx ctx, int porder, int nele
     double *nq = (double *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 2);
     k_ducros_node<<<(npoin + 255) / 256, 256, 0, ctx->stream>>>(npoin, u, divU, vorti, Ml, nq);
-    k_ducros<<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>(nelem, nnode_of(porder), porder, npoin,
-                                                       connec, m->perm, nq, helem, ducros_min_val,
-                                                       mu_e);
+#define SODHIP_DUCROS(KA) \
+    k_ducros<KA><<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>( \
+        nelem, nnode_of(porder), porder, npoin, connec, m->perm, nq, helem, \
+        ducros_min_val, mu_e)
+    SODHIP_BY_LINE(porder, SODHIP_DUCROS);
+#undef SODHIP_DUCROS
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());
     return SODHIP_OK;

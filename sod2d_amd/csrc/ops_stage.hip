@@ -449,6 +449,7 @@ static void *noalloc_ptr(int device)
 // loads of an i-line issued before its arithmetic (fmax is exact, so the order does
 // not change the result); then the min over the block's elements.  At 512 elements,
 // p=3, a thread per element took 36 us, this 4 us; at 87k elements 87 and 71 us.
+template <int KA>
 __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder,
                                                 const int *__restrict__ connec,
                                                 const int *__restrict__ perm,
@@ -465,24 +466,24 @@ __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder
     __shared__ double sh[256];
     __shared__ int alex[125];
     build_alex(perm, nnode, alex);
-    const int KA = porder + 1, nl = KA * KA; // i-lines of KA nodes
+    constexpr int nl = KA * KA; // i-lines of KA nodes
     const TileRange tr = tile_range(nelem);
     double best = 1.0e14;
     for (int t = tr.first; t < tr.end; t += tr.stride) {
         const int el = t * kTile + (threadIdx.x & 15), e = min(el, nelem - 1);
         double L3 = 0.0, maxmu = 0.0;
         for (int l = threadIdx.x >> 4; l < nl; l += 16) {
-            int n[5];
-            size_t ea[5];
+            int n[KA];
+            size_t ea[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                const int a = alex[l * KA + min(j, KA - 1)];
+            for (int j = 0; j < KA; ++j) {
+                const int a = alex[l * KA + j];
                 ea[j] = e + (size_t)nelem * a;
                 n[j] = connec[ea[j]] - 1;
             }
-            double v0[5], v1[5], v2[5], cs[5], mf[5], me[5], sg[5], rh[5];
+            double v0[KA], v1[KA], v2[KA], cs[KA], mf[KA], me[KA], sg[KA], rh[KA];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
+            for (int j = 0; j < KA; ++j) {
                 v0[j] = u[n[j]];
                 v1[j] = u[n[j] + npoin];
                 v2[j] = u[n[j] + 2 * (size_t)npoin];
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder
                 }
             }
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
+            for (int j = 0; j < KA; ++j) {
                 double um = fabs(v0[j]);
                 um = fmax(um, fabs(v1[j]));
                 um = fmax(um, fabs(v2[j]));
@@ -883,9 +884,12 @@ extern "C" int sodhip_adapt_dt_cfl_f64(sodhip_ctx ctx, int porder, int nelem, in
     if ((rc = ensure_host(ctx->hostbuf, (size_t)nb * sizeof(double)))) return rc;
     double *part = (double *)ctx->hostbuf.ptr;
     int tok = prof_begin(ctx, 3);
-    k_dt_cfl<<<nb, 256, 0, ctx->stream>>>(nelem, nnode_of(porder), porder, connec, m->perm, helem,
-                                          u, csound, npoin, cfl_conv, cfl_diff, mu_fluid, mu_sgs,
-                                          mu_e, rho, part);
+#define SODHIP_DT(KA) \
+    k_dt_cfl<KA><<<nb, 256, 0, ctx->stream>>>( \
+        nelem, nnode_of(porder), porder, connec, m->perm, helem, u, csound, npoin, \
+        cfl_conv, cfl_diff, mu_fluid, mu_sgs, mu_e, rho, part)
+    SODHIP_BY_LINE(porder, SODHIP_DT);
+#undef SODHIP_DT
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());
     SODHIP_TRY_HIP(hipStreamSynchronize(ctx->stream));
