@@ -448,7 +448,7 @@ static void *noalloc_ptr(int device)
 // adapt_dt_cfl (mod_time_ops.f90:11-63) over tiles of 16 elements (device.hpp), all
 // loads of an i-line issued before its arithmetic (fmax is exact, so the order does
 // not change the result); then the min over the block's elements.  At 512 elements,
-// p=3, a thread per element took 36 us, this 4 us; at 87k elements 87 and 71 us.
+// p=3, a thread per element took 36 us, this 4 us; at 343k elements, p=2, 97 and 82 us.
 template <int KA>
 __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder,
                                                 const int *__restrict__ connec,
