@@ -194,6 +194,10 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
     // is 20 to 45 % less exact without)
     constexpr bool RHOU = CONS && sizeof(T) == 8;
     constexpr int TEM = 10; // temperature's place in the nodal record
+    constexpr bool DELTA = sizeof(T) == 4; // differences to the own node's values
+    // sums over the three lines, and products with the own node's values
+    constexpr bool WIDE = DELTA && !CONS;
+    using S = std::conditional_t<WIDE, double, T>;
     __shared__ __attribute__((aligned(16))) T area_s[G * L::AREA];
     __shared__ __attribute__((aligned(16))) unsigned char geo_s[G * GEO];
     __shared__ int conn_s[G * 2 * NT];
@@ -470,14 +474,22 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
         T du[3][3], dT[3]; // d u_i / d xi_k, d T / d xi_k
         T gR[3];           // grad rho
         {
-            T Ut[3] = {0, 0, 0}, Qt[3] = {0, 0, 0};
+            T Ut[3] = {0, 0, 0}, Qt[3] = {0, 0, 0}, dr[3], dp[3];
             // RHOU: divQ holds sum z rho(m) = div q + u.grad rho
-            T divU = 0, divQ = 0, dr[3], dp[3];
+            S divU = 0, divQ = 0;
             // Sums start with the own node's share.  FP32 sums the differences to the
             // own node's values (whose share is then the row sum rs of D, zero but for
             // rounding), so that a field's mean costs no digits of its derivative.
-            // FP64 has digits to spare and sums the values.
-            constexpr bool DELTA = sizeof(T) == 4;
+            // FP64 has digits to spare and sums the values.  On nodal noise, which has no
+            // mean to remove, the differences' own rounding made the drop-in operators
+            // less exact than separate derivatives are (error over result, p = 2, 3, 4:
+            // convection's energy 7.2e-8 -> 8.5 to 8.8e-8, viscous momentum 5.9, 6.6,
+            // 7.1e-8 -> 6.6, 7.6, 8.4e-8); with the sums over the lines and the closing
+            // products in FP64 (S, WIDE) they are 6.9 to 7.1e-8 and 5.8, 6.4, 6.9e-8, in the
+            // same time (46k elements, p=4, both operators: 398 us).
+            // The fused stage, whose states are smooth, is more exact than with separate
+            // derivatives as it is (a step's state by 10 to 30 %), and FP64 sums cost it
+            // 2 % of its time (87k elements, p=3: 1.72 -> 1.76 ms per step).
             T rs[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -586,19 +598,19 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                     Rq[i] = vol * (T(0.25) * (Rq[i] + v[i] * B) +
                                    (He[i][0] * dp[0] + He[i][1] * dp[1] + He[i][2] * dp[2]));
             } else if constexpr (CONV) {
-                const T urho = Ut[0] * dr[0] + Ut[1] * dr[1] + Ut[2] * dr[2];
-                const T s = divQ + urho;
+                const S urho = S(Ut[0]) * dr[0] + S(Ut[1]) * dr[1] + S(Ut[2]) * dr[2];
+                const S s = divQ + urho;
                 // the own values' coefficients: div q + u.grad rho for u_i and H,
                 // div u for q_i and rho H, and the own share of sum E and sum C (all of
                 // it where differences are summed)
-                const T ce = s + (b0 + rho * (DELTA ? divU : a0));
-                const T cc = DELTA ? T(2) * divU + a0 : divU + T(2) * a0;
-                Rm = vol * (T(0.5) * (s + rho * divU));
-                Re = vol * (T(0.25) * (Re + (H * ce + rhoH * cc)));
+                const S ce = s + (b0 + rho * (DELTA ? divU : a0));
+                const S cc = DELTA ? S(2) * divU + a0 : divU + S(2) * a0;
+                Rm = T(vol * (S(0.5) * (s + rho * divU)));
+                Re = T(vol * (S(0.25) * (Re + (H * ce + rhoH * cc))));
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
-                    Rq[i] = vol * (T(0.25) * (Rq[i] + (v[i] * ce + q[i] * cc)) +
-                                   (He[i][0] * dp[0] + He[i][1] * dp[1] + He[i][2] * dp[2]));
+                    Rq[i] = T(vol * (S(0.25) * (Rq[i] + (v[i] * ce + q[i] * cc)) +
+                                     (He[i][0] * dp[0] + He[i][1] * dp[1] + He[i][2] * dp[2])));
             }
         }
 
@@ -733,31 +745,43 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
                 conn_issue(u3, slot ^ 1);
             }
             // ---------------- weak divergence
+            S Ws[6]; // WIDE: the own share and the three lines' sums
+            if constexpr (WIDE)
+#pragma unroll
+                for (int f = 0; f < 6; ++f) Ws[f] = W[f];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
+                T l[6] = {0, 0, 0, 0, 0, 0};
+                T(&X)[6] = WIDE ? l : W;
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int o = 0; o < P; ++o) {
                     const int b = nb[k][o] + 6 * k;
                     const T c = L::TLDS ? tcol[(k * P + o) * NT + lane] : ln.t[k][o];
                     const V2 x01 = ld2(b), x23 = ld2(b + 2);
-                    if constexpr (LPS) { // W: mass, momentum 1, 2, 3, energy
-                        W[0] += c * x01.x;
-                        W[4] += c * x01.y;
-                        W[1] += c * x23.x;
-                        W[2] += c * x23.y;
-                        W[3] += c * area[b + 4];
+                    if constexpr (LPS) { // mass, momentum 1, 2, 3, energy
+                        X[0] += c * x01.x;
+                        X[4] += c * x01.y;
+                        X[1] += c * x23.x;
+                        X[2] += c * x23.y;
+                        X[3] += c * area[b + 4];
                     } else {
                         const V2 x45 = ld2(b + 4);
-                        W[0] += c * x01.x;
-                        W[1] += c * x01.y;
-                        W[2] += c * x23.x;
-                        W[3] += c * x23.y;
-                        W[4] += c * x45.x;
-                        W[5] += c * x45.y;
+                        X[0] += c * x01.x;
+                        X[1] += c * x01.y;
+                        X[2] += c * x23.x;
+                        X[3] += c * x23.y;
+                        X[4] += c * x45.x;
+                        X[5] += c * x45.y;
                     }
                 }
+                if constexpr (WIDE)
+#pragma unroll
+                    for (int f = 0; f < 6; ++f) Ws[f] += l[f];
             }
+            if constexpr (WIDE)
+#pragma unroll
+                for (int f = 0; f < 6; ++f) W[f] = T(Ws[f]);
             if constexpr (LPS) {
                 Rm += W[0];
                 Re += W[4];
