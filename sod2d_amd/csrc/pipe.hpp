@@ -38,11 +38,14 @@ template <int W> __device__ __forceinline__ void dma_lds(const void *g, unsigned
         asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "{m0}"(m) : "memory");
 }
 
-// wait until at most N of this wave's vector-memory operations are outstanding
+// wait until at most N of this wave's vector-memory operations are outstanding.  What
+// the copies write may be read right after it: the builtin is not relied on to keep the
+// compiler's reads behind the wait.
 template <int N> __device__ __forceinline__ void wait_vm()
 {
     static_assert(N >= 0 && N <= 63, "vmcnt range");
     __builtin_amdgcn_s_waitcnt((N & 15) | kWaitVm0 | ((N >> 4) << 14));
+    asm volatile("" ::: "memory");
 }
 
 // this wave's LDS reads have returned: a copy may overwrite what they read
