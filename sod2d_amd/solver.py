@@ -329,7 +329,7 @@ class TGVRun:
         if self.op_precision == 4:
             self.mu_e_op.copy_(self.mu_e)
 
-    def _stage(self, lam1, lams, gam, store_R, next_gam=None, at_level1=False):
+    def _stage(self, lam1, lams, gam, store_R, next_gam=None):
         if self.lps:
             # updateF with LPS (EOS, Sutherland, full_convec_ijk, full_proj_ijk,
             # full_diff_stab_ijk), lumped solve and stage combine in one call
@@ -356,10 +356,7 @@ class TGVRun:
                 _ptr(self.invMl), C.byref(self.sp), self.dt, lam1, lams, gam, _ptr(self.rho[0]),
                 _ptr(self.q[0]), _ptr(self.E[0]), _ptr(self.rho[1]), _ptr(self.q[1]),
                 _ptr(self.E[1]), *R)
-        if at_level1:
-            check(lib().sodhip_rk_stage_from_f64(*args, _ptr(self.rho[0]), _ptr(self.q[0]),
-                                                 _ptr(self.E[0])), "rk_stage_from")
-        elif next_gam is None:
+        if next_gam is None:
             check(lib().sodhip_rk_stage_f64(*args), "rk_stage")
         else:
             # the next step's stage 1 goes to level 1, which becomes level 2 at
@@ -414,14 +411,12 @@ class TGVRun:
         # before anything reads it, and on nodes outside lpoin_w both levels
         # keep their initial values.  With the reference sequencing stage 1
         # reads y^n from level 1 only (lam1 = 1, lams = 0 gives the values
-        # of lam1 = 0, lams = 1 on equal levels), and a fresh stage 1 evaluates
-        # its RHS there (sodhip_rk_stage_from_f64), so the conserved levels are
-        # exchanged too (a copy and its launches are 44 us of 2.65 ms at 48k
-        # elements, p=4).  A fresh LPS stage 1 evaluates its RHS at level 2,
-        # and they are copied.
-        level1 = not self.parity and not self.lps
+        # of lam1 = 0, lams = 1 on equal levels), so the conserved levels are
+        # exchanged too; otherwise stage 1 evaluates its RHS at level 2, which a
+        # caller may hold from step to step, and they are copied (36 us of 2626 at
+        # 48k elements, p=4).
         for lv in (self.rho, self.q, self.E):
-            if self.parity or level1:
+            if self.parity:
                 lv[0], lv[1] = lv[1], lv[0]
             else:
                 lv[0].copy_(lv[1])
@@ -443,11 +438,7 @@ class TGVRun:
             self._scalar_convec(self.Reta[:n])
             if self.sensor:
                 self._smart_visc(self.Reta[:n], self.rho[0], self.u[0], self.Tem[0], self.eta[:n])
-            # updateF at y^n: keeps R, y unchanged
-            if level1:
-                self._stage(1.0, 0.0, 0.0, True, at_level1=True)
-            else:
-                self._stage(0.0, 1.0, 0.0, True)
+            self._stage(0.0, 1.0, 0.0, True)  # updateF at y^n: keeps R, y unchanged
         if self.parity and self._next_dt is not None and self._next_dt == self.dt:
             pass  # stage 1 was stored by the previous step's last stage
         elif self.parity:
@@ -457,8 +448,6 @@ class TGVRun:
                 _ptr(self.rho[0]), _ptr(self.q[0]), _ptr(self.E[0]), _ptr(self.rho[1]),
                 _ptr(self.q[1]), _ptr(self.E[1]), _ptr(self.Rmass), _ptr(self.Rmom),
                 _ptr(self.Rener)), "rk_stage_update")
-        elif level1:
-            self._stage(1.0, 0.0, G[1, 0], False, at_level1=True)
         else:
             self._stage(0.0, 1.0, G[1, 0], False)
         self._next_dt = None

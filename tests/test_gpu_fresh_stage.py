@@ -1,8 +1,8 @@
-"""Time steps with a fresh stage 1 (parity=False), whose right-hand side is evaluated
-at level 1 (sodhip_rk_stage_from_f64) instead of at a copy of it, against the oracle.
-Per-step bar of the other time-loop tests (FP64 sums reassociate: 1e-12).  A stage
-from level 1 gives the bits of the stage in place on a copy of it, in both operator
-precisions."""
+"""Time steps with a fresh stage 1 (parity=False) against the oracle, the tensors of
+level 2 that a caller keeps across them, and the stage evaluated at another state than
+the one it overwrites (sodhip_rk_stage_from_f64).  Per-step bar of the other time-loop
+tests (FP64 sums reassociate: 1e-12).  A stage from level 1 gives the bits of the stage
+in place on a copy of it, in both operator precisions."""
 import ctypes as C
 
 import numpy as np
@@ -35,6 +35,28 @@ def test_fresh_stage1(monkeypatch, p, n, clusters, dt_mode):
         s = run.state()
         for k in ("rho", "q", "E"):
             assert relerr(s[k][w], getattr(orc, k)[1][w]) < 1e-12, (k, step)
+
+
+@pytest.mark.parametrize("precision,lps", [(8, False), (4, False), (8, True)])
+def test_level2_tensors_stay_level2(precision, lps):
+    """A caller may take run.rho[1], run.q[1] and run.E[1] once; what it writes there
+    at nodes that no working node stands for stays."""
+    import torch
+    from sod2d_amd.solver import TGVRun
+    g = make_case(3, 3, periodic=True, lengths=(2 * np.pi,) * 3)
+    run = TGVRun(3, geometry=g, parity=False, dt_mode="fixed", op_precision=precision, lps=lps)
+    held = [run.rho[1], run.q[1], run.E[1]]
+    rest = torch.ones(run.npoin, dtype=torch.bool, device="cuda")
+    rest[run.lpoin_w.long() - 1] = False
+    assert rest.any()
+    held[0][rest] = 7.0
+    for step in range(3):
+        before = [x.clone() for x in held]
+        run.step()
+        for x, y, b, lv in zip(held, (run.rho, run.q, run.E), before, "rqE"):
+            assert x is y[1], (lv, step)
+            assert torch.equal(y[0], b) and not torch.equal(x, b), (lv, step)
+        assert (held[0][rest] == 7.0).all()
 
 
 @pytest.mark.parametrize("p", [2, 3, 4])
