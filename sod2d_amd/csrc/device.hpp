@@ -63,39 +63,47 @@ __device__ __forceinline__ void build_alex(const int *__restrict__ perm, int nno
 // index clamped, the tiles were slower than a thread per element on large meshes
 // (343k elements, p=2: CFL step 97 us per thread, 127 clamped, 82 now; 262k, p=3: 200,
 // 236 and 208 us; smart_visc_spectral_imex 142, 164, 124 and 232, 280, 224 us).
-constexpr int kTile = 16;
+// The CFL step and the Ducros limit, which keep nothing between a tile's passes over
+// memory, take tiles of W = 64 on meshes with two of those per CU: on large ones the
+// 128-byte pieces of rows far apart cost more than the shorter walk gains, most where
+// the row length is a power of two (calls, us, per thread / 16 / 64 wide: Ducros 262k
+// elements, p=3: 274, 296, 256; 343k, p=2: 131, 121, 109; 41k, p=4: 149, 102, 98; CFL
+// 221, 222, 183; 108, 90, 74; 92, 76, 70).  Smaller ones would idle CUs (8,000, p=4:
+// Ducros 20 and 27 us, CFL 30 and 36 us, 16 and 64 wide).
+constexpr int kTile = 16, kWideTile = 64;
+inline bool wide_tiles(int nelem, int num_cu) { return nelem / kWideTile >= 2 * num_cu; }
 // launches the kernel for KA = porder + 1 nodes per line (porder checked before)
-#define SODHIP_BY_LINE(porder, launch)                                                     \
+#define SODHIP_BY_LINE(porder, launch, ...)                                                \
     do {                                                                                   \
-        if ((porder) == 2) launch(3);                                                      \
-        else if ((porder) == 3) launch(4);                                                 \
-        else launch(5);                                                                    \
+        if ((porder) == 2) launch(3, ##__VA_ARGS__);                                       \
+        else if ((porder) == 3) launch(4, ##__VA_ARGS__);                                  \
+        else launch(5, ##__VA_ARGS__);                                                     \
     } while (0)
 struct TileRange {
     int first, end, stride; // tiles
 };
-__device__ __forceinline__ TileRange tile_range(int nelem)
+template <int W = kTile> __device__ __forceinline__ TileRange tile_range(int nelem)
 {
-    const int tiles = (nelem + kTile - 1) / kTile, span = (tiles + 7) >> 3;
+    const int tiles = (nelem + W - 1) / W, span = (tiles + 7) >> 3;
     const int b = (blockIdx.x & 7) * span;
     return {b + (int)(blockIdx.x >> 3), min(tiles, b + span), (int)(gridDim.x >> 3)};
 }
 // at most eight blocks per CU
-inline int tile_grid(int nelem, int num_cu)
+inline int tile_grid(int nelem, int num_cu, int width = kTile)
 {
-    const int tiles = (nelem + kTile - 1) / kTile, span = (tiles + 7) / 8;
+    const int tiles = (nelem + width - 1) / width, span = (tiles + 7) / 8;
     return 8 * std::max(1, std::min(span, num_cu));
 }
-// maximum over the 16 threads of each element; every thread returns its
-// element's (sh: 64 doubles)
-__device__ __forceinline__ double tile_max(double v, double *sh)
+// maximum over the 256 / W threads of each element; every thread returns its
+// element's (sh: 4 W doubles)
+template <int W = kTile> __device__ __forceinline__ double tile_max(double v, double *sh)
 {
-    v = fmax(v, __shfl_xor(v, 16, 64));
-    v = fmax(v, __shfl_xor(v, 32, 64));
-    const int el = threadIdx.x & 15;
-    if ((threadIdx.x & 63) < 16) sh[(threadIdx.x >> 6) * 16 + el] = v;
+#pragma unroll
+    for (int s = W; s < 64; s *= 2) v = fmax(v, __shfl_xor(v, s, 64));
+    const int el = threadIdx.x % W;
+    if ((threadIdx.x & 63) < W) sh[(threadIdx.x >> 6) * W + el] = v;
     __syncthreads();
-    const double m = fmax(fmax(sh[el], sh[16 + el]), fmax(sh[32 + el], sh[48 + el]));
+    const double m = fmax(fmax(sh[el], sh[W + el]), fmax(sh[2 * W + el], sh[3 * W + el]));
     __syncthreads();
     return m;
 }

@@ -321,9 +321,9 @@ __global__ __launch_bounds__(256) void k_ducros_node(int npoin, const double *__
     nq[n + P2] = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
 }
 
-// the element pass, over tiles of 16 elements (device.hpp), all loads of an i-line
+// the element pass, over tiles of W elements (device.hpp), all loads of an i-line
 // issued together
-template <int KA>
+template <int KA, int W>
 __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder, int npoin,
                                                 const int *__restrict__ connec,
                                                 const int *__restrict__ perm,
@@ -335,11 +335,11 @@ __global__ __launch_bounds__(256) void k_ducros(int nelem, int nnode, int porder
     build_alex(perm, nnode, alex);
     const size_t P1 = (size_t)npoin, P2 = 2 * (size_t)npoin;
     constexpr int nl = KA * KA;
-    const TileRange tr = tile_range(nelem);
+    const TileRange tr = tile_range<W>(nelem);
     for (int tile = tr.first; tile < tr.end; tile += tr.stride) {
-        const int e = tile * kTile + (threadIdx.x & 15);
+        const int e = tile * W + threadIdx.x % W;
         if (e >= nelem) continue;
-        for (int l = threadIdx.x >> 4; l < nl; l += 16) {
+        for (int l = threadIdx.x / W; l < nl; l += 256 / W) {
             size_t t[KA];
             int n[KA];
 #pragma unroll
@@ -758,11 +758,12 @@ extern "C" int sodhip_ducros_visc_limit_f64(sodhip_ctx ctx, int porder, int nele
     double *nq = (double *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 2);
     k_ducros_node<<<(npoin + 255) / 256, 256, 0, ctx->stream>>>(npoin, u, divU, vorti, Ml, nq);
-#define SODHIP_DUCROS(KA) \
-    k_ducros<KA><<<tile_grid(nelem, ctx->num_cu), 256, 0, ctx->stream>>>( \
+#define SODHIP_DUCROS(KA, W) \
+    k_ducros<KA, W><<<tile_grid(nelem, ctx->num_cu, W), 256, 0, ctx->stream>>>( \
         nelem, nnode_of(porder), porder, npoin, connec, m->perm, nq, helem, \
         ducros_min_val, mu_e)
-    SODHIP_BY_LINE(porder, SODHIP_DUCROS);
+    if (wide_tiles(nelem, ctx->num_cu)) SODHIP_BY_LINE(porder, SODHIP_DUCROS, kWideTile);
+    else SODHIP_BY_LINE(porder, SODHIP_DUCROS, kTile);
 #undef SODHIP_DUCROS
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());

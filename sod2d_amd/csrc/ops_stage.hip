@@ -445,11 +445,11 @@ static void *noalloc_ptr(int device)
 }
 
 // ---------------------------------------------------------------- CFL time step
-// adapt_dt_cfl (mod_time_ops.f90:11-63) over tiles of 16 elements (device.hpp), all
+// adapt_dt_cfl (mod_time_ops.f90:11-63) over tiles of W elements (device.hpp), all
 // loads of an i-line issued before its arithmetic (fmax is exact, so the order does
 // not change the result); then the min over the block's elements.  At 512 elements,
-// p=3, a thread per element took 36 us, this 4 us; at 343k elements, p=2, 97 and 82 us.
-template <int KA>
+// p=3, a thread per element took 36 us, this 4 us.
+template <int KA, int W>
 __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder,
                                                 const int *__restrict__ connec,
                                                 const int *__restrict__ perm,
@@ -467,12 +467,12 @@ __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder
     __shared__ int alex[125];
     build_alex(perm, nnode, alex);
     constexpr int nl = KA * KA; // i-lines of KA nodes
-    const TileRange tr = tile_range(nelem);
+    const TileRange tr = tile_range<W>(nelem);
     double best = 1.0e14;
     for (int t = tr.first; t < tr.end; t += tr.stride) {
-        const int el = t * kTile + (threadIdx.x & 15), e = min(el, nelem - 1);
+        const int el = t * W + threadIdx.x % W, e = min(el, nelem - 1);
         double L3 = 0.0, maxmu = 0.0;
-        for (int l = threadIdx.x >> 4; l < nl; l += 16) {
+        for (int l = threadIdx.x / W; l < nl; l += 256 / W) {
             int n[KA];
             size_t ea[KA];
 #pragma unroll
@@ -504,8 +504,8 @@ __global__ __launch_bounds__(256) void k_dt_cfl(int nelem, int nnode, int porder
                 if (mu_fluid) maxmu = fmax(maxmu, (sg[j] + mf[j] + me[j]) / rh[j]);
             }
         }
-        L3 = tile_max(L3, sh);
-        if (mu_fluid) maxmu = tile_max(maxmu, sh);
+        L3 = tile_max<W>(L3, sh);
+        if (mu_fluid) maxmu = tile_max<W>(maxmu, sh);
         if (el < nelem) {
             const double hh = helem[e] / (double)(2 * porder + 1);
             double dtl = cfl_conv * hh / L3;
@@ -877,18 +877,20 @@ extern "C" int sodhip_adapt_dt_cfl_f64(sodhip_ctx ctx, int porder, int nelem, in
     int rc = get_mesh(ctx, porder, nelem, npoin, connec, &m);
     if (rc) return rc;
     SODHIP_REQUIRE(porder >= 2 && porder <= kMaxP, "porder %d not supported (2..4)", porder);
-    const int nb = tile_grid(nelem, ctx->num_cu);
+    const bool wide = wide_tiles(nelem, ctx->num_cu);
+    const int nb = tile_grid(nelem, ctx->num_cu, wide ? kWideTile : kTile);
     // the blocks' minima (at most eight per CU) go straight to host memory: one
     // synchronisation, where a copy behind the kernel cost a launch and a staging
     // copy more (512 elements, p=3: a time step of 191 us, now 176)
     if ((rc = ensure_host(ctx->hostbuf, (size_t)nb * sizeof(double)))) return rc;
     double *part = (double *)ctx->hostbuf.ptr;
     int tok = prof_begin(ctx, 3);
-#define SODHIP_DT(KA) \
-    k_dt_cfl<KA><<<nb, 256, 0, ctx->stream>>>( \
+#define SODHIP_DT(KA, W) \
+    k_dt_cfl<KA, W><<<nb, 256, 0, ctx->stream>>>( \
         nelem, nnode_of(porder), porder, connec, m->perm, helem, u, csound, npoin, \
         cfl_conv, cfl_diff, mu_fluid, mu_sgs, mu_e, rho, part)
-    SODHIP_BY_LINE(porder, SODHIP_DT);
+    if (wide) SODHIP_BY_LINE(porder, SODHIP_DT, kWideTile);
+    else SODHIP_BY_LINE(porder, SODHIP_DT, kTile);
 #undef SODHIP_DT
     prof_end(ctx, tok);
     SODHIP_TRY_HIP(hipGetLastError());

@@ -116,3 +116,19 @@ def test_sensor_chunk_edges(p, box):
                                          O.visc_params(287.0), fz((ne, nn)))
         assert relerr(ml.cpu().numpy(), oml.ravel(order="F")) < tol
         assert relerr(mu.cpu().numpy(), omu.ravel(order="F")) < tol
+
+
+# A block's second and later tiles: 8,785 tiles of 16 and 2,197 of 64 elements over the
+# 2,048 blocks of 256 CUs at p=2, 2,179 and 2,110 of 16 at p=3 and p=4, each with a part
+# of a tile at the end; and p=4 on either side of the line between the two widths
+ROUNDS = [(2, (51, 52, 53)), (3, (33, 32, 33)), (4, (33, 33, 31)), (4, (32, 33, 31))]
+
+
+@pytest.mark.parametrize("p,box", ROUNDS)
+def test_tile_rounds(p, box):
+    test_tile_edges(p, box)
+
+
+@pytest.mark.parametrize("p,box", ROUNDS[:3])
+def test_sensor_chunk_rounds(p, box):
+    test_sensor_chunk_edges(p, box)
