@@ -834,7 +834,8 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
 // what is read; copied through LDS they are read once and in order, where each lane
 // read its own 72 bytes of He at a stride of 72: entropy convection 432 -> 356 us
 // (262k elements, p=3; 335 us at a large copy's rate), 250 -> 145 us (48k, p=4) and
-// 143 -> 102 us (152k, p=2); DIVCURL 220 -> 127 us (41k, p=4).
+// 143 -> 102 us (152k, p=2); DIVCURL 220 -> 127 us (41k, p=4).  CURL does not copy the
+// gpvol that it does not read: the call 614 -> 591 us (262k, p=3), 410 -> 400 us (85k, p=4).
 enum class GradOp { SFUSED, SFLUX, DIV, CURL, DIVCURL };
 
 // waves per SIMD asked of the compiler: as many as run without spilling
@@ -854,6 +855,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (grad_waves<P, T, OP>())) void k_g
                    CURL = OP == GradOp::CURL || OP == GradOp::DIVCURL;
     constexpr int NN = Q::NN, NL = Q::NL, NT = Q::NT, NE = Q::NE, NW = Q::NW, G = Q::G;
     constexpr int RW = SC ? 1 : (DIV ? 1 : 0) + (CURL ? 3 : 0);
+    constexpr bool VOL = SC || DIV; // the vorticity alone is not weighted
     // nodal records u1 u2 | u3 eta | f1 f2 | f3 -, at a stride of an odd number of
     // pairs, so that 16 consecutive records start in 16 different banks
     constexpr int REC = FLUX ? 10 : 6;
@@ -895,7 +897,7 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (grad_waves<P, T, OP>())) void k_g
     using O = RecOut<P, T, RW>;
 
     In cur, nxt;
-    GeoAt at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, unit(er.begin), geo_at, wl, wv);
+    GeoAt at = geo_issue<P, T, VOL>(A.He, A.gpvol, A.nelem, nunits, A.geo16, unit(er.begin), geo_at, wl, wv);
     conn_issue(unit(er.begin), 0);
     conn_issue(unit(min(er.begin + er.stride, ulast)), 1);
     wait_vm<0>();
@@ -915,14 +917,14 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (grad_waves<P, T, OP>())) void k_g
 #pragma unroll
                 for (int i = 0; i < 3; ++i) He[i][j] = hp[i + 3 * j];
         }
-        const T vol = ((const T *)(geo + Q::HEA + at.gv))[ln.sub * NN + ln.a];
+        const T vol = VOL ? ((const T *)(geo + Q::HEA + at.gv))[ln.sub * NN + ln.a] : T(1);
         typename O::V out[O::NC];
         O::read(out, area, lane);
         lds_done();
         if (prev >= 0) O::store(out, area, A.out, prev, A.nelem, lane);
         load(nxt, slot);
         unit_sync<NW>();
-        at = geo_issue<P, T>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
+        at = geo_issue<P, T, VOL>(A.He, A.gpvol, A.nelem, nunits, A.geo16, u2, geo_at, wl, wv);
         conn_issue(u3, slot ^ 1);
         prev = g * G + sb < nunits ? u : -1;
 
@@ -2269,7 +2271,7 @@ static int div_curl(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
-    A.gpvol = gpvol ? gpvol : He; // not used by the vorticity
+    A.gpvol = gpvol; // not read where only the vorticity is asked for
     A.dl = dl;
     A.inv = inv;
     A.gI = gI;

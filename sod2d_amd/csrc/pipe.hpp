@@ -146,26 +146,31 @@ struct GeoAt {
     int he, gv;
 };
 
-// copies unit's He and gpvol to geo (LDS address); the waves take alternate rows
-template <int P, typename T>
+// copies unit's He and, with VOL, gpvol to geo (LDS address); the waves take alternate
+// rows
+template <int P, typename T, bool VOL = true>
 __device__ __forceinline__ GeoAt geo_issue(const T *He, const T *gpvol, int nelem, int nunits,
                                            bool geo16, int unit, unsigned geo, int wl, int wv)
 {
     using Q = EP<P, T>;
+    constexpr int END = Q::HEA + (VOL ? Q::GVA : 0);
+    constexpr int ROWS16 = (END + 1023) / 1024, ROWS4 = (END + 255) / 256;
     const size_t hb = (size_t)unit * Q::HEB, gb = (size_t)unit * Q::GVB;
     const unsigned char *he = (const unsigned char *)He + hb;
-    const unsigned char *gv = (const unsigned char *)gpvol + gb;
+    // without VOL the lanes past the end of He read its last bytes again
+    const unsigned char *gv = VOL ? (const unsigned char *)gpvol + gb : he;
     const bool last = unit == nunits - 1;
     const bool wide = geo16 && (!last || (Q::ALIGNED && nelem % Q::NE == 0));
     if (wide) {
         const GeoAt at{Q::ALIGNED ? 0 : (int)(hb & 15), Q::ALIGNED ? 0 : (int)(gb & 15)};
         he -= at.he;
-        gv -= at.gv;
+        gv -= VOL ? at.gv : at.he;
 #pragma unroll
-        for (int r0 = 0; r0 < Q::ROWS16; r0 += Q::NW) {
+        for (int r0 = 0; r0 < ROWS16; r0 += Q::NW) {
             const int r = r0 + wv, byte = r * 1024 + wl * 16;
-            const unsigned char *src = byte < Q::HEA ? he + byte : gv + min(byte - Q::HEA, Q::GVA - 16);
-            if (Q::ROWS16 % Q::NW == 0 || r < Q::ROWS16) dma_lds<16>(src, geo + r * 1024);
+            const unsigned char *src = byte < Q::HEA ? he + byte
+                                                     : gv + (VOL ? min(byte - Q::HEA, Q::GVA - 16) : Q::HEA - 16);
+            if (ROWS16 % Q::NW == 0 || r < ROWS16) dma_lds<16>(src, geo + r * 1024);
         }
         return at;
     }
@@ -173,9 +178,10 @@ __device__ __forceinline__ GeoAt geo_issue(const T *He, const T *gpvol, int nele
     const int ne = min(Q::NE, nelem - unit * Q::NE);
     const int hlim = ne * (Q::HEB / Q::NE) - 4, glim = ne * (Q::GVB / Q::NE) - 4;
 #pragma unroll 1
-    for (int r = wv; r < Q::ROWS4; r += Q::NW) {
+    for (int r = wv; r < ROWS4; r += Q::NW) {
         const int byte = r * 256 + wl * 4;
-        const unsigned char *src = byte < Q::HEA ? he + min(byte, hlim) : gv + min(byte - Q::HEA, glim);
+        const unsigned char *src =
+            byte < Q::HEA || !VOL ? he + min(byte, hlim) : gv + min(byte - Q::HEA, glim);
         dma_lds<4>(src, geo + r * 256);
     }
     return {0, 0};
