@@ -19,10 +19,9 @@ __device__ __forceinline__ void lds_barrier()
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// s_waitcnt immediates (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] |
-// vmcnt[5:4] << 14)
-constexpr int kWaitVm0 = 0x0F70;   // vmcnt(0)
-constexpr int kWaitLgkm0 = 0xC07F; // lgkmcnt(0)
+// s_waitcnt immediate of vmcnt(0) (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] |
+// lgkmcnt[11:8] | vmcnt[5:4] << 14)
+constexpr int kWaitVm0 = 0x0F70;
 
 // Element order of the lane-per-node element loops: the blocks of one XCD
 // (blockIdx % 8; the grid is a multiple of 8) walk one contiguous eighth of

@@ -16,8 +16,6 @@ template <int P> struct EG {
 template <int P, typename T> struct LineTab {
     int off[3][P];
     T ds[3], d[3][P]; // d/dxi_k at the lane's point: own and other coefficients
-    T t[3][P];        // transposed: d/dxi_k of the lane's basis function at the
-                      // other nodes (weak divergence)
 };
 
 template <int P, typename T>
@@ -43,7 +41,6 @@ __device__ __forceinline__ void build_linetab(int a, const T *__restrict__ dl,
             const int b = min(max(inv[idx[0] + N1 * (idx[1] + N1 * idx[2])] - 1, 0), NN - 1);
             t.off[k][o] = b;
             t.d[k][o] = dl[a + NN * (k + 3 * m)];
-            t.t[k][o] = dl[b + NN * (k + 3 * own[k])];
         }
     }
 }

@@ -32,7 +32,6 @@ namespace sodhip {
 
 template <typename T> struct RhsArgs {
     int nelem, npoin;
-    size_t EN;
     const int *connecT;
     const T *He, *gpvol, *dl;
     const int *inv, *gI, *gJ, *gK;
@@ -1321,7 +1320,6 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
 
     const int role = threadIdx.x >> 6; // 0: convection, 1: viscous (wave-uniform)
     const int lane = threadIdx.x & 63;
-    const bool act = true;
     const bool visc = role == 1;
 
     constexpr int RUN = L::RUN, RSH = 1;
@@ -1455,18 +1453,12 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
         // the lane read its handover from); the viscous wave stores them
         auto finish = [&]() {
             const V2 h01 = s2[3 * pa], h23 = s2[3 * pa + 1], h4 = s2[3 * pa + 2];
-            if constexpr (RW == 6) {
-                s2[3 * pa] = V2{pend[0] + h01.x, pend[1] + h01.y};
-                s2[3 * pa + 1] = V2{pend[2] + h23.x, pend[3] + h23.y};
-                s2[3 * pa + 2] = V2{pend[4] + h4.x, T(0)};
-            } else {
-                T *d = (T *)s2 + 5 * pa;
-                d[0] = pend[0] + h01.x;
-                d[1] = pend[1] + h01.y;
-                d[2] = pend[2] + h23.x;
-                d[3] = pend[3] + h23.y;
-                d[4] = pend[4] + h4.x;
-            }
+            T *d = (T *)s2 + RW * pa;
+            d[0] = pend[0] + h01.x;
+            d[1] = pend[1] + h01.y;
+            d[2] = pend[2] + h23.x;
+            d[3] = pend[3] + h23.y;
+            d[4] = pend[4] + h4.x;
         };
         for (int t = 0; t < nit; ++t) {
             wait_vm<(AH - 1) * L::NOPS0>();
@@ -1483,11 +1475,9 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                 for (int d = 0; d < 3; ++d) u[d] = T(ud[d]);
                 p = T(pd - A.p_ref);
                 H = T(hd + 0.5 * umag);
-                if (act) {
-                    s1[(own + 0) >> 1] = V2{u[0], u[1]};
-                    s1[(own + 2) >> 1] = V2{u[2], rho};
-                    s1[(own + 4) >> 1] = V2{p, H};
-                }
+                s1[(own + 0) >> 1] = V2{u[0], u[1]};
+                s1[(own + 2) >> 1] = V2{u[2], rho};
+                s1[(own + 4) >> 1] = V2{p, H};
             }
             lds_barrier(); // B2
             {
@@ -1660,7 +1650,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                 Tk = T(Td);
                 const double mfe = A.mu_factor_e ? A.mu_factor_e[elem_of(t)] : A.mu_factor;
                 muf = T(sutherland<double>(mfe, Td));
-                if (act) s1[(own + 6) >> 1] = V2{Tk, T(0)};
+                s1[(own + 6) >> 1] = V2{Tk, T(0)};
             }
             lds_barrier(); // B2
             // the previous element's records go into the
@@ -1727,12 +1717,10 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                     gr[r] = h0 * tau[r][0] + h1 * tau[r][1] + h2 * tau[r][2];
                     tuk += gr[r] * u[r]; // tau is symmetric: contravariant (tau u)_k
                 }
-                if (act) {
-                    s2[(g + 6 * k + 0) >> 1] = V2{h0 * gR[0] + h1 * gR[1] + h2 * gR[2],
-                                                h0 * gt[0] + h1 * gt[1] + h2 * gt[2]};
-                    s2[(g + 6 * k + 2) >> 1] = V2{tuk, gr[0]};
-                    s2[(g + 6 * k + 4) >> 1] = V2{gr[1], gr[2]};
-                }
+                s2[(g + 6 * k + 0) >> 1] = V2{h0 * gR[0] + h1 * gR[1] + h2 * gR[2],
+                                            h0 * gt[0] + h1 * gt[1] + h2 * gt[2]};
+                s2[(g + 6 * k + 2) >> 1] = V2{tuk, gr[0]};
+                s2[(g + 6 * k + 4) >> 1] = V2{gr[1], gr[2]};
             }
             // this wave alone reads s2 next: its LDS instructions execute in order
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
@@ -1768,11 +1756,9 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-            if (act) {
-                s2[3 * pa] = V2{nu_e * W6[0], W6[3]};
-                s2[3 * pa + 1] = V2{W6[4], W6[5]};
-                s2[3 * pa + 2] = V2{W6[2] + kappa * W6[1], T(0)};
-            }
+            s2[3 * pa] = V2{nu_e * W6[0], W6[3]};
+            s2[3 * pa + 1] = V2{W6[4], W6[5]};
+            s2[3 * pa + 2] = V2{W6[2] + kappa * W6[1], T(0)};
         }
         // the last element's records, completed by the convection wave
         lds_barrier();
@@ -1878,16 +1864,12 @@ static int full_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const i
     RhsArgs<T> A{};
     A.nelem = nelem;
     A.npoin = npoin;
-    A.EN = EN;
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
     A.gpvol = gpvol;
     A.dl = dl;
     A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
     A.u = u;
     A.q = q;
     A.rho = rho;
@@ -1926,16 +1908,12 @@ static int full_diffusion(sodhip_ctx ctx, int porder, int nelem, int npoin, cons
     RhsArgs<T> A{};
     A.nelem = nelem;
     A.npoin = npoin;
-    A.EN = EN;
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
     A.gpvol = gpvol;
     A.dl = dl;
     A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
     A.rho = rho;
     A.u = u;
     A.rho_n = rho_n;
@@ -1969,25 +1947,20 @@ int fused_record_width(int porder, int op_bytes)
 
 template <typename T>
 int rhs_fused_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *He,
-                       const T *gpvol, const T *dl, const int *inv, const int *gI, const int *gJ,
-                       const int *gK, const double *rho, const double *q, const double *E,
-                       const T *mu_e, double gamma, double Rgas, double Cp, double Pr,
+                       const T *gpvol, const T *dl, const int *inv, const double *rho,
+                       const double *q, const double *E, const T *mu_e, double gamma, double Rgas, double Cp, double Pr,
                        double mu_factor, const double *mu_factor_e, double c_rho, double c_ener,
                        double p_ref, T *out)
 {
     RhsArgs<T> A{};
     A.nelem = m->nelem;
     A.npoin = m->npoin;
-    A.EN = (size_t)m->nelem * nnode_of(porder);
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
     A.gpvol = gpvol;
     A.dl = dl;
     A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
     A.cr = rho;
     A.cq = q;
     A.cE = E;
@@ -2023,7 +1996,6 @@ int rhs_cluster_stage(sodhip_ctx ctx, const MeshCache *m, const ClusterTables *c
     RhsArgs<T> A{};
     A.nelem = m->nelem;
     A.npoin = m->npoin;
-    A.EN = (size_t)m->nelem * 64;
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
@@ -2101,7 +2073,6 @@ int lps_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const LpsArgs &
     RhsArgs<double> A{};
     A.nelem = m->nelem;
     A.npoin = m->npoin;
-    A.EN = (size_t)m->nelem * nnode_of(porder);
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = L.He;
@@ -2159,17 +2130,15 @@ int lps_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const LpsArgs &
 }
 
 template int rhs_fused_elements<double>(sodhip_ctx, int, const MeshCache *, const double *,
-                                        const double *, const double *, const int *, const int *,
-                                        const int *, const int *, const double *, const double *,
-                                        const double *, const double *, double, double, double,
-                                        double, double, const double *, double, double, double,
-                                        double *);
+                                        const double *, const double *, const int *,
+                                        const double *, const double *, const double *,
+                                        const double *, double, double, double, double, double,
+                                        const double *, double, double, double, double *);
 template int rhs_fused_elements<float>(sodhip_ctx, int, const MeshCache *, const float *,
-                                       const float *, const float *, const int *, const int *,
-                                       const int *, const int *, const double *, const double *,
-                                       const double *, const float *, double, double, double,
-                                       double, double, const double *, double, double, double,
-                                       float *);
+                                       const float *, const float *, const int *, const double *,
+                                       const double *, const double *, const float *, double,
+                                       double, double, double, double, const double *, double,
+                                       double, double, float *);
 
 template <int P, typename T, GradOp OP>
 static void launch_grad_p(sodhip_ctx ctx, RhsArgs<T> A, const T *f = nullptr, const T *eta = nullptr)
@@ -2199,16 +2168,12 @@ static int scalar_convec(sodhip_ctx ctx, int porder, int nelem, int npoin, const
     RhsArgs<T> A{};
     A.nelem = nelem;
     A.npoin = npoin;
-    A.EN = EN;
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
     A.gpvol = gpvol;
     A.dl = dl;
     A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
     A.u = u;
     A.out = (T *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 3);
@@ -2267,16 +2232,12 @@ static int div_curl(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin_
     RhsArgs<T> A{};
     A.nelem = nelem;
     A.npoin = npoin;
-    A.EN = EN;
     A.connecT = m->connecT;
     A.perm = m->perm;
     A.He = He;
     A.gpvol = gpvol; // not read where only the vorticity is asked for
     A.dl = dl;
     A.inv = inv;
-    A.gI = gI;
-    A.gJ = gJ;
-    A.gK = gK;
     A.u = u;
     A.out = (T *)ctx->scratch.ptr;
     int tok = prof_begin(ctx, 3);

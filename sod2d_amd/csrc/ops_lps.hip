@@ -194,11 +194,7 @@ static int lps_common(sodhip_ctx ctx, int porder, int nelem, int npoin, const in
 // full_proj_ijk into the caller's projections, records through out (12 x EN)
 static int proj_run(sodhip_ctx ctx, int porder, const MeshCache *m, LpsArgs A,
                     const double *invMl, double *ProjMass, double *ProjEner, double *ProjMX,
-                    double *ProjMY, double *ProjMZ, double *prj = nullptr);
-
-static int proj_run(sodhip_ctx ctx, int porder, const MeshCache *m, LpsArgs A,
-                    const double *invMl, double *ProjMass, double *ProjEner, double *ProjMX,
-                    double *ProjMY, double *ProjMZ, double *prj)
+                    double *ProjMY, double *ProjMZ, double *prj = nullptr)
 {
     int tok = prof_begin(ctx, 4);
     const int rc = lps_elements(ctx, porder, m, A, LpsKernel::proj);

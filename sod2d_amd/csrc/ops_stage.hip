@@ -26,9 +26,8 @@ namespace sodhip {
 
 template <typename T>
 int rhs_fused_elements(sodhip_ctx ctx, int porder, const MeshCache *m, const T *He,
-                       const T *gpvol, const T *dl, const int *inv, const int *gI, const int *gJ,
-                       const int *gK, const double *rho, const double *q, const double *E,
-                       const T *mu_e, double gamma, double Rgas, double Cp, double Pr,
+                       const T *gpvol, const T *dl, const int *inv, const double *rho,
+                       const double *q, const double *E, const T *mu_e, double gamma, double Rgas, double Cp, double Pr,
                        double mu_factor, const double *mu_factor_e, double c_rho, double c_ener,
                        double p_ref, T *out);
 int fused_record_width(int porder, int op_bytes);
@@ -322,8 +321,9 @@ static int rk_stage_on(sodhip_ctx ctx, int porder, const MeshCache *m, int npoin
         return set_error(SODHIP_ERR_ARG, "the stage needs %zu bytes of record scratch, %zu available",
                          rw * EN * sizeof(T), scr_bytes);
     T *scr = (T *)scr_mem;
-    int rc = rhs_fused_elements<T>(ctx, porder, m, He, gpvol, dl, inv, gI, gJ, gK, st[0], st[1], st[2], mu_e,
-                                   prm->gamma_gas, prm->Rgas, prm->Cp, prm->Pr, prm->mu_factor, prm->mu_factor_e,
+    int rc = rhs_fused_elements<T>(ctx, porder, m, He, gpvol, dl, inv, st[0], st[1], st[2], mu_e,
+                                   prm->gamma_gas, prm->Rgas, prm->Cp, prm->Pr,
+                                   prm->mu_factor, prm->mu_factor_e,
                                    prm->c_rho, prm->c_ener, prm->p_ref, scr);
     if (rc) return rc;
     SODHIP_TRY_HIP(hipGetLastError());
@@ -381,8 +381,9 @@ static int rk4_stage(sodhip_ctx ctx, int porder, int nelem, int npoin, int npoin
     const int rw = fused_record_width(porder, (int)sizeof(T));
     if ((rc = ensure_buf(ctx->scratch, rw * EN * sizeof(T)))) return rc;
     T *scr = (T *)ctx->scratch.ptr;
-    rc = rhs_fused_elements<T>(ctx, porder, m, He, gpvol, dl, inv, gI, gJ, gK, srho, sq, sE, mu_e,
-                               prm->gamma_gas, prm->Rgas, prm->Cp, prm->Pr, prm->mu_factor, prm->mu_factor_e,
+    rc = rhs_fused_elements<T>(ctx, porder, m, He, gpvol, dl, inv, srho, sq, sE, mu_e,
+                               prm->gamma_gas, prm->Rgas, prm->Cp, prm->Pr, prm->mu_factor,
+                               prm->mu_factor_e,
                                prm->c_rho, prm->c_ener, prm->p_ref, scr);
     if (rc) return rc;
     int tok = prof_begin(ctx, 1);
