@@ -1279,8 +1279,9 @@ __device__ __forceinline__ void split_read(const unsigned char *sl, int a, int p
 //   flux record (18 values): for k = 1..3, G_k of (grad rho, grad T, tau u,
 //                            tau_1., tau_2., tau_3.)
 // Both operators are evaluated as k_rhs evaluates them (the FP64 stage's K and z
-// coefficients, the same sums in the same order), so that this assembly and the
-// node-ordered one differ by the order of a surface node's terms only.
+// coefficients, the same sums in the same order; only the conductivity takes Cp/Pr as
+// one factor), so that this assembly and the node-ordered one differ by the order of a
+// surface node's terms and that rounding.
 // The block walks element clusters, one after the other; the viscous wave adds each element's residual records into
 // an LDS accumulator per cluster-local node instead of storing them, and after
 // a cluster's last element finishes its interior nodes (mass inverse and
@@ -1557,6 +1558,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
         lds_barrier();
     } else {
         // ======================= viscous wave
+        const T cp_pr = A.Cp / A.Pr;
         T tt[3][P];
         {
             const int own3[3] = {min(max(A.gI[a] - 1, 0), P), min(max(A.gJ[a] - 1, 0), P),
@@ -1677,6 +1679,14 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                 for (int o = 0; o < P; ++o) vt += lt.d[k][o] * LD1(nb[k][o] + 6);
                 dT[k] = vt;
             }
+            // formed here, while the convection wave is on its lines, and with one
+            // division: at the end of the element, where they are used, three divisions
+            // held up both waves (element kernel at 262k elements 1684 -> 1595 us,
+            // 1,728 elements 340 -> 311 us)
+            T nu_e = A.c_rho * mue / rho;
+            T kappa = (muf + A.c_ener * mue) * cp_pr;
+            pin(nu_e);
+            pin(kappa);
             lds_barrier(); // B3
             T gU[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
             T dr[3];
@@ -1751,8 +1761,6 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                         W6[5] += c * x45.y;
                     }
             }
-            const T nu_e = A.c_rho * mue / rho;
-            const T kappa = muf * A.Cp / A.Pr + A.c_ener * mue * A.Cp / A.Pr;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
