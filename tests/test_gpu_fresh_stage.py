@@ -59,6 +59,26 @@ def test_level2_tensors_stay_level2(precision, lps):
         assert (held[0][rest] == 7.0).all()
 
 
+def test_arrays_put_in_the_lists_are_the_levels():
+    """A caller may put arrays of its own into run.rho, run.q and run.E."""
+    import torch
+    from sod2d_amd.solver import TGVRun
+    g = make_case(2, 3, periodic=True, lengths=(2 * np.pi,) * 3)
+    a, b = (TGVRun(2, geometry=g, parity=False, dt_mode="fixed") for _ in range(2))
+    b.q[1] = b.q[1].clone()
+    b.E[0] = b.E[0].clone()
+    for step in range(3):
+        a.step()
+        b.step()
+        for x, y in zip((a.rho, a.q, a.E), (b.rho, b.q, b.E)):
+            assert torch.equal(x[0], y[0]) and torch.equal(x[1], y[1]), step
+    a.parity = b.parity = True  # from here on the levels are exchanged
+    for step in range(3):
+        a.step()
+        b.step()
+        assert torch.equal(a.E[1], b.E[1]) and torch.equal(a.q[0], b.q[0]), step
+
+
 @pytest.mark.parametrize("p", [2, 3, 4])
 @pytest.mark.parametrize("precision", [8, 4])
 def test_stage_from_level1_is_the_stage_on_a_copy(p, precision):
