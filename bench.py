@@ -389,10 +389,9 @@ def main(argv=None):
                     help="keep the default launch shape of the fused stage instead of the "
                          "autotuner's (sod2d_amd/autotune.py, run after the warm-up steps)")
     ap.add_argument("--stage-config", default=None, metavar="B,G,T",
-                    help="use this launch shape of the fused stage (element blocks per CU, "
+                    help="use this launch shape of the fused stage (elem_blocks_per_cu, "
                          "16-byte geometry rows 0/1, gather threads) instead of autotuning, "
-                         "e.g. to profile the shape a tuned run chose; with --lps the element "
-                         "kernel rounds B down to whole rounds of the blocks a CU holds")
+                         "e.g. to profile the shape a tuned run chose")
     ap.add_argument("--op-n", type=int, default=128,
                     help="elements per direction of the operator workload's box")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
@@ -506,8 +505,8 @@ def main(argv=None):
     k_ms, k_n = prof[0]
     g_ms, g_n = prof[1]
     if a.lps:
-        # one element kernel (convection and the stabilised viscous operator,
-        # two waves per element at p=3) and one gather/update per stage;
+        # one element kernel (convection and the stabilised viscous operator)
+        # and one gather/update per stage;
         # full_proj_ijk (its element kernel and projection gather) is timed apart
         t_elem = k_ms / (prof_steps * nrhs)
         t_gath = g_ms / (prof_steps * nrhs)

@@ -166,9 +166,11 @@ int sodhip_copy_present(sodhip_ctx ctx, const void *src_host, void *dst_host, si
  * kind: 0 element operator kernel, 1 node gather/update kernel, 2 sensor,
  * 3 other nodal kernels, 4 the LPS projections (full_proj_ijk's element
  * kernel and gather). */
-/* Launch shape of the fused RK stage on this context: blocks per CU of the
- * element kernel (1..64; 16 is the library's own rule, other values scale the elements each
- * workgroup takes), whether the geometry moves through LDS in 16-byte lane
+/* Launch shape of the fused RK stage on this context: elem_blocks_per_cu (1..64)
+ * sets how many elements a workgroup of the element kernel takes, relative to the
+ * library's own rule for the mesh's size, which is 16: 8 doubles them, 32 halves them,
+ * at least one group of units and at most 64 each; where the rule gives one group (small
+ * meshes), 16 and all larger values are the same launch.  Then whether the geometry moves through LDS in 16-byte lane
  * rows when He and gpvol are aligned for it (1) or in 4-byte rows (0), and
  * the gather/update block size (64, 128 or 256).  Defaults 16, 1, 256.  The
  * results do not depend on the shape.  No counterpart in the reference: the

@@ -1,8 +1,9 @@
 """Launch-shape autotuner of the fused Runge-Kutta stage.
 
-The blocks per CU of the stage's element kernel set how many elements each
-workgroup takes; its geometry moves
-through LDS in 16-byte or 4-byte lane rows (two LDS layouts of the same
+elem_blocks_per_cu sets how many elements each workgroup of the stage's element
+kernel takes, relative to the library's rule (16; smaller values give it more
+elements, and on small meshes 16 and larger ones are the same launch); its
+geometry moves through LDS in 16-byte or 4-byte lane rows (two LDS layouts of the same
 records); the gather/update runs in blocks of 64, 128 or 256 nodes.  None of
 these changes a result.  tune_stage() times every candidate shape on the
 run's own mesh and state, keeps the fastest in the run's context
@@ -54,7 +55,7 @@ def _stage_call(run, y):
 
 
 def tune_stage(run, reps: int = 5, cands=None, path: str | None = None) -> dict:
-    """Times each candidate (blocks per CU, 16-byte geometry rows, gather
+    """Times each candidate (elem_blocks_per_cu, 16-byte geometry rows, gather
     threads) over ``reps`` stages after one warm-up, by HIP events on the
     library's stream; sets the fastest on run.ctx and returns
     {"choice": ..., "table": [...]} (written as JSON to ``path`` if given)."""

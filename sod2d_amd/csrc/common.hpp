@@ -146,7 +146,7 @@ struct sodhip_ctx_s {
     // 0.37 -> 0.29 ms gather per stage at 64^3)
     bool cluster_stage = false;
     // launch shape of the fused stage (sodhip_set_stage_config): element-kernel
-    // blocks per CU, 16-byte geometry rows when aligned, gather block size
+    // elem_blocks_per_cu, 16-byte geometry rows when aligned, gather block size
     int stage_bpc = 16;
     int stage_geo16 = 1;
     int gather_threads = 256;

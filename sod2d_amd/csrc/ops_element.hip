@@ -2,13 +2,14 @@
 // operator and the generic scalar convection, the node-ordered assembly gather,
 // and their drop-in C-ABI entry points.
 //
-// The operators run on the element pipeline of pipe.hpp (lane-per-node, line
-// order, geometry through LDS); the fused stage at p=3 and the entropy and
-// velocity operators have kernels of their own below.  Element residuals go to a
-// scratch array of 5-field records per element-node (whole elements: coalesced
-// writes); a second kernel gathers them per node through the node-ordered
-// incidence table in the reference's serial (element, node) order --
-// deterministic, no atomics.
+// All operators, the fused stages at every order among them, run on the element
+// pipeline of pipe.hpp (lane-per-node, line order, geometry through LDS): k_rhs the
+// right-hand sides, k_grad the first-derivative operators; the opt-in brick-local
+// assembly of the p=3 FP64 stage has a kernel of its own (k_rhs_split).  Element
+// residuals go to a scratch array of 5-field records per element-node (whole elements:
+// coalesced writes); a second kernel gathers them per node through the node-ordered
+// incidence table in the reference's serial (element, node) order -- deterministic, no
+// atomics.
 //
 // Arithmetic restatement: the split forms are evaluated through identities that
 // hold for arbitrary nodal inputs (linearity of the discrete derivative and
@@ -48,7 +49,7 @@ template <typename T> struct RhsArgs {
     const int *perm; // element-local scratch position of each node
     T *out;          // records of 5 (mass, mom1, mom2, mom3, energy) per element-node;
                      // (e,a) at record e*NN + perm[a]
-    int run, wide;   // unit_range of k_rhs
+    int run, wide;   // unit_range
     int geo16;       // He and gpvol blocks of every element are 16-byte aligned
     // brick-local assembly of the fused p=3 stage (see ClusterTables): the
     // element order, local-node tables, the partial records of surface nodes,
@@ -65,8 +66,8 @@ template <typename T> struct RhsArgs {
     double *Rm, *Rq, *Re;
     double nx_l1, nx_gdt;
     double *nxr, *nxq, *nxE;
-    // LPS stage (the viscous wave evaluates full_diff_stab_ijk): node
-    // projection records (kProjRec values), comp_tau's tau_stab, c_lps
+    // LPS operators: node projection records (kProjRec values; the fused stage),
+    // comp_tau's tau_stab, c_lps
     const double *prj, *tau;
     double c_lps;
     const double *pMass, *pEner, *pMX, *pMY, *pMZ; // or arrays (npoin,3) (drop-in)
@@ -484,8 +485,9 @@ __global__ __launch_bounds__((EP<P, T>::NTB), (elem_waves<P, T, CONV, VISC>())) 
             // less exact than separate derivatives are (error over result, p = 2, 3, 4:
             // convection's energy 7.2e-8 -> 8.5 to 8.8e-8, viscous momentum 5.9, 6.6,
             // 7.1e-8 -> 6.6, 7.6, 8.4e-8); with the sums over the lines and the closing
-            // products in FP64 (S, WIDE) they are 6.9 to 7.1e-8 and 5.8, 6.4, 6.9e-8, in the
-            // same time (46k elements, p=4, both operators: 398 us).
+            // products in FP64 (S, WIDE) they are 6.9 to 7.1e-8 and 5.8, 6.4, 6.9e-8
+            // (46k elements, p=4, both operators: 402 -> 405 us; 2.1M, convection: 8.5 ->
+            // 8.7 ms).
             // The fused stage, whose states are smooth, is more exact than with separate
             // derivatives as it is (a step's state by 10 to 30 %), and FP64 sums cost it
             // 2 % of its time (87k elements, p=3: 1.72 -> 1.76 ms per step).
@@ -1133,26 +1135,23 @@ __global__ __launch_bounds__(256) void k_gather_entropy(int npoin, const int *__
 // ---------------------------------------------------------------- launch helpers
 // ---------------------------------------------------------------------------
 // Element kernel of the brick-local assembly (the opt-in mode of the fused FP64
-// stage at p=3), with the work of each element split over two
-// waves that share its LDS: wave 0 evaluates the split-form convection, wave 1
-// the viscous operator and hands its residuals to wave 0 through LDS; wave 0
-// puts their sum back into the same LDS slots and wave 1 stores it during the
-// next element.  Each wave holds only its own operator's live state, which
-// keeps both free of register spills in FP64 at p=3 (a single wave doing both
-// spills).  Requires (p+1)^3 == 64: one wave per operator, one lane per node.
+// stage at p=3).  Two waves share an element and its LDS: wave 0 evaluates the
+// split-form convection, wave 1 the viscous operator and hands its residuals to wave 0
+// through LDS; wave 0 puts their sum back as the element's records, and wave 1 adds
+// those to the cluster's accumulator during the next element.  Each wave holds its own
+// operator's live state, which leaves registers (214 of 256) for what the ring's copies
+// and the accumulator's tables need.  Requires (p+1)^3 == 64: one wave per operator, one
+// lane per node.
 //
 // The inputs stream through an LDS ring AH elements deep.  Every input of
 // element e (He and gpvol, the five conserved fields at its nodes, mu_e) is
 // copied global -> LDS by direct-to-LDS loads, which hold no registers while
 // in flight, AH elements before e is evaluated; its connectivity row arrives
 // AH elements earlier still, since the field addresses are read from it.
-// The copies are issued through inline assembly, outside the compiler's wait
-// tracking (which cannot tell ring slots apart and would wait for every copy
-// in flight before any read of the ring), and each wave waits for its own
-// copies with an explicit vector-memory count: a wave issues the same number
-// NOPS of copies per element, always in the same order, and loads complete in
-// issue order, so element e's copies are complete once at most (AH-1)*NOPS of
-// the wave's operations are outstanding.  The wave's stores count as well and
+// Each wave waits for its own copies with an explicit vector-memory count: a wave
+// issues the same number NOPS of copies per element, always in the same order, and loads
+// complete in issue order, so element e's copies are complete once at most (AH-1)*NOPS
+// of the wave's operations are outstanding.  The wave's stores count as well and
 // can only make that wait longer.
 //
 // Per element, both waves pass three LDS-only barriers:
@@ -1164,6 +1163,11 @@ __global__ __launch_bounds__(256) void k_gather_entropy(int npoin, const int *__
 //   B3  line derivatives of u and rho handed over: wave 0 forms them for the
 //       convection terms, and wave 1 takes them for grad u and grad rho
 //       instead of forming the same sums again
+//
+// What bounds it: 48.7 KB of LDS leave three workgroups per CU (k_rhs: 16 KB per wave,
+// two waves per SIMD), and a cluster's flush waits for its node tables and state loads.
+// Per stage at 262k elements: 1.60 ms and 0.28 ms for the gather over the surface nodes,
+// against 0.64 and 0.37 ms in the node-ordered assembly.
 template <int P, typename T, bool G16> struct SplitLDS {
     static constexpr int NN = (P + 1) * (P + 1) * (P + 1);
     static constexpr int AH = 2; // ring depth (elements in flight per block)
@@ -1282,11 +1286,11 @@ __device__ __forceinline__ void split_read(const unsigned char *sl, int a, int p
 // coefficients, the same sums in the same order; only the conductivity takes Cp/Pr as
 // one factor), so that this assembly and the node-ordered one differ by the order of a
 // surface node's terms and that rounding.
-// The block walks element clusters, one after the other; the viscous wave adds each element's residual records into
-// an LDS accumulator per cluster-local node instead of storing them, and after
+// The block walks element clusters, one after the other; the viscous wave adds each
+// element's residual records into an LDS accumulator per cluster-local node, and after
 // a cluster's last element finishes its interior nodes (mass inverse and
 // stage combine, as k_gather_update) and stores one partial record per
-// surface node.  mu_e runs are then pairs of elements.
+// surface node.
 template <int P, typename T, bool G16>
 __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
 {
@@ -1324,7 +1328,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
     const bool visc = role == 1;
 
     constexpr int RUN = L::RUN, RSH = 1;
-    // over runs of RUN elements, or over clusters
+    // over clusters
     const ElemRange er = elem_range(A.ncl);
     if (er.begin >= er.end) return;
     const int nunits = (er.end - er.begin + er.stride - 1) / er.stride;
@@ -1342,16 +1346,14 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
     }
     for (int i = threadIdx.x; i < 5 * kClusterLMax; i += 128) acc_s[i] = 0.0;
     __syncthreads();
-    // element of iteration t.  Past the block's last run, and past nelem in
-    // the last run, elements repeat: the copies stay unconditional and a
-    // repeated element stores the same records again.  In cluster mode past
-    // the block's last element the copies repeat that element.
+    // element of iteration t.  Past the block's last element the copies, which stay
+    // unconditional, repeat that element.
     auto elem_of = [&](int t) {
         const int i = min(t, nit - 1);
         const int e = cel_s[i];
         return e >= 0 ? e : cel_s[i - i % G];
     };
-    // FP64 mu_e blocks: iteration t (t >= -2 RUN) copies its share of the
+    // mu_e blocks: iteration t (t >= -2 RUN) copies its share of the
     // block of run t/RUN + 2 (floor); the block of run r is read from
     // iteration RUN r on
     auto mu_at = [&](int t) {
@@ -1585,7 +1587,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
 #pragma unroll
             for (int f = 0; f < 5; ++f) ac[f] += (double)d[f];
         };
-        // cluster mode, after the last element of the cluster of iteration tt:
+        // after the last element of the cluster of iteration tt:
         // interior working nodes get R = fact * sum * invMl and the stage
         // combine (k_gather_update's arithmetic; the sum runs over the same
         // elements in the same ascending order), surface working nodes one
@@ -1640,7 +1642,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
             lds_barrier(); // B1
             T He[3][3], vol;
             split_read<P, T, G16>(ring + slot_of(t), a, pa, He, vol, cur);
- cur.mue = mu_read(t, a);
+            cur.mue = mu_read(t, a);
             T rho, u[3], Tk, muf;
             const T mue = cur.mue;
             {
@@ -1665,9 +1667,6 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
                 mu_at(t);
                 cloc_issue(t + AH);
             }
-            // residual records of the previous element, completed in s2 by the
-            // convection wave: their stores complete while this element runs
-            // (read here, before this wave's flux records overwrite s2)
             if (t != 0 && t % G == 0) cl_flush(t - 1);
             // grad T from the T lines; grad u and grad rho from the line
             // derivatives handed over by the convection wave
@@ -1781,7 +1780,7 @@ __global__ __launch_bounds__(128, 2) void k_rhs_split(RhsArgs<T> A)
 #undef GL2
 }
 
-// Launches the operators' element kernel.  bpc: the stage's blocks-per-CU setting
+// Launches the operators' element kernel.  bpc: the stage's elem_blocks_per_cu setting
 // (16: the kernel's own launch shape; others scale the units a block takes).
 template <int P, typename T, bool CONV, int VISC, bool CONS>
 static void launch_rhs_p(sodhip_ctx ctx, RhsArgs<T> A, int bpc)

@@ -2,7 +2,7 @@
 //
 // A workgroup evaluates one unit of NE elements at a time (two at p=2, whose
 // 27 nodes would leave more than half of a wave idle; one at p=3 and p=4) and
-// walks its units in a grid-stride loop.  Lane L owns the node at position L
+// walks a tile's units (unit_range).  Lane L owns the node at position L
 // of the unit in lexicographic (I fastest) line order, so that
 //   * the four or five nodes of an i-line, neighbours in memory on a mesh
 //     numbered along i, are read by consecutive lanes: one gather of a field
@@ -13,8 +13,8 @@
 // Geometry (He, then gpvol) is copied HBM -> LDS by direct-to-LDS loads, one
 // unit ahead, in rows of 64 lanes x 16 bytes.  A unit whose He block does not
 // start on a 16-byte boundary (odd units at p=4: 9000 bytes per element) is
-// copied from the boundary before it; the lanes then read from `mis` bytes
-// past the start of the LDS copy.  Rows of 4-byte lanes serve arrays that do
+// copied from the boundary before it; the lanes then read from that many bytes
+// (GeoAt) past the start of the LDS copy.  Rows of 4-byte lanes serve arrays that do
 // not start on a 16-byte boundary and the last unit, whose rounded-up copy
 // would run past the end of the arrays.
 #pragma once
@@ -116,7 +116,7 @@ __device__ __forceinline__ UnitRange unit_range(int nunits, int run, int wide)
 // The launch over nelem elements.  A tile is as wide as the XCD has CUs (four
 // times that for blocks of one wave), and a block takes up to 16 groups of
 // units, fewer where that would leave the chip with less than two rounds of
-// blocks; bpc, the stage's blocks-per-CU setting, scales it (16: as is).  At 553k
+// blocks; bpc, the stage's elem_blocks_per_cu setting, divides it by bpc / 16.  At 553k
 // elements, p=3, FP64 the convection takes 1.25 ms with 16 groups in tiles of 32
 // blocks, 1.29 ms with tiles of 128 and 1.26 ms with 8 groups; at 63k elements,
 // p=4, 336, 349 and 347 us.  (One grid-stride walk over 128 blocks per CU, which

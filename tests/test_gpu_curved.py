@@ -5,8 +5,8 @@ the same at all nodes of an element, so an element kernel that took one
 node's geometry for another's would pass them.  Here the nodes of a
 non-periodic box are moved by U(-0.1, 0.1) x the local GLL spacing per axis
 (every node off the domain boundary), so He and gpvol differ from node to
-node, and the device time loop (two-wave element kernel at p=3, its LPS mode,
-the single-wave kernel at p=2 and p=4) is compared with the oracle's
+node, and the device time loop (the element kernel of the fused stage and its LPS
+form) is compared with the oracle's
 restatement step by step, with the bars of the periodic time-loop tests:
 rho, rho*u, E within 1e-12 normwise relative, mu_e within 1e-10; the
 FP32-operator mode with the bounds of its periodic test."""
@@ -49,7 +49,7 @@ def test_time_loop_on_jittered_box(oracle, p, n, lps):
 
 
 def test_time_loop_fp32_operators_on_jittered_box(oracle):
-    """The FP32-operator mode of the two-wave kernel (FP64 state, gather, mass
+    """The FP32-operator mode (FP64 state, gather, mass
     inverse and combine) on the non-affine box against the FP64 oracle after 4
     steps, with the bounds of the periodic FP32-operator test (rho 2e-7,
     rho*u 1e-5, E 2e-7)."""
