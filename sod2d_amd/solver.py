@@ -197,12 +197,13 @@ class TGVRun:
         # levels 1, 2; a level's conserved fields lie in one array, each from a
         # 512-byte boundary on
         self._level_at = [0, n + -n % 64, n + -n % 64 + 3 * n + -3 * n % 64]
-        self._level = [z(self._level_at[2] + n) for _ in range(2)]
+        whole = z(self._level_at[2] + n)
+        for o, k in zip(self._level_at, ("rho", "q", "E")):
+            x = np.ascontiguousarray(np.asarray(ic[k]).ravel(order="F"))
+            whole[o:o + x.size].copy_(torch.from_numpy(x))
+        self._level = [whole, whole.clone()]
         self.rho, self.q, self.E = ([lv[o:o + k * n] for lv in self._level]
                                     for o, k in zip(self._level_at, (1, 3, 1)))
-        for lv, k in ((self.rho, "rho"), (self.q, "q"), (self.E, "E")):
-            for x in lv:
-                x.copy_(_dev(ic[k]))
         self.u = [_dev(ic["u"]), _dev(ic["u"])]
         self.pr = [_dev(ic["pr"]), _dev(ic["pr"])]
         self.Tem = [_dev(ic["Tem"]), _dev(ic["Tem"])]

@@ -79,6 +79,31 @@ def test_arrays_put_in_the_lists_are_the_levels():
         assert torch.equal(a.E[1], b.E[1]) and torch.equal(a.q[0], b.q[0]), step
 
 
+@pytest.mark.parametrize("p,precision,lps", [(3, 8, False), (2, 4, False), (4, 8, True)])
+def test_captured_steps(p, precision, lps):
+    """Two captured steps, the copies of the levels among them, give the bits of eager
+    ones on every replay, with the other run's eager work between the replays."""
+    import torch
+    from sod2d_amd.solver import TGVRun
+    g = make_case(p, 3, periodic=True, lengths=(2 * np.pi,) * 3)
+    a, b = (TGVRun(p, geometry=g, parity=False, dt_mode="fixed", op_precision=precision, lps=lps)
+            for _ in range(2))
+    a.step()
+    b.step()
+    held = b.E[1]
+    graph = b.capture()
+    for rep in range(4):
+        a.step()
+        a.step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert held is b.E[1]
+        for x, y in zip((*a.rho, *a.q, *a.E, a.mu_e), (*b.rho, *b.q, *b.E, b.mu_e)):
+            assert torch.equal(x, y), rep
+    graph.release()
+
+
 @pytest.mark.parametrize("p", [2, 3, 4])
 @pytest.mark.parametrize("precision", [8, 4])
 def test_stage_from_level1_is_the_stage_on_a_copy(p, precision):
